@@ -103,100 +103,209 @@ int precond_free(pdes_ctx* c) {
 }
 
 // ---------------------------------------------------------------------------
-// block-Jacobi setup: gather the element block from the BSR matrix into LDS
-// (FP32) and invert it in place by Gauss-Jordan elimination with partial
-// (row) pivoting; the inverse is stored column-major so that the apply is a
+// block-Jacobi setup: each element's block is gathered from the BSR matrix
+// (FP32) and inverted in place by Gauss-Jordan elimination with partial (row)
+// pivoting; the inverse is stored column-major so that the apply is a
 // coalesced matrix-vector product.
+//
+// A chain of N pivots, so what bounds it is the latency of one step, not its
+// flops.  The block lives in registers: G x G threads, thread (tr, tc) holds
+// the rows tr + G i and the columns tc + G j (one wave for N <= 32, where the
+// barriers cost nothing, four beyond).  A step puts the pivot column in LDS,
+// every wave finds the pivot for itself (rows are never moved: a row's place
+// in the interchanged matrix is tracked instead), the pivot row's threads put
+// the scaled row in LDS, and all update: two barriers a step, about 0.5 us.
+// With the block in LDS and its rows moved a step took eight barriers and
+// 1.9 us.  One level of the ILU(0) factorization, same bits (MI355X): 48 x 48
+// blocks (2D diagonal-E p=2, 37 elements) 106 -> 36 us, 50 x 50 (3D Omega
+// p=2, 150 elements) 243 -> 87 us, 72 x 72 230 -> 70 us, 12 x 12 34 -> 17 us.
 // ---------------------------------------------------------------------------
 template <int N>
-__device__ void gauss_jordan_inverse(float (*A)[N + 1], int* perm, float* fcol, int* pivrow, int32_t* err) {
-  const int tid = threadIdx.x;
-  for (int k = 0; k < N; ++k) {
-    // pivot: max |A[r][k]| over r >= k, lowest row on ties (first wave,
-    // butterfly reduction of (value, row) pairs)
-    if (tid < 64) {
-      float best = -1.0f;
-      int bi = N;
-      for (int r = k + tid; r < N; r += 64) {
-        const float v = fabsf(A[r][k]);
-        if (v > best) { best = v; bi = r; }
+struct GjShape {
+  static constexpr int G = N <= 32 ? 8 : 16;
+  static constexpr int R = (N + G - 1) / G;      // rows and columns per thread
+  static constexpr int THREADS = G * G;
+};
+
+// max over the 64 lanes of a wave, in every lane
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+  auto step = [&](uint32_t y) { x = y > x ? y : x; };
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));   // row_shr:1
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));   // row_shr:2
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));   // row_shr:4
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));   // row_shr:8
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));   // row_bcast:15
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));   // row_bcast:31
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+template <int N>
+struct GjSmem {
+  static constexpr int NPAD = GjShape<N>::G * GjShape<N>::R;   // rows beyond N hold zeros
+  float fcol[2][NPAD];   // pivot column, alternate steps
+  float prow[2][NPAD];   // scaled pivot row
+  int pos[N];            // final place of each stored row
+  int row_at[N];         // its inverse
+};
+
+// Inverts the block held in a (thread (tr, tc), see above; zero beyond N) and
+// stores it column-major.  Every thread of the workgroup calls it.
+template <int N>
+__device__ __forceinline__ void gauss_jordan_inverse(float (&a)[GjShape<N>::R][GjShape<N>::R], GjSmem<N>& sh,
+                                                     float* __restrict__ out, int32_t* __restrict__ err) {
+  constexpr int G = GjShape<N>::G, R = GjShape<N>::R;
+  constexpr int LR = (N + 63) / 64;              // rows per lane in the pivot search
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int tr = tid % G, tc = tid / G;
+  int pos[LR];                                   // place of rows lane + 64 u in the interchanged matrix
+#pragma unroll
+  for (int u = 0; u < LR; ++u) pos[u] = lane + 64 * u < N ? lane + 64 * u : -1;
+  bool singular = false;
+  // k = kj G + kt: the register that holds column k is known at compile time
+#pragma unroll
+  for (int kj = 0; kj < R; ++kj) {
+    const int kt_n = N - kj * G < G ? N - kj * G : G;
+    for (int kt = 0; kt < kt_n; ++kt) {
+      const int k = kj * G + kt;
+      float* const fcol = sh.fcol[k & 1];
+      float* const prow = sh.prow[k & 1];
+      if (tc == kt) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) fcol[tr + G * i] = a[i][kj];
       }
-      for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+      __syncthreads();
+      // pivot: max |column k| over the rows at places >= k, lowest place on
+      // ties; a NaN is never chosen.  Keys are the value's bits plus one, 0
+      // for rows that do not take part.
+      uint32_t key = 0;
+      int kpos = N, krow = 0;
+      float kval = 0.0f;
+#pragma unroll
+      for (int u = 0; u < LR; ++u) {
+        const int r = lane + 64 * u;
+        const float x = fcol[r < N ? r : 0], v = fabsf(x);
+        const uint32_t q = (pos[u] >= k && v >= 0.0f) ? __float_as_uint(v) + 1u : 0u;
+        const bool take = q > key || (q == key && pos[u] < kpos);
+        key = take ? q : key;
+        kpos = take ? pos[u] : kpos;
+        krow = take ? r : krow;
+        kval = take ? x : kval;
       }
-      if (tid == 0) {
-        *pivrow = bi;
-        perm[k] = bi;
-        if (!(best > 0.0f)) err[0] = 1;
+      const uint32_t best = wave_max_u32(key);
+      uint64_t cand = __ballot(key == best);
+      int l = __builtin_ctzll(cand);
+      if (best == 0) {                           // a column of NaN: the row in place k
+#pragma unroll
+        for (int u = 0; u < LR; ++u) {
+          const uint64_t at = __ballot(pos[u] == k);
+          if (at) {
+            l = __builtin_ctzll(at);
+            krow = lane + 64 * u;
+            kpos = k;
+            kval = fcol[krow < N ? krow : 0];
+          }
+        }
+      } else if (cand & (cand - 1)) {
+        int ppos = __builtin_amdgcn_readlane(kpos, l);
+        for (cand &= cand - 1; cand; cand &= cand - 1) {
+          const int m = __builtin_ctzll(cand);
+          const int q = __builtin_amdgcn_readlane(kpos, m);
+          if (q < ppos) { ppos = q; l = m; }
+        }
+      }
+      const int p = __builtin_amdgcn_readlane(krow, l);
+      const int ppos = __builtin_amdgcn_readlane(kpos, l);
+      const float pivot = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kval), l));
+      singular |= best <= 1;                     // zero pivot
+#pragma unroll
+      for (int u = 0; u < LR; ++u)               // rows k and ppos of the interchanged matrix swap
+        pos[u] = lane + 64 * u == p ? k : pos[u] == k ? ppos : pos[u];
+      const float pinv = 1.0f / pivot;
+      const int pt = p % G, pi = p / G;
+      if (tr == pt) {
+        float v[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          v[j] = a[0][j];
+#pragma unroll
+          for (int i = 1; i < R; ++i) v[j] = pi == i ? a[i][j] : v[j];
+          v[j] = v[j] * pinv;
+        }
+        v[kj] = tc == kt ? pinv : v[kj];
+#pragma unroll
+        for (int j = 0; j < R; ++j) prow[tc + G * j] = v[j];
+      }
+      __syncthreads();
+      float f[R], pr[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) f[i] = fcol[tr + G * i];
+#pragma unroll
+      for (int j = 0; j < R; ++j) pr[j] = prow[tc + G * j];
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        a[i][kj] = tc == kt ? 0.0f : a[i][kj];
+        const bool is_p = tr + G * i == p;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          float x = a[i][j];
+          x -= f[i] * pr[j];
+          a[i][j] = is_p ? pr[j] : x;
+        }
       }
     }
-    __syncthreads();
-    const int p = *pivrow;
-    if (p != k)
-      for (int cc = tid; cc < N; cc += blockDim.x) {
-        const float t0 = A[k][cc];
-        A[k][cc] = A[p][cc];
-        A[p][cc] = t0;
-      }
-    __syncthreads();
-    const float pinv = 1.0f / A[k][k];
-    __syncthreads();
-    // column k of the identity takes the pivot's place, then row k is scaled
-    if (tid == 0) A[k][k] = 1.0f;
-    for (int r = tid; r < N; r += blockDim.x) fcol[r] = (r == k) ? 0.0f : A[r][k];
-    __syncthreads();
-    for (int cc = tid; cc < N; cc += blockDim.x) A[k][cc] *= pinv;
-    for (int r = tid; r < N; r += blockDim.x)
-      if (r != k) A[r][k] = 0.0f;
-    __syncthreads();
-    for (int t = tid; t < N * N; t += blockDim.x) {
-      const int r = t / N, cc = t - r * N;
-      if (r != k) A[r][cc] -= fcol[r] * A[k][cc];
-    }
-    __syncthreads();
   }
-  // undo the row interchanges as column interchanges, last first
-  for (int k = N - 1; k >= 0; --k) {
-    const int p = perm[k];
-    if (p != k)
-      for (int r = tid; r < N; r += blockDim.x) {
-        const float t0 = A[r][k];
-        A[r][k] = A[r][p];
-        A[r][p] = t0;
+  if (singular && tid == 0) err[0] = 1;
+  // row r of the array is row pos[r] of the inverse, and column c the column
+  // of the row that ended in place c
+  if (tid < 64) {
+#pragma unroll
+    for (int u = 0; u < LR; ++u)
+      if (lane + 64 * u < N) {
+        sh.pos[lane + 64 * u] = pos[u];
+        sh.row_at[pos[u]] = lane + 64 * u;
       }
-    __syncthreads();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    if (tc + G * j >= N) continue;
+    const int col = sh.row_at[tc + G * j];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (tr + G * i < N) out[col * N + sh.pos[tr + G * i]] = a[i][j];
   }
 }
 
 template <int NP, int ND, class BT>
-__global__ void __launch_bounds__(256)
+__device__ __forceinline__ void load_own_block(const BT* __restrict__ vals, const int64_t* run,
+                                               float (&a)[GjShape<NP * ND>::R][GjShape<NP * ND>::R]) {
+  constexpr int N = NP * ND, G = GjShape<N>::G, R = GjShape<N>::R;
+  const int tr = threadIdx.x % G, tc = threadIdx.x / G;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int r = tr + G * i, c = tc + G * j;
+      a[i][j] = 0.0f;
+      if (r < N && c < N && run[r / ND] >= 0)
+        a[i][j] = (float)vals[(run[r / ND] + c / ND) * (ND * ND) + (r % ND) * ND + c % ND];
+    }
+}
+
+template <int NP, int ND, class BT>
+__global__ void __launch_bounds__(GjShape<NP * ND>::THREADS)
 bjacobi_factor_kernel(const int32_t* __restrict__ el_list, const int64_t* __restrict__ rowptr,
                       const int32_t* __restrict__ colind, const BT* __restrict__ vals, float* __restrict__ inv,
                       int32_t* __restrict__ err) {
   constexpr int N = NP * ND;
-  __shared__ float A[N][N + 1];
-  __shared__ float fcol[N];
-  __shared__ int perm[N];
-  __shared__ int pivrow;
-  const int tid = threadIdx.x;
+  __shared__ GjSmem<N> sh;
+  __shared__ int64_t run[NP];
   const int64_t e = el_list ? (int64_t)el_list[blockIdx.x] : (int64_t)blockIdx.x;
-  for (int t = tid; t < NP * NP; t += blockDim.x) {
-    const int i = t / NP, j = t - i * NP;
-    const int64_t row = e * NP + i;
-    const int64_t pos = bsr_find(rowptr, colind, row, (int32_t)(e * NP + j));
-    for (int a = 0; a < ND; ++a)
-      for (int b = 0; b < ND; ++b)
-        A[i * ND + a][j * ND + b] = pos >= 0 ? (float)vals[pos * ND * ND + a * ND + b] : 0.0f;
-  }
+  for (int i = threadIdx.x; i < NP; i += blockDim.x) run[i] = bsr_find(rowptr, colind, e * NP + i, (int32_t)(e * NP));
   __syncthreads();
-  gauss_jordan_inverse<N>(A, perm, fcol, &pivrow, err);
-  float* out = inv + e * N * N;
-  for (int t = tid; t < N * N; t += blockDim.x) {
-    const int cc = t / N, r = t - cc * N;
-    out[t] = A[r][cc];
-  }
+  float a[GjShape<N>::R][GjShape<N>::R];
+  load_own_block<NP, ND>(vals, run, a);
+  gauss_jordan_inverse<N>(a, sh, inv + e * N * N, err);
 }
 
 // block-Jacobi apply: x_e = inv_e b_e; EPB = 256 / N elements per block, thread
@@ -241,34 +350,54 @@ bjacobi_apply_kernel(const int32_t* __restrict__ el_list, int64_t nel, const flo
 // Elements are processed level by level (a level holds elements whose lower
 // neighbours are all in earlier levels), each level in one launch.
 // ---------------------------------------------------------------------------
-template <int NP, int ND, int NS, class BT>
-__global__ void __launch_bounds__(256)
+//
+// The products run on the threads and registers of the elimination: thread
+// (tr, tc) forms the entries that it holds, from operands in LDS.  A block's
+// place in its row is read off the row's layout (lower neighbours, the NP own
+// blocks from own[row] on, upper neighbours) instead of searched for, and the
+// three operands of a face are loaded together: what is left besides the
+// elimination is a short chain of loads per face.
+template <int NP, int ND, int NS, bool DIAGE, class BT>
+__global__ void __launch_bounds__(GjShape<NP * ND>::THREADS)
 ilu_factor_level_kernel(const int32_t* __restrict__ lev_el, const int64_t* __restrict__ rowptr,
-                        const int32_t* __restrict__ colind, const BT* __restrict__ vals,
-                        const pdes::ElFace* __restrict__ elface, int nfaces, const int32_t* __restrict__ perm,
+                        const int32_t* __restrict__ colind, const int32_t* __restrict__ own,
+                        const BT* __restrict__ vals, const pdes::ElFace* __restrict__ elface, int nfaces,
+                        const int32_t* __restrict__ perm, const int32_t* __restrict__ nodepos,
                         float* __restrict__ inv, int32_t* __restrict__ err, const int32_t* __restrict__ el_inst,
                         const int32_t* __restrict__ inst_active) {
   constexpr int N = NP * ND;
   constexpr int M = NS * ND;
-  __shared__ float A[N][N + 1];
+  constexpr int G = GjShape<N>::G, R = GjShape<N>::R, RM = (M + G - 1) / G;
+  constexpr int T = GjShape<N>::THREADS, LM = (M * M + T - 1) / T;
+  static_assert(DIAGE || NS == NP, "dense faces couple all nodes of both elements");
   __shared__ float B1[M][M + 1];
   __shared__ float B2[M][M + 1];
   __shared__ float B3[M][M + 1];
-  __shared__ float fcol[N];
-  __shared__ int permk[N];
-  __shared__ int pivrow;
+  __shared__ float B4[M][M + 1];
+  __shared__ GjSmem<N> sh;
   __shared__ int Ce[NS], Rk[NS];
+  __shared__ int64_t run[NP];
+  __shared__ int64_t at_ke[NS][DIAGE ? NS : 1], at_ek[NS][DIAGE ? NS : 1];
   const int tid = threadIdx.x;
+  const int tr = tid % G, tc = tid / G;
   const int64_t e = lev_el[blockIdx.x];
   if (inst_active && !inst_active[el_inst[e]]) return;
-  for (int t = tid; t < NP * NP; t += blockDim.x) {
-    const int i = t / NP, j = t - i * NP;
-    const int64_t pos = bsr_find(rowptr, colind, e * NP + i, (int32_t)(e * NP + j));
-    for (int a = 0; a < ND; ++a)
-      for (int b = 0; b < ND; ++b)
-        A[i * ND + a][j * ND + b] = pos >= 0 ? (float)vals[pos * ND * ND + a * ND + b] : 0.0f;
-  }
+  for (int i = tid; i < NP; i += T) run[i] = rowptr[e * NP + i] + own[e * NP + i];
   __syncthreads();
+  float a[R][R];
+  load_own_block<NP, ND>(vals, run, a);
+  // where the blocks (row, first + node) of a neighbour element begin (dense
+  // faces: NP blocks in a run) or the one block (row, first + node) is
+  // (diagonal-E); -1 if absent
+  auto place = [&](int64_t row, bool lower, int64_t first, int node) -> int64_t {
+    const int64_t p0 = rowptr[row], o = own[row];
+    const int64_t b = lower ? p0 : p0 + o + NP, n = lower ? p0 + o : rowptr[row + 1];
+    const int32_t want = (int32_t)(first + (DIAGE ? node : 0));
+    int64_t q = -1;
+    for (int64_t p = b; p < n; p += DIAGE ? 1 : NP)
+      if (colind[p] == want) q = p;
+    return q;
+  };
   for (int f = 0; f < nfaces; ++f) {
     const pdes::ElFace r = elface[e * nfaces + f];
     if (r.x < 0 || r.x >= e) continue;   // boundary face or upper neighbour (uniform over the block)
@@ -278,47 +407,94 @@ ilu_factor_level_kernel(const int32_t* __restrict__ lev_el, const int64_t* __res
       Ce[tid] = perm[tid * nfaces + f];
       Rk[tid] = perm[tid * nfaces + fk];
     }
+    for (int t = tid; t < (DIAGE ? NS * NS : NS); t += T) {
+      const int s1 = DIAGE ? t / NS : t, s2 = DIAGE ? t % NS : 0;
+      at_ke[s1][s2] = place(k * NP + perm[s1 * nfaces + fk], false, e * NP, perm[s2 * nfaces + f]);
+      at_ek[s1][s2] = place(e * NP + perm[s1 * nfaces + f], true, k * NP, perm[s2 * nfaces + fk]);
+    }
     __syncthreads();
-    // B1 = [D'_k^-1](Rk,Rk), B2 = S_ke = A(k rows Rk, e cols Ce)
+    // B1 = [D'_k^-1](Rk,Rk), B2 = S_ke = A(k rows Rk, e cols Ce), B4 = S_ek = A(e rows Ce, k cols Rk)
     const float* Ik = inv + k * N * N;
-    for (int t = tid; t < M * M; t += blockDim.x) {
-      const int r1 = t / M, c1 = t - r1 * M;
-      const int s1 = r1 / ND, a = r1 - s1 * ND, s2 = c1 / ND, b = c1 - s2 * ND;
-      B1[r1][c1] = Ik[(Rk[s2] * ND + b) * N + Rk[s1] * ND + a];
-      const int64_t pos = bsr_find(rowptr, colind, k * NP + Rk[s1], (int32_t)(e * NP + Ce[s2]));
-      B2[r1][c1] = pos >= 0 ? (float)vals[pos * ND * ND + a * ND + b] : 0.0f;
+    float v1[LM], v2[LM], v4[LM];
+#pragma unroll
+    for (int u = 0; u < LM; ++u) {
+      const int t = tid + u * T;
+      v1[u] = v2[u] = v4[u] = 0.0f;
+      if (t < M * M) {
+        const int r1 = t / M, c1 = t - r1 * M;
+        const int s1 = r1 / ND, x = r1 - s1 * ND, s2 = c1 / ND, y = c1 - s2 * ND;
+        v1[u] = Ik[(Rk[s1] * ND + x) * N + Rk[s2] * ND + y];   // transposed: lanes along a stored column
+        const int64_t q2 = at_ke[s1][DIAGE ? s2 : 0], q4 = at_ek[s1][DIAGE ? s2 : 0];
+        if (q2 >= 0) v2[u] = (float)vals[(q2 + (DIAGE ? 0 : Ce[s2])) * (ND * ND) + x * ND + y];
+        if (q4 >= 0) v4[u] = (float)vals[(q4 + (DIAGE ? 0 : Rk[s2])) * (ND * ND) + x * ND + y];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < LM; ++u) {
+      const int t = tid + u * T;
+      if (t < M * M) {
+        const int r1 = t / M, c1 = t - r1 * M;
+        B1[c1][r1] = v1[u];
+        B2[r1][c1] = v2[u];
+        B4[r1][c1] = v4[u];
+      }
     }
     __syncthreads();
-    for (int t = tid; t < M * M; t += blockDim.x) {
-      const int r1 = t / M, c1 = t - r1 * M;
-      float acc = 0.0f;
-      for (int l = 0; l < M; ++l) acc += B1[r1][l] * B2[l][c1];
-      B3[r1][c1] = acc;
+    float acc[RM][RM];
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int j = 0; j < RM; ++j) acc[i][j] = 0.0f;
+    for (int l = 0; l < M; ++l) {
+      float u[RM], w[RM];
+#pragma unroll
+      for (int i = 0; i < RM; ++i) u[i] = tr + G * i < M ? B1[tr + G * i][l] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < RM; ++j) w[j] = tc + G * j < M ? B2[l][tc + G * j] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int j = 0; j < RM; ++j) acc[i][j] += u[i] * w[j];
     }
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int j = 0; j < RM; ++j)
+        if (tr + G * i < M && tc + G * j < M) B3[tr + G * i][tc + G * j] = acc[i][j];
     __syncthreads();
-    // B1 = S_ek = A(e rows Ce, k cols Rk)
-    for (int t = tid; t < M * M; t += blockDim.x) {
-      const int r1 = t / M, c1 = t - r1 * M;
-      const int s1 = r1 / ND, a = r1 - s1 * ND, s2 = c1 / ND, b = c1 - s2 * ND;
-      const int64_t pos = bsr_find(rowptr, colind, e * NP + Ce[s1], (int32_t)(k * NP + Rk[s2]));
-      B1[r1][c1] = pos >= 0 ? (float)vals[pos * ND * ND + a * ND + b] : 0.0f;
+    // D'_e -= S_ek B3 on the rows and columns of the face's stencil nodes
+    int ri[R], cj[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int rr = tr + G * i, cc = tc + G * i;
+      const int sr = rr < N ? nodepos[(rr / ND) * nfaces + f] : -1, sc = cc < N ? nodepos[(cc / ND) * nfaces + f] : -1;
+      ri[i] = sr >= 0 ? sr * ND + rr % ND : -1;
+      cj[i] = sc >= 0 ? sc * ND + cc % ND : -1;
     }
-    __syncthreads();
-    for (int t = tid; t < M * M; t += blockDim.x) {
-      const int r1 = t / M, c1 = t - r1 * M;
-      float acc = 0.0f;
-      for (int l = 0; l < M; ++l) acc += B1[r1][l] * B3[l][c1];
-      const int s1 = r1 / ND, a = r1 - s1 * ND, s2 = c1 / ND, b = c1 - s2 * ND;
-      A[Ce[s1] * ND + a][Ce[s2] * ND + b] -= acc;
+    float upd[R][R];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < R; ++j) upd[i][j] = 0.0f;
+    for (int l = 0; l < M; ++l) {
+      float u[R], w[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) u[i] = ri[i] >= 0 ? B4[ri[i]][l] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < R; ++j) w[j] = cj[j] >= 0 ? B3[l][cj[j]] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < R; ++j) upd[i][j] += u[i] * w[j];
     }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        if (ri[i] >= 0 && cj[j] >= 0) a[i][j] -= upd[i][j];
     __syncthreads();
   }
-  gauss_jordan_inverse<N>(A, permk, fcol, &pivrow, err);
-  float* out = inv + e * N * N;
-  for (int t = tid; t < N * N; t += blockDim.x) {
-    const int cc = t / N, r = t - cc * N;
-    out[t] = A[r][cc];
-  }
+  gauss_jordan_inverse<N>(a, sh, inv + e * N * N, err);
 }
 
 // One level of a sweep.  Forward: x_e = D'_e^-1 (b_e - sum_{k<e} A_ek x_k).
@@ -951,22 +1127,23 @@ int ilu_range_levels(const pdes_ctx* c, int64_t el0, int64_t el1, int* lf, int* 
   return PDES_OK;
 }
 
-template <int NP, int ND, int NS>
+template <int NP, int ND, int NS, bool DIAGE>
 static int ilu_factor(pdes_ctx* c) {
   pdes_jacobian* j = c->jac;
   pdes_precond* p = c->pc_obj;
+  const dim3 block(GjShape<NP * ND>::THREADS);
   for (size_t l = 0; l + 1 < p->fptr.size(); ++l) {
     const int64_t cnt = p->fptr[l + 1] - p->fptr[l];
     if (cnt == 0) continue;
     const int32_t* lev = p->d_fel + p->fptr[l];
     if (j->fp64)
-      hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, double>), dim3((unsigned)cnt), dim3(256), 0, c->stream,
-                         lev, j->d_rowptr, j->d_colind, (const double*)j->d_vals, c->d_elface, c->nfaces, c->d_perm,
-                         p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
+      hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, DIAGE, double>), dim3((unsigned)cnt), block, 0, c->stream,
+                         lev, j->d_rowptr, j->d_colind, p->d_own, (const double*)j->d_vals, c->d_elface, c->nfaces,
+                         c->d_perm, c->d_nodepos, p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
     else
-      hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, float>), dim3((unsigned)cnt), dim3(256), 0, c->stream,
-                         lev, j->d_rowptr, j->d_colind, (const float*)j->d_vals, c->d_elface, c->nfaces, c->d_perm,
-                         p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
+      hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, DIAGE, float>), dim3((unsigned)cnt), block, 0, c->stream,
+                         lev, j->d_rowptr, j->d_colind, p->d_own, (const float*)j->d_vals, c->d_elface, c->nfaces,
+                         c->d_perm, c->d_nodepos, p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
   }
   PDES_HIP(hipGetLastError());
   return PDES_OK;
@@ -1049,12 +1226,12 @@ static int bj_factor(pdes_ctx* c) {
   pdes_jacobian* j = c->jac;
   pdes_precond* p = c->pc_obj;
   if (c->active_count() == 0) return PDES_OK;
-  const dim3 grid((unsigned)c->active_count());
+  const dim3 grid((unsigned)c->active_count()), block(GjShape<NP * ND>::THREADS);
   if (j->fp64)
-    hipLaunchKernelGGL((bjacobi_factor_kernel<NP, ND, double>), grid, dim3(256), 0, c->stream, c->active_list(),
+    hipLaunchKernelGGL((bjacobi_factor_kernel<NP, ND, double>), grid, block, 0, c->stream, c->active_list(),
                        j->d_rowptr, j->d_colind, (const double*)j->d_vals, p->d_inv, j->d_err);
   else
-    hipLaunchKernelGGL((bjacobi_factor_kernel<NP, ND, float>), grid, dim3(256), 0, c->stream, c->active_list(),
+    hipLaunchKernelGGL((bjacobi_factor_kernel<NP, ND, float>), grid, block, 0, c->stream, c->active_list(),
                        j->d_rowptr, j->d_colind, (const float*)j->d_vals, p->d_inv, j->d_err);
   PDES_HIP(hipGetLastError());
   return PDES_OK;
@@ -1100,7 +1277,7 @@ __global__ void copy_kernel(const double* __restrict__ a, double* __restrict__ b
 
 static int ilu_factor_dispatch(pdes_ctx* c) {
 #define PDES_ILU_F(D_, NP_, NF_, NS_, DE_) \
-  if (c->dim == D_ && c->Np == NP_ && (c->diag_e != 0) == DE_) return ilu_factor<NP_, D_ + 2, NS_>(c);
+  if (c->dim == D_ && c->Np == NP_ && (c->diag_e != 0) == DE_) return ilu_factor<NP_, D_ + 2, NS_, DE_>(c);
   PDES_FOR_EACH_SHAPE(PDES_ILU_F)
 #undef PDES_ILU_F
   set_error("no ILU(0) kernel for this operator");
