@@ -329,9 +329,9 @@ int pdes_estimate_bytes(const pdes_mesh_desc* m, const pdes_sbp_desc* s, int fp6
     // and the dependency-driven sweeps' vector
     b += nel * Np * 4 + 2 * 4 * nel * 4 + ndof * 8;
   }
-  // GMRES basis and vectors (multi-dot partials: 2048 workgroups per basis
-  // vector), Newton step and right-hand side
-  b += (gmres_restart + 1) * ndof * 8 + 2 * ndof * 8 + (int64_t)(gmres_restart + 2) * 2048 * 8;
+  // GMRES basis and vectors (two sets of block partials, 512 workgroups per
+  // basis vector), Newton step and right-hand side
+  b += (gmres_restart + 1) * ndof * 8 + 2 * ndof * 8 + (int64_t)(gmres_restart + 1) * 2 * 512 * 8;
   b += 2 * ndof * 8;
   if (batched) b += 2 * nel * 4 + 2 * ndof * 8 + (ndof / 4096 + 1) * (8 + 4 + 4 + 64 * 8);
   *bytes = b;

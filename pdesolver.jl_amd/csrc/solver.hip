@@ -1449,67 +1449,208 @@ int pc_setup(pdes_ctx* c, int kind) {
 // ---------------------------------------------------------------------------
 // GMRES building blocks
 // ---------------------------------------------------------------------------
-constexpr int MD_THREADS = 256;
-constexpr int MD_BLOCKS = 2048;
+// CGS2 against the basis V_0 .. V_{m-1} (h = V^T w, w -= V h, twice, then
+// w /= ||w||) in four launches, each passing once over the basis:
+//   cgs_pass<MG, false>  partial dots of w
+//   cgs_pass<MG, true>   sums them to h, w -= V h, and the partial dots of the
+//                        new w from the basis values still in registers
+//   cgs_norm             sums those, w -= V h, partial sum of w^2
+//   cgs_finish           sums that, w /= ||w||, the Hessenberg column to the host
+// Small systems are bound by the number of dependent launches and by the
+// latency inside each, large ones by the basis traffic; both fall with the
+// passes fused.  A workgroup's sums over its slice go to partial[i][block] and
+// every workgroup of the next launch adds them up for itself in block order,
+// so the bits depend on n only.  Up to n = 524,288 there are at most 256
+// workgroups (at n = 131,000 and 30 vectors the second pass takes 11.6 us with
+// 256, 15.6 with 128, 24 with 64); beyond, 512 and a launch of multidot_reduce
+// before each use (at n = 300,000 a step takes 58 us the first way and 62 the
+// second).  Separate kernels for each dot, update and sum (11 launches and a
+// wait of the host a step) took 73 us a step at n = 9,600 with the operator
+// and the preconditioner, these take 38.
+constexpr int CGS_THREADS = 256;
+constexpr int CGS_SELF_REDUCE = 256, CGS_MAX_BLOCKS = 512;
 
-// partial[i][b] = sum over block b's slice of V_i . w.  MD_GROUP basis
-// vectors per pass over the slice, so w is read once per group; each vector's
-// terms are summed in the same order, and reduced by the same tree, as one
-// vector at a time would be.
-constexpr int MD_GROUP = 8;
-__global__ void __launch_bounds__(MD_THREADS)
-multidot_partial(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ w, int64_t n,
-                 double* __restrict__ partial) {
-  __shared__ double sh[MD_GROUP][MD_THREADS];
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int i0 = 0; i0 < m; i0 += MD_GROUP) {
-    const int g_n = m - i0 < MD_GROUP ? m - i0 : MD_GROUP;
-    double acc[MD_GROUP];
+static int cgs_blocks(int64_t n) {
+  const int64_t full = std::max<int64_t>(1, ceil_div(n, CGS_THREADS));
+  if (full <= 8 * CGS_SELF_REDUCE) return (int)std::min<int64_t>(CGS_SELF_REDUCE, full);
+  return (int)std::min<int64_t>(CGS_MAX_BLOCKS, full);
+}
+
+__device__ __forceinline__ double wave_sum(double x) {
 #pragma unroll
-    for (int g = 0; g < MD_GROUP; ++g) acc[g] = 0.0;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
-      const double wt = w[t];
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
+}
+
+// Sums of NV values over the lanes of a wave, NV a power of two up to 64: each
+// exchange halves the values a lane keeps, so NV - 1 of them serve all.  Lane
+// l ends with the sum of value l / (64 / NV).
+template <int NV, int HALF = NV / 2, int OFF = 32>
+__device__ __forceinline__ double wave_sums(double (&v)[NV]) {
+  if constexpr (OFF == 0) {
+    return v[0];
+  } else if constexpr (HALF == 0) {
+    v[0] += __shfl_xor(v[0], OFF, 64);
+    return wave_sums<NV, 0, OFF / 2>(v);
+  } else {
+    const bool up = threadIdx.x & OFF;
 #pragma unroll
-      for (int g = 0; g < MD_GROUP; ++g)
-        if (g < g_n) acc[g] += V[(int64_t)(i0 + g) * ldv + t] * wt;
+    for (int k = 0; k < HALF; ++k) {
+      const double give = up ? v[k] : v[k + HALF], keep = up ? v[k + HALF] : v[k];
+      v[k] = keep + __shfl_xor(give, OFF, 64);
     }
+    return wave_sums<NV, HALF / 2, OFF / 2>(v);
+  }
+}
+
+// h[i] = sum of partial[i][0 .. nb), i < m: each wave sums 8 rows at a time
+__device__ __forceinline__ void sum_partial_rows(const double* __restrict__ partial, int m, int nb, double* h) {
+  const int lane = threadIdx.x & 63;
+  for (int i0 = 8 * (threadIdx.x >> 6); i0 < m; i0 += 8 * (CGS_THREADS / 64)) {
+    double x[8];
 #pragma unroll
-    for (int g = 0; g < MD_GROUP; ++g) sh[g][threadIdx.x] = acc[g];
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) {
+    for (int i = 0; i < 8; ++i) x[i] = 0.0;
+    // (all of a wave's loads in flight together)
+    double v[8][CGS_SELF_REDUCE / 64];
 #pragma unroll
-        for (int g = 0; g < MD_GROUP; ++g) sh[g][threadIdx.x] += sh[g][threadIdx.x + s];
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int k = 0; k < CGS_SELF_REDUCE / 64; ++k) {
+        const int b = lane + 64 * k;
+        v[i][k] = i0 + i < m && b < nb ? partial[(int64_t)(i0 + i) * nb + b] : 0.0;
       }
-      __syncthreads();
-    }
-    if ((int)threadIdx.x < g_n) partial[(int64_t)(i0 + threadIdx.x) * gridDim.x + blockIdx.x] = sh[threadIdx.x][0];
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int k = 0; k < CGS_SELF_REDUCE / 64; ++k) x[i] += v[i][k];
+    const double y = wave_sums<8>(x);
+    if (lane % 8 == 0 && i0 + lane / 8 < m) h[i0 + lane / 8] = y;
   }
-}
-
-__global__ void multidot_reduce(const double* __restrict__ partial, int nb, double* __restrict__ out) {
-  __shared__ double sh[256];
-  const int i = blockIdx.x;
-  double acc = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) acc += partial[(int64_t)i * nb + b];
-  sh[threadIdx.x] = acc;
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[i] = sh[0];
 }
 
-// w -= sum_i h[i] V_i
-__global__ void multiaxpy(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ h,
-                          double* __restrict__ w, int64_t n) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
-    double acc = w[t];
-    for (int i = 0; i < m; ++i) acc -= h[i] * V[(int64_t)i * ldv + t];
-    w[t] = acc;
+// AXPY: h = sums of pin's rows (nb_in each), w -= sum_i h_i V_i (kept in hsave
+// by workgroup 0).  Then pout[i][block] = sum over the block's slice of V_i . w.
+// The first 8 MG basis values of an entry stay in registers for both uses; the
+// basis vectors beyond (m > 32) are read again, 32 at a time.
+template <int MG, bool AXPY>
+__global__ void __launch_bounds__(CGS_THREADS)
+cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ w, int64_t n,
+         const double* __restrict__ pin, int nb_in, double* __restrict__ hsave, double* __restrict__ pout) {
+  constexpr int NV = 8 * MG;
+  extern __shared__ double sh_h[];
+  __shared__ double sh_w[CGS_THREADS / 64][NV];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if constexpr (AXPY) {
+    sum_partial_rows(pin, m, nb_in, sh_h);
+    if (blockIdx.x == 0)
+      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
+  }
+  const int64_t stride = (int64_t)gridDim.x * CGS_THREADS, t0 = (int64_t)blockIdx.x * CGS_THREADS + tid;
+  for (int i0 = 0; i0 < m; i0 += NV) {
+    double acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = 0.0;
+    for (int64_t t = t0; t < n; t += stride) {
+      double v[NV];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = i0 + i < m ? V[(int64_t)(i0 + i) * ldv + t] : 0.0;
+      double wt = w[t];
+      if (AXPY && i0 == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (i < m) wt -= sh_h[i] * v[i];
+        for (int i = NV; i < m; ++i) wt -= sh_h[i] * V[(int64_t)i * ldv + t];
+        w[t] = wt;
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[i] += v[i] * wt;
+    }
+    const double x = wave_sums<NV>(acc);
+    if (lane % (64 / NV) == 0) sh_w[wave][lane / (64 / NV)] = x;
+    __syncthreads();
+    if (tid < NV && i0 + tid < m) {
+      double y = 0.0;
+#pragma unroll
+      for (int k = 0; k < CGS_THREADS / 64; ++k) y += sh_w[k][tid];
+      pout[(int64_t)(i0 + tid) * gridDim.x + blockIdx.x] = y;
+    }
+    __syncthreads();
+  }
+}
+
+// w -= sum_i h_i V_i with h the sums of pin's rows, and the partial sum of w^2
+// (m = 0: w = b - w, the residual of a cycle's start)
+template <int MG>
+__global__ void __launch_bounds__(CGS_THREADS)
+cgs_norm(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ b, const double* w, double* out,
+         int64_t n, const double* __restrict__ pin, int nb_in, double* __restrict__ hsave,
+         double* __restrict__ pout) {
+  extern __shared__ double sh_h[];
+  __shared__ double sh_w[CGS_THREADS / 64];
+  const int tid = threadIdx.x;
+  if (m > 0) {
+    sum_partial_rows(pin, m, nb_in, sh_h);
+    if (blockIdx.x == 0)
+      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
+  }
+  const int64_t stride = (int64_t)gridDim.x * CGS_THREADS;
+  double acc = 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * CGS_THREADS + tid; t < n; t += stride) {
+    double wt = m > 0 ? w[t] : (w ? b[t] - w[t] : b[t]);
+    for (int i0 = 0; i0 < m; i0 += 8 * MG) {
+      double v[8 * MG];
+#pragma unroll
+      for (int i = 0; i < 8 * MG; ++i) v[i] = i0 + i < m ? V[(int64_t)(i0 + i) * ldv + t] : 0.0;
+#pragma unroll
+      for (int i = 0; i < 8 * MG; ++i)
+        if (i0 + i < m) wt -= sh_h[i0 + i] * v[i];
+    }
+    out[t] = wt;
+    acc += wt * wt;
+  }
+  acc = wave_sum(acc);
+  if ((tid & 63) == 0) sh_w[tid >> 6] = acc;
+  __syncthreads();
+  if (tid == 0) {
+    double y = 0.0;
+#pragma unroll
+    for (int k = 0; k < CGS_THREADS / 64; ++k) y += sh_w[k];
+    pout[blockIdx.x] = y;
+  }
+}
+
+// w /= ||w|| (left alone when the norm is not positive); the column h1 + h2
+// and the norm go to host memory that the host reads after the step's event
+__global__ void __launch_bounds__(CGS_THREADS)
+cgs_finish(double* __restrict__ w, int64_t n, const double* __restrict__ pin, int nb_in, int m,
+           const double* __restrict__ h1, const double* __restrict__ h2, double* __restrict__ host) {
+  __shared__ double sh_h[8];
+  sum_partial_rows(pin, 1, nb_in, sh_h);
+  const double hn = sqrt(sh_h[0]);
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < m; i += CGS_THREADS) host[i] = h1[i] + h2[i];
+    if (threadIdx.x == 0) host[m] = hn;
+  }
+  const double inv = hn > 0.0 ? 1.0 / hn : 1.0;
+  const int64_t stride = (int64_t)gridDim.x * CGS_THREADS;
+  for (int64_t t = (int64_t)blockIdx.x * CGS_THREADS + threadIdx.x; t < n; t += stride) w[t] = inv * w[t];
+}
+
+// out[i] = sum of partial[i][0 .. nb)
+__global__ void __launch_bounds__(CGS_THREADS)
+multidot_reduce(const double* __restrict__ partial, int nb, double* __restrict__ out) {
+  __shared__ double sh[CGS_THREADS / 64];
+  double acc = 0.0;
+  for (int b = threadIdx.x; b < nb; b += CGS_THREADS) acc += partial[(int64_t)blockIdx.x * nb + b];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double y = 0.0;
+#pragma unroll
+    for (int k = 0; k < CGS_THREADS / 64; ++k) y += sh[k];
+    out[blockIdx.x] = y;
   }
 }
 
@@ -1540,9 +1681,10 @@ struct GmresWork {
   double* V = nullptr;      // (restart+1) x n
   double* w = nullptr;
   double* z = nullptr;
-  double* partial = nullptr;
-  double* coef = nullptr;   // device small buffer
-  double* hcoef = nullptr;  // pinned host buffer
+  double* partial = nullptr;    // two sets of block partials, [restart+1][CGS_MAX_BLOCKS] each
+  double* coef = nullptr;       // h of the two passes, reduced rows, solution coefficients
+  double* hcol = nullptr;       // pinned host buffer: a Hessenberg column per step, [restart+1][restart+2]
+  hipEvent_t ev[2] = {nullptr, nullptr};
   int restart = 0;
   int64_t n = 0;
 };
@@ -1561,10 +1703,13 @@ static int gmres_alloc(pdes_ctx* c, GmresWork& W, int restart) {
   if (hipMalloc((void**)&W.V, (size_t)(restart + 1) * n * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&W.w, n * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&W.z, n * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&W.partial, (size_t)(restart + 2) * MD_BLOCKS * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&W.coef, (size_t)(2 * restart + 8) * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void**)&W.hcoef, (size_t)(2 * restart + 8) * sizeof(double)) != hipSuccess) {
+      hipMalloc((void**)&W.partial, (size_t)2 * (restart + 1) * CGS_MAX_BLOCKS * sizeof(double)) != hipSuccess ||
+      hipMalloc((void**)&W.coef, (size_t)4 * (restart + 2) * sizeof(double)) != hipSuccess ||
+      hipHostMalloc((void**)&W.hcol, (size_t)(restart + 1) * (restart + 2) * sizeof(double)) != hipSuccess ||
+      hipEventCreateWithFlags(&W.ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&W.ev[1], hipEventDisableTiming) != hipSuccess) {
     set_error("GMRES workspace allocation failed");
+    gmres_free(W);
     return PDES_ERR_NOMEM;
   }
   return PDES_OK;
@@ -1580,7 +1725,9 @@ static void gmres_free(GmresWork& W) {
   if (W.z) hipFree(W.z);
   if (W.partial) hipFree(W.partial);
   if (W.coef) hipFree(W.coef);
-  if (W.hcoef) hipHostFree(W.hcoef);
+  if (W.hcol) hipHostFree(W.hcol);
+  for (hipEvent_t& e : W.ev)
+    if (e) hipEventDestroy(e);
   W = GmresWork();
 }
 
@@ -1592,17 +1739,73 @@ void gmres_release(pdes_ctx* c) {
   }
 }
 
-// dots of w with V_0..V_{m-1} into W.coef[off..off+m)
-static int multidot(pdes_ctx* c, GmresWork& W, int m, const double* w, int off) {
-  const int nb = (int)std::min<int64_t>(MD_BLOCKS, std::max<int64_t>(1, ceil_div(W.n, MD_THREADS)));
-  hipLaunchKernelGGL(multidot_partial, dim3(nb), dim3(MD_THREADS), 0, c->stream, W.V, m, W.n, w, W.n, W.partial);
-  hipLaunchKernelGGL(multidot_reduce, dim3(m), dim3(256), 0, c->stream, W.partial, nb, W.coef + off);
+// rows of block partials as the next launch reads them: as they are, or
+// summed once where there are many
+static void cgs_rows(pdes_ctx* c, GmresWork& W, int m, double*& rows, int& nb) {
+  if (nb <= CGS_SELF_REDUCE) return;
+  double* out = W.coef + 2 * (W.restart + 2);
+  hipLaunchKernelGGL(multidot_reduce, dim3(m), dim3(CGS_THREADS), 0, c->stream, rows, nb, out);
+  rows = out;
+  nb = 1;
+}
+
+template <bool AXPY>
+static void launch_cgs_pass(pdes_ctx* c, GmresWork& W, int m, double* w, const double* pin, int nb_in, double* pout,
+                            int nb) {
+  const size_t lds = AXPY ? (size_t)m * sizeof(double) : 0;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(CGS_THREADS), lds, c->stream, W.V, m, W.n, w, W.n, pin, nb_in, W.coef,
+                       pout);
+  };
+  if (m <= 8) go(cgs_pass<1, AXPY>);
+  else if (m <= 16) go(cgs_pass<2, AXPY>);
+  else go(cgs_pass<4, AXPY>);
+}
+
+// w is made orthogonal to V_0 .. V_{m-1} and normalised; the column (m
+// coefficients and the norm) goes to the host slot of step m - 1
+static int cgs2_step(pdes_ctx* c, GmresWork& W, int m, double* w) {
+  const int nb0 = cgs_blocks(W.n);
+  double* pa = W.partial;
+  double* pb = W.partial + (size_t)(W.restart + 1) * CGS_MAX_BLOCKS;
+  double* h1 = W.coef;
+  double* h2 = W.coef + W.restart + 2;
+  launch_cgs_pass<false>(c, W, m, w, nullptr, 0, pa, nb0);
+  double* rows = pa;
+  int nb = nb0;
+  cgs_rows(c, W, m, rows, nb);
+  launch_cgs_pass<true>(c, W, m, w, rows, nb, pb, nb0);
+  rows = pb;
+  nb = nb0;
+  cgs_rows(c, W, m, rows, nb);
+  auto norm = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb0), dim3(CGS_THREADS), (size_t)m * sizeof(double), c->stream, W.V, m, W.n,
+                       (const double*)nullptr, w, w, W.n, rows, nb, h2, pa);
+  };
+  if (m <= 8) norm(cgs_norm<1>);
+  else if (m <= 16) norm(cgs_norm<2>);
+  else norm(cgs_norm<4>);
+  rows = pa;
+  nb = nb0;
+  cgs_rows(c, W, 1, rows, nb);
+  hipLaunchKernelGGL(cgs_finish, dim3(nb0), dim3(CGS_THREADS), 0, c->stream, w, W.n, rows, nb, m, h1, h2,
+                     W.hcol + (size_t)(m - 1) * (W.restart + 2));
   PDES_HIP(hipGetLastError());
   return PDES_OK;
 }
 
-static int norm2_dev(pdes_ctx* c, GmresWork& W, const double* x, int off) {
-  return launch_wnorm2(c, x, nullptr, W.n, W.coef + off);
+// V_0 = (b - w) / ||b - w|| (w null: b / ||b||); the norm goes to the host
+static int cgs_start(pdes_ctx* c, GmresWork& W, const double* b, double* w) {
+  const int nb0 = cgs_blocks(W.n);
+  hipLaunchKernelGGL(cgs_norm<1>, dim3(nb0), dim3(CGS_THREADS), 0, c->stream, (const double*)nullptr, 0, W.n, b, w, W.V,
+                     W.n, (const double*)nullptr, 0, (double*)nullptr, W.partial);
+  double* rows = W.partial;
+  int nb = nb0;
+  cgs_rows(c, W, 1, rows, nb);
+  hipLaunchKernelGGL(cgs_finish, dim3(nb0), dim3(CGS_THREADS), 0, c->stream, W.V, W.n, rows, nb, 0,
+                     (const double*)nullptr, (const double*)nullptr, W.hcol);
+  PDES_HIP(hipGetLastError());
+  return PDES_OK;
 }
 
 static int apply_op(pdes_ctx* c, int mode, const double* x, double* y) {
@@ -1612,6 +1815,10 @@ static int apply_op(pdes_ctx* c, int mode, const double* x, double* y) {
     st = launch_homotopy(c, c->d_q, x, 1.0 - c->hom_lambda, c->hom_lambda, nullptr, y);
   return st ? st : launch_ptc_shift(c, x, y);
 }
+
+// how far above the tolerance the residual estimate has to be for the next
+// Arnoldi step to be enqueued ahead of it
+constexpr double GMRES_NEAR = 4.0;
 
 // GMRES(restart), right preconditioned, x0 = x on entry (device vectors).
 int gmres_device(pdes_ctx* c, const double* b, double* x, double rtol, double atol, int restart, int maxit,
@@ -1624,45 +1831,48 @@ int gmres_device(pdes_ctx* c, const double* b, double* x, double rtol, double at
   int total = 0;
   double beta = 0.0, beta0 = -1.0;
   if (x_zero) PDES_HIP(hipMemsetAsync(x, 0, n * sizeof(double), c->stream));
-  bool converged = false;
+  // one Arnoldi step: launches only; its Hessenberg column is on the host
+  // once its event has passed
+  auto enqueue = [&](int j) -> int {
+    double* Vn = W.V + (int64_t)(j + 1) * n;
+    int sst;
+    if ((sst = pc_apply(c, W.V + (int64_t)j * n, W.z)) != 0) return sst;
+    if ((sst = apply_op(c, mode, W.z, Vn)) != 0) return sst;
+    if ((sst = cgs2_step(c, W, j + 1, Vn)) != 0) return sst;
+    PDES_HIP(hipEventRecord(W.ev[j & 1], c->stream));
+    return PDES_OK;
+  };
   while (true) {
-    // r = b - A x  -> V_0
+    // r = b - A x  -> V_0 = r / ||r||
     if (x_zero && total == 0) {
-      hipLaunchKernelGGL(copy_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, b, W.V, n);
+      if ((st = cgs_start(c, W, b, nullptr)) != 0) goto done;
     } else {
-        if ((st = apply_op(c, mode, x, W.w)) != 0) goto done;
-      hipLaunchKernelGGL(copy_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, b, W.V, n);
-      hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.w, W.V, -1.0, 1, n);
+      if ((st = apply_op(c, mode, x, W.w)) != 0) goto done;
+      if ((st = cgs_start(c, W, b, W.w)) != 0) goto done;
     }
-    if ((st = norm2_dev(c, W, W.V, 0)) != 0) goto done;
-    PDES_HIP(hipMemcpyAsync(W.hcoef, W.coef, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     PDES_HIP(hipStreamSynchronize(c->stream));
-    beta = std::sqrt(W.hcoef[0]);
+    beta = W.hcol[0];
     if (beta0 < 0) beta0 = beta;
-    if (beta <= std::max(rtol * beta0, atol) || total >= maxit) { converged = beta <= std::max(rtol * beta0, atol); break; }
-    hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.V, W.V, 1.0 / beta, 0, n);
+    const double tol = std::max(rtol * beta0, atol);
+    if (beta <= tol || total >= maxit) break;
     std::fill(g.begin(), g.end(), 0.0);
     g[0] = beta;
-    int jdone = 0;
+    int jdone = 0, enqueued = 0;
     double res_est = beta;
     for (int j = 0; j < restart && total < maxit; ++j) {
-      double* Vj = W.V + (int64_t)j * n;
-      double* Vn = W.V + (int64_t)(j + 1) * n;
-      if ((st = pc_apply(c, Vj, W.z)) != 0) goto done;
-      if ((st = apply_op(c, mode, W.z, Vn)) != 0) goto done;
-      // CGS2: h = V^T w ; w -= V h ; twice
-      if ((st = multidot(c, W, j + 1, Vn, 0)) != 0) goto done;
-      hipLaunchKernelGGL(multiaxpy, dim3(grid_for(n)), dim3(256), 0, c->stream, W.V, j + 1, n, W.coef, Vn, n);
-      if ((st = multidot(c, W, j + 1, Vn, restart + 2)) != 0) goto done;
-      hipLaunchKernelGGL(multiaxpy, dim3(grid_for(n)), dim3(256), 0, c->stream, W.V, j + 1, n,
-                         W.coef + restart + 2, Vn, n);
-      if ((st = norm2_dev(c, W, Vn, 2 * restart + 4)) != 0) goto done;
-      PDES_HIP(hipMemcpyAsync(W.hcoef, W.coef, (2 * restart + 5) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-      PDES_HIP(hipStreamSynchronize(c->stream));
-      double hn = std::sqrt(W.hcoef[2 * restart + 4]);
-      for (int i = 0; i <= j; ++i) H[(size_t)i * restart + j] = W.hcoef[i] + W.hcoef[restart + 2 + i];
+      if (enqueued == j && (st = enqueue(enqueued++)) != 0) goto done;
+      // The next step is enqueued before this one's column is read, so the
+      // device does not wait for the host in between (about 20 us a step),
+      // unless the estimate is within a factor GMRES_NEAR of the tolerance and
+      // this step may be the last: a step past the last one only costs time.
+      if (enqueued == j + 1 && enqueued < restart && total + 1 < maxit && res_est > GMRES_NEAR * tol &&
+          (st = enqueue(enqueued++)) != 0)
+        goto done;
+      PDES_HIP(hipEventSynchronize(W.ev[j & 1]));
+      const double* col = W.hcol + (size_t)j * (restart + 2);
+      const double hn = col[j + 1];
+      for (int i = 0; i <= j; ++i) H[(size_t)i * restart + j] = col[i];
       H[(size_t)(j + 1) * restart + j] = hn;
-      if (hn > 0) hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, Vn, Vn, 1.0 / hn, 0, n);
       // Givens
       for (int i = 0; i < j; ++i) {
         double a = H[(size_t)i * restart + j], bb = H[(size_t)(i + 1) * restart + j];
@@ -1680,25 +1890,28 @@ int gmres_device(pdes_ctx* c, const double* b, double* x, double rtol, double at
       res_est = std::fabs(g[j + 1]);
       ++total;
       jdone = j + 1;
-      if (res_est <= std::max(rtol * beta0, atol) || hn == 0.0) break;
+      if (res_est <= tol || hn == 0.0) break;
     }
     // y = H^-1 g ; x += M^-1 V y
     {
+      // (the stream may still be running a step past the last one, which
+      // writes its host slot, V_{jdone+1} and the work vectors only)
       std::vector<double> y(jdone);
       for (int i = jdone - 1; i >= 0; --i) {
         double s = g[i];
         for (int k = i + 1; k < jdone; ++k) s -= H[(size_t)i * restart + k] * y[k];
         y[i] = s / H[(size_t)i * restart + i];
       }
-      for (int i = 0; i < jdone; ++i) W.hcoef[i] = y[i];
-      PDES_HIP(hipMemcpyAsync(W.coef, W.hcoef, jdone * sizeof(double), hipMemcpyHostToDevice, c->stream));
-      hipLaunchKernelGGL(combine_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.V, jdone, n, W.coef, W.w, n);
+      double* ypin = W.hcol + (size_t)restart * (restart + 2);
+      double* yd = W.coef + 3 * (restart + 2);
+      for (int i = 0; i < jdone; ++i) ypin[i] = y[i];
+      PDES_HIP(hipMemcpyAsync(yd, ypin, jdone * sizeof(double), hipMemcpyHostToDevice, c->stream));
+      hipLaunchKernelGGL(combine_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.V, jdone, n, yd, W.w, n);
       if ((st = pc_apply(c, W.w, W.z)) != 0) goto done;
       if (x_zero && total == jdone)
         hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.z, x, 1.0, 0, n);
       else
         hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, W.z, x, 1.0, 1, n);
-      PDES_HIP(hipStreamSynchronize(c->stream));
     }
     // The Givens estimate res_est is the residual of x + M^-1 V y only when
     // M^-1 is applied exactly; the block preconditioners apply it in FP32, so
@@ -1712,7 +1925,6 @@ done:
   if ((st = pc_check(c)) != 0) return st;
   if (iters) *iters = total;
   if (resnorm) *resnorm = beta;
-  (void)converged;
   return PDES_OK;
 }
 
