@@ -166,8 +166,8 @@ __device__ __forceinline__ void ir_zvars(const PhysConst& p, const T* q, T* z) {
 // When logs of both arguments are at hand (lgL, lgR, e.g. staged per node),
 // log(aL/aR) is taken as lgL - lgR (the branch is only taken for
 // |f| >= 0.0316, where the difference loses no accuracy that matters).
-template <class T, class LP>
-__device__ __forceinline__ T logavg_factor(const T& aL, const T& aR, const T& r, LP lgL, LP lgR) {
+template <class T, class TR, class LP>
+__device__ __forceinline__ T logavg_factor(const T& aL, const TR& aR, const T& r, LP lgL, LP lgR) {
   const T f = (aL - aR) * r;
   const T u = f * f;
   if (re(u) < 1e-3) {
@@ -193,8 +193,10 @@ __device__ __forceinline__ T logavg_factor(const T& aL, const T& aR, const T& r,
 // log z1, with log z4 LS elements further; read only on the log branch of
 // logavg), or nullptr.  dl: optional output {log(zL1/zR1), log(zL4/zR4)},
 // which the logavg factors give without a log: log(aL/aR) = 2 F f.
-template <int DIM, int NDIR, class T, class LP = std::nullptr_t, int LS = 1, class TN = double>
-__device__ __forceinline__ void ir_flux_z(const PhysConst& p, const T* zL, const T* zR,
+// TR: the right state's type, T or, for derivatives with respect to the left
+// state only, double.
+template <int DIM, int NDIR, class T, class LP = std::nullptr_t, int LS = 1, class TN = double, class TR = T>
+__device__ __forceinline__ void ir_flux_z(const PhysConst& p, const T* zL, const TR* zR,
                                           const TN* dir, T* F, LP lzL = nullptr, LP lzR = nullptr,
                                           T* dl = nullptr) {
   constexpr int ND = DIM + 2;

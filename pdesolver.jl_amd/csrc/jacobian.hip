@@ -69,7 +69,8 @@ template <class Op, int VOL, int FLUX, class BT>
 static int launch_jac(pdes_ctx* c) {
   pdes_jacobian* j = c->jac;
   if (c->active_count() == 0) return PDES_OK;
-  hipLaunchKernelGGL((euler_jacobian_kernel<Op, VOL, FLUX, BT>), dim3((unsigned)c->active_count()), dim3(256), 0, c->stream,
+  const unsigned blocks = (unsigned)ceil_div(c->active_count(), jac_epb<Op, VOL, FLUX>());
+  hipLaunchKernelGGL((euler_jacobian_kernel<Op, VOL, FLUX, BT>), dim3(blocks), dim3(256), 0, c->stream,
                      c->devmesh(), c->devsbp(), c->pc, c->d_q, j->d_rowptr, j->d_colind,
                      (BT*)j->d_vals, j->d_err, c->d_ptc_diag, c->ptc_on ? c->d_ptc_scale : nullptr);
   PDES_HIP(hipGetLastError());

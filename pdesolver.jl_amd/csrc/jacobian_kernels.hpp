@@ -9,19 +9,61 @@
 // scatters them with ADD_VALUES into a block matrix (assembleElement /
 // assembleInterface / assembleBoundary, src/jacobian/jacobian.jl:822-1759).
 //
-// Here one workgroup owns one element and writes every block of that
-// element's rows (its own Np x Np block plus the blocks coupling it to each
+// Here a workgroup owns a few elements and writes every block of their rows
+// (each element's own Np x Np blocks plus those coupling it to each
 // neighbour) directly into the BSR value array: each block is written by
 // exactly one workgroup, no atomics and no assembly pass.  Point derivatives
-// come from forward-mode dual numbers with 2*ndof directions (dF/dqL, dF/dqR),
-// the analytic counterpart of the reference's hand-differentiated *_diff
-// functions.
+// come from forward-mode dual numbers (dF/dqL, dF/dqR), the analytic
+// counterpart of the reference's hand-differentiated *_diff functions.
+//
+// The kernel is written so that no thread runs long and none spills: a face
+// node's derivative is one thread per seeded component (dual<1>), a volume
+// pair one thread per ordered pair, differentiated in the combined direction
+// with respect to one state only (the flux is symmetric: the other state's
+// derivative is the other ordered pair's), and the weak form's blocks are
+// formed and stored a BSR row at a time, lane by value.  With one thread per
+// block and per face node, all components seeded at once (dual<2 ndof>, 300 to
+// 480 bytes of spills a lane) and DIM fluxes per pair and row, the assembly
+// took (MI355X, FP32 blocks) 2487 us for 4,050 triangles diagonal-E p=3 split
+// form and 976 us for 6,000 tets Omega p=2 Roe; it takes 109 us and 182 us (the
+// stores alone, at the copy rate, 20 us and 60 us).  The row loops of the weak
+// form stay rolled: unrolled, the hoisted weights spill (454 us for the tets).
 #pragma once
 #include "residual_kernels.hpp"
 
 namespace pdes {
 
+// what a workgroup holds per element
 template <class Op, int VOL, int FLUX>
+struct JacElem {
+  static constexpr int NP = Op::NP, ND = Op::ND, DIM = Op::DIM, NF = Op::NF, NFACES = Op::NFACES;
+  double q[NP][ND];
+  double A[(VOL == VOL_WEAK) ? NP * DIM : 1][ND][ND];   // dF_d/dq at node j
+  // split form: the IR parameter vector of every node and its derivative
+  double z[(VOL == VOL_SPLIT) ? NP : 1][ND];
+  double dz[(VOL == VOL_SPLIT) ? NP : 1][ND][ND];
+  // partial sums of the diagonal blocks, one per thread of a column
+  static constexpr int KP = 4;
+  double diag[(VOL == VOL_SPLIT) ? NP : 1][(VOL == VOL_SPLIT) ? KP : 1][ND][ND];
+  // dense faces: weight of slot k's flux in row i's residual, sgn B R[i][kown]
+  static constexpr bool CW = VOL == VOL_WEAK && !Op::DIAGE;
+  double cw[CW ? NFACES : 1][CW ? NP : 1][CW ? NF : 1];
+  double qf[NFACES][NF][2][ND];         // face-node states (entropy variables for ESLF): elementL's, elementR's
+  double dFo[NFACES][NF][ND][ND];       // dF_k/dq_own   (k: elementL face node numbering)
+  double dFn[NFACES][NF][ND][ND];       // dF_k/dq_nbr
+  ElFace rec[NFACES];
+  int32_t kown[NFACES][NF];             // own face node of slot k
+  int32_t knbr[NFACES][NF];             // neighbour face node of slot k
+  int32_t kslot[NFACES][NF];            // slot of own face node m
+  double sgn[NFACES];
+  int64_t own_run[NP];                  // first own block of each row
+  // first block of the neighbour's run in each row (dense faces), or the one
+  // block of each face node (diagonal-E, [NFACES][NF])
+  int64_t nbr_run[NFACES][Op::DIAGE ? NF : NP];
+  int64_t e;
+};
+
+template <class Op, int VOL, int FLUX, int EPB>
 struct JacSmem {
   static constexpr int NP = Op::NP, ND = Op::ND, DIM = Op::DIM, NF = Op::NF, NFACES = Op::NFACES;
   double Q[DIM][NP][NP];
@@ -29,14 +71,25 @@ struct JacSmem {
   int32_t perm[Op::ST][NFACES];
   int32_t nodepos[NP][NFACES];
   double wface[NF];
-  double q[NP][ND];
-  double A[(VOL == VOL_WEAK) ? NP * DIM : 1][ND][ND];   // dF_d/dq at node j
-  double dFo[NFACES][NF][ND][ND];   // dF_k/dq_own   (k: elementL face node numbering)
-  double dFn[NFACES][NF][ND][ND];   // dF_k/dq_nbr
-  ElFace rec[NFACES];
-  int32_t kown[NFACES][NF];         // own face node of slot k
-  int32_t knbr[NFACES][NF];         // neighbour face node of slot k
-  double sgn[NFACES];
+  JacElem<Op, VOL, FLUX> el[EPB];
+};
+
+// what the entropy-stable block functions read: the tables and one element
+template <class Op, int VOL, int FLUX, int EPB>
+struct JacView {
+  const double (&interp)[Op::ST][Op::NF];
+  const int32_t (&perm)[Op::ST][Op::NFACES];
+  const double (&wface)[Op::NF];
+  const double (&q)[Op::NP][Op::ND];
+  const double (&dFo)[Op::NFACES][Op::NF][Op::ND][Op::ND];
+  const double (&dFn)[Op::NFACES][Op::NF][Op::ND][Op::ND];
+  const ElFace (&rec)[Op::NFACES];
+  const int32_t (&kown)[Op::NFACES][Op::NF];
+  const int32_t (&knbr)[Op::NFACES][Op::NF];
+  const double (&sgn)[Op::NFACES];
+  __device__ __forceinline__ JacView(const JacSmem<Op, VOL, FLUX, EPB>& s, const JacElem<Op, VOL, FLUX>& x)
+      : interp(s.interp), perm(s.perm), wface(s.wface), q(x.q), dFo(x.dFo), dFn(x.dFn), rec(x.rec), kown(x.kown),
+        knbr(x.knbr), sgn(x.sgn) {}
 };
 
 template <class BT> __device__ __forceinline__ BT to_block(double x) { return (BT)x; }
@@ -200,6 +253,75 @@ __device__ __forceinline__ void eslf_nbr_block(const Sm& sm, const DevSBP& sbp, 
     }
 }
 
+// own block (i, j) of an entropy-stable operator: face f's contribution
+// (interior: the entropy-stable integral; boundary: the Roe flux against the
+// boundary state)
+template <class Op, class Sm>
+__device__ __forceinline__ void es_own_face(const Sm& sm, const DevSBP& sbp, const DevMesh& mesh,
+                                            const PhysConst& phys, const double* qin, int f, int i, int j, int si,
+                                            int sj, double (*B)[Op::ND]) {
+  constexpr int NF = Op::NF, ND = Op::ND;
+  if (sm.rec[f].x >= 0) {
+    eslf_own_block<Op>(sm, sbp, mesh, phys, qin, f, i, j, si, sj, B);
+    return;
+  }
+  for (int k = 0; k < NF; ++k) {
+    const int m = sm.kown[f][k];
+    const double wgt = sm.sgn[f] * sm.wface[m] * sm.interp[si][m] * sm.interp[sj][m];
+#pragma unroll
+    for (int a = 0; a < ND; ++a)
+#pragma unroll
+      for (int c = 0; c < ND; ++c) B[a][c] += wgt * sm.dFo[f][k][a][c];
+  }
+}
+
+// the flux at a face node as a function of one seeded component: side 0 is
+// elementL's state, side 1 elementR's (qs: both states; comp of `side` seeded)
+template <class Op, int FLUX>
+__device__ __forceinline__ void face_derivative(const PhysConst& phys, const double (*qs)[Op::ND], int side, int comp,
+                                                const double* nrm, double scale, double* dF) {
+  constexpr int DIM = Op::DIM, ND = Op::ND;
+  dual<1> qL[ND], qR[ND], F[ND];
+#pragma unroll
+  for (int c = 0; c < ND; ++c) {
+    qL[c] = dual<1>(qs[0][c]);
+    qL[c].d[0] = side == 0 && c == comp ? 1.0 : 0.0;
+    qR[c] = dual<1>(qs[1][c]);
+    qR[c].d[0] = side == 1 && c == comp ? 1.0 : 0.0;
+  }
+  if constexpr (FLUX == PDES_FLUX_ROE) {
+    roe_flux<DIM>(phys, qL, qR, nrm, F);
+  } else if constexpr (FLUX == PDES_FLUX_IRSLF) {
+    irslf_flux<DIM>(phys, qL, qR, nrm, F);
+  } else {
+    // entropy penalty (calcEntropyPenaltyIntegral, faceElementIntegrals.jl:
+    // 199-290) of the interpolated IR entropy variables
+    dual<1> qa[ND], qlr[ND], dw[ND];
+    ir_to_conservative<DIM>(phys, qL, qa);
+    ir_to_conservative<DIM>(phys, qR, qlr);
+#pragma unroll
+    for (int c = 0; c < ND; ++c) {
+      qa[c] = 0.5 * (qa[c] + qlr[c]);
+      dw[c] = qL[c] - qR[c];
+      F[c] = dual<1>(0.0);
+    }
+    lf_entropy_apply<DIM>(phys, qa, dw, nrm, scale, F);
+  }
+#pragma unroll
+  for (int a = 0; a < ND; ++a) dF[a] = F[a].d[0];
+}
+
+// elements per workgroup: as many as give every thread about one row of
+// values (weak form: NP ndof^2 of them) or one volume pair column, in at most
+// 40 KB of LDS, so that four workgroups fit a CU
+template <class Op, int VOL, int FLUX>
+constexpr int jac_epb() {
+  constexpr int per = VOL == VOL_WEAK ? Op::NP * Op::ND * Op::ND : Op::NP * JacElem<Op, VOL, FLUX>::KP;
+  constexpr int fit = 40960 / (int)sizeof(JacElem<Op, VOL, FLUX>), want = 256 / per;
+  constexpr int n = want < fit ? want : fit;
+  return n < 1 ? 1 : n;
+}
+
 template <class Op, int VOL, int FLUX, class BT>
 __global__ void __launch_bounds__(256)
 euler_jacobian_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys, const double* __restrict__ qin,
@@ -207,27 +329,36 @@ euler_jacobian_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys, const double* __
                       BT* __restrict__ vals, int32_t* __restrict__ err,
                       const double* __restrict__ ptc_diag, const double* __restrict__ ptc_scale) {
   constexpr int DIM = Op::DIM, NP = Op::NP, NF = Op::NF, ST = Op::ST, ND = Op::ND, NFACES = Op::NFACES;
-  constexpr int NB = ND * ND;
-  using Smem = JacSmem<Op, VOL, FLUX>;
-  __shared__ Smem sm;
+  constexpr int NB = ND * ND, T = 256, SLOTS = NFACES * NF;
+  constexpr int EPB = jac_epb<Op, VOL, FLUX>();
+  constexpr bool ES = FLUX == PDES_FLUX_ESLF;
+  using Elem = JacElem<Op, VOL, FLUX>;
+  __shared__ JacSmem<Op, VOL, FLUX, EPB> sm;
   const int tid = threadIdx.x;
-  const int64_t e = element_of(mesh, blockIdx.x);
-  for (int x = tid; x < DIM * NP * NP; x += blockDim.x) (&sm.Q[0][0][0])[x] = sbp.Q[x];
-  for (int x = tid; x < ST * NF; x += blockDim.x) (&sm.interp[0][0])[x] = sbp.interp[x];
-  for (int x = tid; x < ST * NFACES; x += blockDim.x) (&sm.perm[0][0])[x] = sbp.perm[x];
-  for (int x = tid; x < NP * NFACES; x += blockDim.x) (&sm.nodepos[0][0])[x] = sbp.nodepos[x];
-  for (int x = tid; x < NF; x += blockDim.x) sm.wface[x] = sbp.wface[x];
-  for (int x = tid; x < NP * ND; x += blockDim.x) (&sm.q[0][0])[x] = qin[e * NP * ND + x];
-  if (tid < NFACES) {
-    ElFace r = mesh.elface[e * NFACES + tid];
-    sm.rec[tid] = r;
-    const int side = (r.x >= 0) ? ((r.z >> 16) & 1) : 0;
-    sm.sgn[tid] = side == 0 ? -1.0 : 1.0;
+  const int64_t s0 = (int64_t)blockIdx.x * EPB;
+  const int nel = (int)(launch_count(mesh) - s0 < EPB ? launch_count(mesh) - s0 : EPB);
+  for (int x = tid; x < DIM * NP * NP; x += T) (&sm.Q[0][0][0])[x] = sbp.Q[x];
+  for (int x = tid; x < ST * NF; x += T) (&sm.interp[0][0])[x] = sbp.interp[x];
+  for (int x = tid; x < ST * NFACES; x += T) (&sm.perm[0][0])[x] = sbp.perm[x];
+  for (int x = tid; x < NP * NFACES; x += T) (&sm.nodepos[0][0])[x] = sbp.nodepos[x];
+  for (int x = tid; x < NF; x += T) sm.wface[x] = sbp.wface[x];
+  for (int t = tid; t < nel * NP * ND; t += T) {
+    const int l = t / (NP * ND), x = t - l * (NP * ND);
+    (&sm.el[l].q[0][0])[x] = qin[element_of(mesh, s0 + l) * NP * ND + x];
+  }
+  for (int t = tid; t < nel * NFACES; t += T) {
+    const int l = t / NFACES, f = t - l * NFACES;
+    const int64_t e = element_of(mesh, s0 + l);
+    const ElFace r = mesh.elface[e * NFACES + f];
+    sm.el[l].e = e;
+    sm.el[l].rec[f] = r;
+    sm.el[l].sgn[f] = r.x >= 0 && ((r.z >> 16) & 1) ? 1.0 : -1.0;
   }
   __syncthreads();
-  for (int t = tid; t < NFACES * NF; t += blockDim.x) {
-    const int f = t / NF, k = t - f * NF;
-    const ElFace r = sm.rec[f];
+  for (int t = tid; t < nel * SLOTS; t += T) {
+    const int l = t / SLOTS, f = (t - l * SLOTS) / NF, k = t % NF;
+    Elem& el = sm.el[l];
+    const ElFace r = el.rec[f];
     int ko = k, kn = k;
     if (r.x >= 0) {
       const int o = (r.z >> 8) & 0xff;
@@ -236,280 +367,342 @@ euler_jacobian_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys, const double* __
       ko = side == 0 ? k : kR;
       kn = side == 0 ? kR : k;
     }
-    sm.kown[f][k] = ko;
-    sm.knbr[f][k] = kn;
+    el.kown[f][k] = ko;
+    el.knbr[f][k] = kn;
+    el.kslot[f][ko] = k;
+    if constexpr (Op::DIAGE) {
+      // slot k couples own node perm[ko][f] with neighbour node perm[kn][fN]
+      int64_t pos = -1;
+      if (r.x >= 0) {
+        pos = bsr_find(rowptr, colind, el.e * NP + sm.perm[ko][f], (int32_t)((int64_t)r.x * NP + sm.perm[kn][r.z & 0xff]));
+        if (pos < 0) err[0] = 1;
+      }
+      el.nbr_run[f][k] = pos;
+    }
   }
-
-  // ---- point derivatives
-  if constexpr (VOL == VOL_WEAK) {
-    for (int t = tid; t < NP * DIM; t += blockDim.x) {
-      const int j = t / DIM, d = t - j * DIM;
-      dual<ND> qd[ND];
+  // where each row's runs of NP blocks begin: own, and per neighbour for dense faces
+  constexpr int RUNS = Op::DIAGE ? 1 : 1 + NFACES;
+  for (int t = tid; t < nel * NP * RUNS; t += T) {
+    const int l = t / (NP * RUNS), x = t - l * (NP * RUNS), f = x / NP - 1, i = x % NP;
+    Elem& el = sm.el[l];
+    const int64_t ce = f < 0 ? el.e : (int64_t)el.rec[f].x;
+    int64_t pos = -1;
+    if (ce >= 0) {
+      pos = bsr_find(rowptr, colind, el.e * NP + i, (int32_t)(ce * NP));
+      if (pos < 0 || colind[pos + NP - 1] != ce * NP + NP - 1) { err[0] = 1; pos = -1; }
+    }
+    if (f < 0) el.own_run[i] = pos;
+    else if constexpr (!Op::DIAGE) el.nbr_run[f][i] = pos;
+  }
+  // states at the face nodes, one thread per (slot, side, component)
+  for (int t = tid; t < nel * SLOTS * 2 * ND; t += T) {
+    const int l = t / (SLOTS * 2 * ND);
+    int x = t - l * (SLOTS * 2 * ND);
+    const int c = x % ND, sd = (x / ND) & 1;
+    x /= 2 * ND;
+    const int f = x / NF, k = x - f * NF;
+    Elem& el = sm.el[l];
+    const ElFace r = el.rec[f];
+    double v = 0.0;
+    if (r.x < 0) {
+      if (sd == 0)
+        for (int s = 0; s < ST; ++s) v += sm.interp[s][k] * el.q[sm.perm[s][f]][c];
+      else
+        v = mesh.qbc[((int64_t)r.y * NF + k) * ND + c];
+    } else {
+      const int fN = r.z & 0xff, side = (r.z >> 16) & 1, o = (r.z >> 8) & 0xff;
+      const int kk = sd == 0 ? k : sbp.nbrperm[k * sbp.norient + o];
+      const bool own = sd == side;
+      const double* qnb = qin + (int64_t)r.x * NP * ND;
+      for (int s = 0; s < ST; ++s) {
+        if constexpr (ES) {
+          double qs[ND], w[ND];
 #pragma unroll
-      for (int c = 0; c < ND; ++c) { qd[c] = dual<ND>(sm.q[j][c]); qd[c].d[c] = 1.0; }
+          for (int a = 0; a < ND; ++a) qs[a] = own ? el.q[sm.perm[s][f]][a] : qnb[sm.perm[s][fN] * ND + a];
+          to_ir_vars<DIM>(phys, qs, w);
+          double wc = w[0];
+#pragma unroll
+          for (int a = 1; a < ND; ++a) wc = a == c ? w[a] : wc;
+          v += sm.interp[s][kk] * wc;
+        } else {
+          v += sm.interp[s][kk] * (own ? el.q[sm.perm[s][f]][c] : qnb[sm.perm[s][fN] * ND + c]);
+        }
+      }
+    }
+    el.qf[f][k][sd][c] = v;
+  }
+  if constexpr (VOL == VOL_WEAK) {
+    for (int t = tid; t < nel * NP * DIM * ND; t += T) {
+      const int l = t / (NP * DIM * ND);
+      int x = t - l * (NP * DIM * ND);
+      const int comp = x % ND, d = (x / ND) % DIM, j = x / (ND * DIM);
+      Elem& el = sm.el[l];
+      dual<1> qd[ND], F[ND];
+#pragma unroll
+      for (int c = 0; c < ND; ++c) { qd[c] = dual<1>(el.q[j][c]); qd[c].d[0] = c == comp ? 1.0 : 0.0; }
       double nrm[DIM];
 #pragma unroll
-      for (int x = 0; x < DIM; ++x) nrm[x] = metric<DIM, NP>(mesh, e, j)[x * DIM + d];
-      dual<ND> F[ND];
+      for (int y = 0; y < DIM; ++y) nrm[y] = metric<DIM, NP>(mesh, el.e, j)[y * DIM + d];
       euler_flux<DIM>(phys, qd, nrm, F);
 #pragma unroll
-      for (int r = 0; r < ND; ++r)
-#pragma unroll
-        for (int c = 0; c < ND; ++c) sm.A[j * DIM + d][r][c] = F[r].d[c];
+      for (int r = 0; r < ND; ++r) el.A[j * DIM + d][r][comp] = F[r].d[0];
     }
-  }
-  __syncthreads();
-  for (int t = tid; t < NFACES * NF; t += blockDim.x) {
-    const int f = t / NF, k = t - f * NF;
-    const ElFace r = sm.rec[f];
-    dual<2 * ND> qL[ND], qR[ND], F[ND];
-    if (r.x < 0) {
-      // boundary: seed the interior state (directions 0..ND-1)
+  } else {
+    for (int t = tid; t < nel * NP * ND; t += T) {
+      const int l = t / (NP * ND), j = (t - l * (NP * ND)) / ND, comp = t % ND;
+      Elem& el = sm.el[l];
+      dual<1> qd[ND], z[ND];
 #pragma unroll
-      for (int c = 0; c < ND; ++c) {
-        double v = 0.0;
-        for (int s = 0; s < ST; ++s) v += sm.interp[s][k] * sm.q[sm.perm[s][f]][c];
-        qL[c] = dual<2 * ND>(v);
-        qL[c].d[c] = 1.0;
+      for (int c = 0; c < ND; ++c) { qd[c] = dual<1>(el.q[j][c]); qd[c].d[0] = c == comp ? 1.0 : 0.0; }
+      ir_zvars<DIM>(phys, qd, z);
+#pragma unroll
+      for (int r = 0; r < ND; ++r) el.dz[j][r][comp] = z[r].d[0];
+      if (comp == 0) {
+#pragma unroll
+        for (int r = 0; r < ND; ++r) el.z[j][r] = z[r].v;
       }
-      double qg[ND];
-      bc_state<DIM>(mesh, r, k, NF, qg);
-#pragma unroll
-      for (int c = 0; c < ND; ++c) qR[c] = dual<2 * ND>(qg[c]);
-      roe_flux<DIM>(phys, qL, qR, mesh.nrm_bndry + ((int64_t)r.y * NF + k) * DIM, F);
-#pragma unroll
-      for (int a = 0; a < ND; ++a)
-#pragma unroll
-        for (int c = 0; c < ND; ++c) { sm.dFo[f][k][a][c] = F[a].d[c]; sm.dFn[f][k][a][c] = 0.0; }
-    } else if constexpr (FLUX == PDES_FLUX_ESLF) {
-      // entropy penalty at face node k (calcEntropyPenaltyIntegral,
-      // faceElementIntegrals.jl:199-290) as a function of the interpolated
-      // IR entropy variables wl, wr: dP/dw_own and dP/dw_nbr; the chain
-      // through dw/dq of each stencil node is applied in the block tasks
-      const int fN = r.z & 0xff;
-      const int side = (r.z >> 16) & 1;
-      const int o = (r.z >> 8) & 0xff;
-      const int kR = sbp.nbrperm[k * sbp.norient + o];
-      const double* qnb = qin + r.x * NP * ND;
-      double wlv[ND], wrv[ND];
-#pragma unroll
-      for (int c = 0; c < ND; ++c) { wlv[c] = 0.0; wrv[c] = 0.0; }
-      for (int sn = 0; sn < ST; ++sn) {
-        double qo[ND], qn[ND], wo[ND], wn[ND];
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          qo[c] = sm.q[sm.perm[sn][f]][c];
-          qn[c] = qnb[sm.perm[sn][fN] * ND + c];
-        }
-        to_ir_vars<DIM>(phys, qo, wo);
-        to_ir_vars<DIM>(phys, qn, wn);
-        const double rl = sm.interp[sn][k], rr = sm.interp[sn][kR];
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          wlv[c] += rl * (side == 0 ? wo[c] : wn[c]);
-          wrv[c] += rr * (side == 0 ? wn[c] : wo[c]);
-        }
-      }
-      dual<2 * ND> wl[ND], wr[ND], qa[ND], qlr[ND], dw[ND];
-#pragma unroll
-      for (int c = 0; c < ND; ++c) {
-        wl[c] = dual<2 * ND>(wlv[c]);
-        wl[c].d[c] = 1.0;
-        wr[c] = dual<2 * ND>(wrv[c]);
-        wr[c].d[ND + c] = 1.0;
-      }
-      ir_to_conservative<DIM>(phys, wl, qa);
-      ir_to_conservative<DIM>(phys, wr, qlr);
-#pragma unroll
-      for (int c = 0; c < ND; ++c) {
-        qa[c] = 0.5 * (qa[c] + qlr[c]);
-        dw[c] = wl[c] - wr[c];
-        F[c] = dual<2 * ND>(0.0);
-      }
-      lf_entropy_apply<DIM>(phys, qa, dw, mesh.nrm_face + ((int64_t)r.y * NF + k) * DIM, sm.wface[k], F);
-      const int oo = side == 0 ? 0 : ND, on = side == 0 ? ND : 0;
-#pragma unroll
-      for (int a = 0; a < ND; ++a)
-#pragma unroll
-        for (int c = 0; c < ND; ++c) { sm.dFo[f][k][a][c] = F[a].d[oo + c]; sm.dFn[f][k][a][c] = F[a].d[on + c]; }
-    } else {
-      const int64_t nb = r.x;
-      const int fN = r.z & 0xff;
-      const int side = (r.z >> 16) & 1;
-      const int kR = sm.kown[f][k] == k ? sm.knbr[f][k] : sm.kown[f][k];
-      const int fL = side == 0 ? f : fN, fR = side == 0 ? fN : f;
-      const double* qnb = qin + nb * NP * ND;
-#pragma unroll
-      for (int c = 0; c < ND; ++c) {
-        double vl = 0.0, vr = 0.0;
-        // own side from LDS, neighbour side from global memory (separate
-        // branches: no pointer select across address spaces)
-        if (side == 0) {
-          for (int s = 0; s < ST; ++s) {
-            vl += sm.interp[s][k] * sm.q[sm.perm[s][fL]][c];
-            vr += sm.interp[s][kR] * qnb[sm.perm[s][fR] * ND + c];
-          }
-        } else {
-          for (int s = 0; s < ST; ++s) {
-            vl += sm.interp[s][k] * qnb[sm.perm[s][fL] * ND + c];
-            vr += sm.interp[s][kR] * sm.q[sm.perm[s][fR]][c];
-          }
-        }
-        qL[c] = dual<2 * ND>(vl);
-        qL[c].d[c] = 1.0;
-        qR[c] = dual<2 * ND>(vr);
-        qR[c].d[ND + c] = 1.0;
-      }
-      const double* nrm = mesh.nrm_face + ((int64_t)r.y * NF + k) * DIM;
-      if constexpr (FLUX == PDES_FLUX_ROE) roe_flux<DIM>(phys, qL, qR, nrm, F);
-      else irslf_flux<DIM>(phys, qL, qR, nrm, F);
-      const int oo = side == 0 ? 0 : ND, on = side == 0 ? ND : 0;
-#pragma unroll
-      for (int a = 0; a < ND; ++a)
-#pragma unroll
-        for (int c = 0; c < ND; ++c) { sm.dFo[f][k][a][c] = F[a].d[oo + c]; sm.dFn[f][k][a][c] = F[a].d[on + c]; }
     }
   }
   __syncthreads();
 
-  // ---- blocks of this element's rows
-  // tasks: own blocks (i, j), then per face f the neighbour blocks
-  constexpr int NBFACE = Op::DIAGE ? NF : NP * NP;
-  const int ntask = NP * NP + NFACES * NBFACE;
-  for (int t = tid; t < ntask; t += blockDim.x) {
-    double B[ND][ND];
+  // ---- face derivatives, one thread per (slot, side, component)
+  for (int t = tid; t < nel * SLOTS * 2 * ND; t += T) {
+    const int l = t / (SLOTS * 2 * ND);
+    int x = t - l * (SLOTS * 2 * ND);
+    const int comp = x % ND, sd = (x / ND) & 1;
+    x /= 2 * ND;
+    const int f = x / NF, k = x - f * NF;
+    Elem& el = sm.el[l];
+    const ElFace r = el.rec[f];
+    double dF[ND];
+    if (r.x < 0) {
+      if (sd == 0) face_derivative<Op, PDES_FLUX_ROE>(phys, el.qf[f][k], 0, comp, mesh.nrm_bndry + ((int64_t)r.y * NF + k) * DIM, 1.0, dF);
+    } else {
+      face_derivative<Op, FLUX>(phys, el.qf[f][k], sd, comp, mesh.nrm_face + ((int64_t)r.y * NF + k) * DIM,
+                                sm.wface[k], dF);
+    }
+    const bool own = r.x < 0 ? sd == 0 : sd == ((r.z >> 16) & 1);
+    if (r.x < 0 && sd == 1) {
 #pragma unroll
-    for (int a = 0; a < ND; ++a)
+      for (int a = 0; a < ND; ++a) dF[a] = 0.0;
+    }
 #pragma unroll
-      for (int c = 0; c < ND; ++c) B[a][c] = 0.0;
-    int64_t row, col;
-    if (t < NP * NP) {
-      const int i = t / NP, j = t - i * NP;
-      row = e * NP + i;
-      col = e * NP + j;
-      if constexpr (VOL == VOL_WEAK) {
-        // d/dq_j of sum_d Q_d[j][i] F_d(q_j)
+    for (int a = 0; a < ND; ++a) (own ? el.dFo : el.dFn)[f][k][a][comp] = dF[a];
+  }
+  __syncthreads();
+
+  if constexpr (Elem::CW) {
+    for (int t = tid; t < nel * NP * SLOTS; t += T) {
+      const int l = t / (NP * SLOTS), x = t - l * (NP * SLOTS), i = x / SLOTS, f = (x % SLOTS) / NF, k = x % NF;
+      Elem& el = sm.el[l];
+      const int m = el.kown[f][k], si = sm.nodepos[i][f];
+      el.cw[f][i][k] = si >= 0 ? el.sgn[f] * sm.wface[m] * sm.interp[si][m] : 0.0;
+    }
+    __syncthreads();
+  }
+
+  // ---- blocks of the elements' rows
+  // a face's contribution to the value `ent` of the own block (i, i) of a
+  // diagonal-E operator
+  auto diage_face = [&](const Elem& el, int i, int ent) {
+    double v = 0.0;
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-          const double qji = sm.Q[d][j][i];
+    for (int f = 0; f < NFACES; ++f) {
+      const int si = sm.nodepos[i][f];
+      if (si < 0) continue;
+      v += el.sgn[f] * sm.wface[si] * (&el.dFo[f][el.kslot[f][si]][0][0])[ent];
+    }
+    return v;
+  };
+  // implicit-Euler globalization (applyEuler, globalization.jl): -M/tau_vec on the diagonal
+  auto ptc_term = [&](const Elem& el, int i, int ent) {
+    if (!ptc_scale || ent % (ND + 1) != 0) return 0.0;
+    return ptc_diag[el.e * NP + i] * ptc_scale[mesh.el_inst ? mesh.el_inst[el.e] : 0];
+  };
+
+  if constexpr (VOL == VOL_WEAK) {
+    // lane (j, ent): value ent of column j, for every row i in turn, so that a
+    // row's run of NP blocks is stored by consecutive lanes
+    constexpr int JE = NP * NB;
+    for (int t = tid; t < nel * JE; t += T) {
+      const int l = t / JE, je = t - l * JE, j = je / NB, ent = je - j * NB;
+      const Elem& el = sm.el[l];
+      double Aq[DIM];
 #pragma unroll
-          for (int a = 0; a < ND; ++a)
+      for (int d = 0; d < DIM; ++d) Aq[d] = (&el.A[j * DIM + d][0][0])[ent];
+      if constexpr (Op::DIAGE) {
+#pragma unroll 1
+        for (int i = 0; i < NP; ++i) {
+          double v = 0.0;
 #pragma unroll
-            for (int c = 0; c < ND; ++c) B[a][c] += qji * sm.A[j * DIM + d][a][c];
+          for (int d = 0; d < DIM; ++d) v += sm.Q[d][j][i] * Aq[d];
+          if (i == j) v = v + diage_face(el, i, ent) - ptc_term(el, i, ent);
+          if (el.own_run[i] >= 0) vals[(el.own_run[i] + j) * NB + ent] = to_block<BT>(v);
         }
       } else {
-        // split form: res_i -= sum_k 2 S_ik F*(q_i, q_k) (reference orientation F(q_max, q_min))
-        for (int k = 0; k < NP; ++k) {
-          if (k == i) continue;
-          if (i != j && k != j) continue;
-          const int hi = i > k ? i : k, lo = i > k ? k : i;
-          dual<2 * ND> qa[ND], qb[ND];
+        double P[NFACES][NF];
 #pragma unroll
-          for (int c = 0; c < ND; ++c) {
-            qa[c] = dual<2 * ND>(sm.q[hi][c]); qa[c].d[c] = 1.0;
-            qb[c] = dual<2 * ND>(sm.q[lo][c]); qb[c].d[ND + c] = 1.0;
+        for (int f = 0; f < NFACES; ++f) {
+          const int sj = sm.nodepos[j][f];
+#pragma unroll
+          for (int k = 0; k < NF; ++k)
+            P[f][k] = sj >= 0 ? sm.interp[sj][el.kown[f][k]] * (&el.dFo[f][k][0][0])[ent] : 0.0;
+        }
+#pragma unroll 1
+        for (int i = 0; i < NP; ++i) {
+          double v = 0.0;
+#pragma unroll
+          for (int d = 0; d < DIM; ++d) v += sm.Q[d][j][i] * Aq[d];
+#pragma unroll
+          for (int f = 0; f < NFACES; ++f) {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) v += el.cw[f][i][k] * P[f][k];
           }
-          dual<2 * ND> za[ND], zb[ND], Fd[DIM * ND];
-          ir_zvars<DIM>(phys, qa, za);
-          ir_zvars<DIM>(phys, qb, zb);
-          double nrmD[DIM * DIM];
+          if (i == j) v -= ptc_term(el, i, ent);
+          if (el.own_run[i] >= 0) vals[(el.own_run[i] + j) * NB + ent] = to_block<BT>(v);
+        }
 #pragma unroll
-          for (int x = 0; x < DIM; ++x)
+        for (int f = 0; f < NFACES; ++f) {
+          const ElFace r = el.rec[f];
+          if (r.x < 0) continue;
+          const int sj = sbp.nodepos[j * NFACES + (r.z & 0xff)];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) nrmD[x * DIM + d] = metric<DIM, NP>(mesh, e, hi)[x * DIM + d];
-          ir_flux_z<DIM, DIM>(phys, za, zb, nrmD, Fd);
-          // derivative w.r.t. q_j: directions of hi or lo
-          const int off = (j == hi) ? 0 : ND;
+          for (int k = 0; k < NF; ++k)
+            P[f][k] = sj >= 0 ? sm.interp[sj][el.knbr[f][k]] * (&el.dFn[f][k][0][0])[ent] : 0.0;
+#pragma unroll 1
+          for (int i = 0; i < NP; ++i) {
+            double v = 0.0;
 #pragma unroll
-          for (int d = 0; d < DIM; ++d) {
-            const double s_ik = 0.5 * (sm.Q[d][i][k] - sm.Q[d][k][i]);
-#pragma unroll
-            for (int a = 0; a < ND; ++a)
-#pragma unroll
-              for (int c = 0; c < ND; ++c) B[a][c] -= 2 * s_ik * Fd[d * ND + a].d[off + c];
+            for (int k = 0; k < NF; ++k) v += el.cw[f][i][k] * P[f][k];
+            if (el.nbr_run[f][i] >= 0) vals[(el.nbr_run[f][i] + j) * NB + ent] = to_block<BT>(v);
           }
         }
       }
-      // face and boundary terms with both indices on this element
+    }
+  } else {
+    // split form: res_i -= sum_k 2 S_ik F*(q_i, q_k).  With D the derivative
+    // with respect to q_c of the flux of the pair (c, r) in the direction
+    // sum_d 2 S_d[c][r] dxidx_d, block (r, c) is +D and block (c, c) collects
+    // -D.  Thread (c, part) takes the rows r = part, part + KP, ...
+    constexpr int KP = Elem::KP;
+    for (int t = tid; t < nel * NP * KP; t += T) {
+      const int l = t / (NP * KP), x = t - l * (NP * KP), c = x / KP, part = x - c * KP;
+      Elem& el = sm.el[l];
+      dual<ND> zc[ND];
 #pragma unroll
-      for (int f = 0; f < NFACES; ++f) {
-        const int si = sm.nodepos[i][f], sj = sm.nodepos[j][f];
-        if (si < 0 || sj < 0) continue;
-        const double sg = sm.sgn[f];
-        if constexpr (Op::DIAGE) {
-          if (i != j) continue;
-          // own face node si; find the slot k with kown == si
-          int k = 0;
-          for (int kk = 0; kk < NF; ++kk) if (sm.kown[f][kk] == si) k = kk;
-          const double wgt = sg * sm.wface[si];
+      for (int a = 0; a < ND; ++a) {
+        zc[a].v = el.z[c][a];
 #pragma unroll
-          for (int a = 0; a < ND; ++a)
+        for (int b = 0; b < ND; ++b) zc[a].d[b] = el.dz[c][a][b];
+      }
+      double dg[ND][ND];
 #pragma unroll
-            for (int c = 0; c < ND; ++c) B[a][c] += wgt * sm.dFo[f][k][a][c];
-        } else if (FLUX == PDES_FLUX_ESLF && sm.rec[f].x >= 0) {
-          if constexpr (FLUX == PDES_FLUX_ESLF) eslf_own_block<Op>(sm, sbp, mesh, phys, qin, f, i, j, si, sj, B);
-        } else {
-          for (int k = 0; k < NF; ++k) {
-            const int m = sm.kown[f][k];
-            const double wgt = sg * sm.wface[m] * sm.interp[si][m] * sm.interp[sj][m];
+      for (int a = 0; a < ND; ++a)
 #pragma unroll
-            for (int a = 0; a < ND; ++a)
+        for (int b = 0; b < ND; ++b) dg[a][b] = 0.0;
+      for (int r = part; r < NP; r += KP) {
+        if (r == c) continue;
+        const double* mt = metric<DIM, NP>(mesh, el.e, r > c ? r : c);
+        double n[DIM], zr[ND];
 #pragma unroll
-              for (int c = 0; c < ND; ++c) B[a][c] += wgt * sm.dFo[f][k][a][c];
-          }
+        for (int y = 0; y < DIM; ++y) {
+          n[y] = 0.0;
+#pragma unroll
+          for (int d = 0; d < DIM; ++d) n[y] += (sm.Q[d][c][r] - sm.Q[d][r][c]) * mt[y * DIM + d];
         }
-      }
-      // implicit-Euler globalization (applyEuler, globalization.jl): -M/tau_vec on the diagonal
-      if (ptc_scale && i == j) {
-        const double s = ptc_scale[mesh.el_inst ? mesh.el_inst[e] : 0];
-        const double d = ptc_diag[e * NP + i] * s;
 #pragma unroll
-        for (int a = 0; a < ND; ++a) B[a][a] -= d;
-      }
-    } else {
-      const int tt = t - NP * NP;
-      const int f = tt / NBFACE, u = tt - f * NBFACE;
-      const ElFace r = sm.rec[f];
-      if (r.x < 0) continue;  // boundary face: no neighbour block
-      const int fN = r.z & 0xff;
-      const double sg = sm.sgn[f];
-      if constexpr (Op::DIAGE) {
-        // slot k couples own node perm[kown][f] with neighbour node perm[knbr][fN]
-        const int k = u;
-        const int m = sm.kown[f][k], mn = sm.knbr[f][k];
-        row = e * NP + sm.perm[m][f];
-        col = (int64_t)r.x * NP + sm.perm[mn][fN];
-        const double wgt = sg * sm.wface[m];
+        for (int a = 0; a < ND; ++a) zr[a] = el.z[r][a];
+        dual<ND> F[ND];
+        ir_flux_z<DIM, 1>(phys, zc, zr, n, F);
+        double B[ND][ND];
 #pragma unroll
         for (int a = 0; a < ND; ++a)
 #pragma unroll
-          for (int c = 0; c < ND; ++c) B[a][c] = wgt * sm.dFn[f][k][a][c];
-      } else {
-        const int i = u / NP, jn = u - i * NP;
-        row = e * NP + i;
-        col = (int64_t)r.x * NP + jn;
-        const int si = sm.nodepos[i][f], sj = sbp.nodepos[jn * NFACES + fN];
-        if constexpr (FLUX == PDES_FLUX_ESLF) {
-          if (si >= 0 && sj >= 0) eslf_nbr_block<Op>(sm, sbp, mesh, phys, qin, f, jn, si, sj, B);
-        } else if (si >= 0 && sj >= 0) {
-          for (int k = 0; k < NF; ++k) {
-            const int m = sm.kown[f][k], mn = sm.knbr[f][k];
-            const double wgt = sg * sm.wface[m] * sm.interp[si][m] * sm.interp[sj][mn];
+          for (int b = 0; b < ND; ++b) {
+            dg[a][b] -= F[a].d[b];
+            B[a][b] = F[a].d[b];
+          }
+        if constexpr (ES) {
+          const JacView<Op, VOL, FLUX, EPB> vw(sm, el);
+#pragma unroll
+          for (int f = 0; f < NFACES; ++f) {
+            const int sr = sm.nodepos[r][f], sc = sm.nodepos[c][f];
+            if (sr < 0 || sc < 0) continue;
+            es_own_face<Op>(vw, sbp, mesh, phys, qin, f, r, c, sr, sc, B);
+          }
+        }
+        if (el.own_run[r] >= 0) {
+          BT* dst = vals + (el.own_run[r] + c) * NB;
+#pragma unroll
+          for (int a = 0; a < ND; ++a)
+#pragma unroll
+            for (int b = 0; b < ND; ++b) dst[a * ND + b] = to_block<BT>(B[a][b]);
+        }
+      }
+      if constexpr (ES) {
+        if (part == 0) {
+          const JacView<Op, VOL, FLUX, EPB> vw(sm, el);
+#pragma unroll
+          for (int f = 0; f < NFACES; ++f) {
+            const int sc = sm.nodepos[c][f];
+            if (sc >= 0) es_own_face<Op>(vw, sbp, mesh, phys, qin, f, c, c, sc, sc, dg);
+          }
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < ND; ++a)
+#pragma unroll
+        for (int b = 0; b < ND; ++b) el.diag[c][part][a][b] = dg[a][b];
+    }
+    __syncthreads();
+    for (int t = tid; t < nel * NP * NB; t += T) {
+      const int l = t / (NP * NB), c = (t - l * (NP * NB)) / NB, ent = t % NB;
+      const Elem& el = sm.el[l];
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < KP; ++k) v += (&el.diag[c][k][0][0])[ent];
+      if constexpr (Op::DIAGE) v += diage_face(el, c, ent);
+      v -= ptc_term(el, c, ent);
+      if (el.own_run[c] >= 0) vals[(el.own_run[c] + c) * NB + ent] = to_block<BT>(v);
+    }
+    if constexpr (ES) {
+      for (int t = tid; t < nel * NFACES * NP * NP; t += T) {
+        const int l = t / (NFACES * NP * NP), x = t - l * (NFACES * NP * NP);
+        const int f = x / (NP * NP), i = (x / NP) % NP, jn = x % NP;
+        const Elem& el = sm.el[l];
+        if (el.rec[f].x < 0) continue;
+        const int si = sm.nodepos[i][f], sj = sbp.nodepos[jn * NFACES + (el.rec[f].z & 0xff)];
+        double B[ND][ND];
+#pragma unroll
+        for (int a = 0; a < ND; ++a)
+#pragma unroll
+          for (int b = 0; b < ND; ++b) B[a][b] = 0.0;
+        if (si >= 0 && sj >= 0) {
+          const JacView<Op, VOL, FLUX, EPB> vw(sm, el);
+          eslf_nbr_block<Op>(vw, sbp, mesh, phys, qin, f, jn, si, sj, B);
+        }
+        if constexpr (!Op::DIAGE) {
+          if (el.nbr_run[f][i] >= 0) {
+            BT* dst = vals + (el.nbr_run[f][i] + jn) * NB;
 #pragma unroll
             for (int a = 0; a < ND; ++a)
 #pragma unroll
-              for (int c = 0; c < ND; ++c) B[a][c] += wgt * sm.dFn[f][k][a][c];
+              for (int b = 0; b < ND; ++b) dst[a * ND + b] = to_block<BT>(B[a][b]);
           }
         }
       }
     }
-    const int64_t pos = bsr_find(rowptr, colind, row, (int32_t)col);
-    if (pos < 0) { err[0] = 1; continue; }
-    BT* dst = vals + pos * NB;
-#pragma unroll
-    for (int a = 0; a < ND; ++a)
-#pragma unroll
-      for (int c = 0; c < ND; ++c) dst[a * ND + c] = to_block<BT>(B[a][c]);
+  }
+  if constexpr (Op::DIAGE) {
+    // the blocks across the faces
+    for (int t = tid; t < nel * SLOTS * NB; t += T) {
+      const int l = t / (SLOTS * NB), x = t - l * (SLOTS * NB), slot = x / NB, ent = x - slot * NB;
+      const int f = slot / NF, k = slot - f * NF;
+      const Elem& el = sm.el[l];
+      if (el.rec[f].x < 0 || el.nbr_run[f][k] < 0) continue;
+      vals[el.nbr_run[f][k] * NB + ent] =
+          to_block<BT>(el.sgn[f] * sm.wface[el.kown[f][k]] * (&el.dFn[f][k][0][0])[ent]);
+    }
   }
 }
 
