@@ -17,6 +17,7 @@
 #include <thread>
 
 #include "jacobian.hpp"
+#include "krylov_kernels.hpp"
 
 namespace pdes {
 int pc_setup(pdes_ctx* c, int kind);
@@ -32,8 +33,8 @@ namespace {
 
 using namespace pdes;
 
-constexpr int CHUNK = 4096;     // dofs per reduction chunk (aligned to the instance start)
-constexpr int SEG_THREADS = 256;
+constexpr int CHUNK = 1024;     // dofs per reduction chunk (aligned to the instance start)
+constexpr int SEG_THREADS = CGS_THREADS;
 
 // ---------------------------------------------------------------------------
 // kernels over the active dofs: launch index t -> element el_list[t / dpe]
@@ -43,78 +44,181 @@ __device__ __forceinline__ int64_t active_dof(const int32_t* el_list, int64_t t,
   return (int64_t)el_list[s] * dpe + (t - s * dpe);
 }
 
-// partial[c][i] = sum over chunk c of V_i . w  (wt: optional weights, then
-// sum of V_i^2 wt).  SEG_GROUP basis vectors per pass over the chunk, so w is
-// read once per group; each vector's terms are summed in the same order, and
-// reduced by the same tree, as one vector at a time would be.
-constexpr int SEG_GROUP = 8;
-__global__ void __launch_bounds__(SEG_THREADS)
-seg_dot_partial(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ w,
-                const double* __restrict__ wt, const int64_t* __restrict__ cbeg, const int32_t* __restrict__ clen,
-                const int32_t* __restrict__ clist, double* __restrict__ partial, int mstride,
-                const int32_t* __restrict__ chunk_inst, const int32_t* __restrict__ mask) {
-  __shared__ double sh[SEG_GROUP][SEG_THREADS];
-  const int c = clist[blockIdx.x];
-  if (mask && !mask[chunk_inst[c]]) return;
-  const int64_t b0 = cbeg[c];
-  const int len = clen[c];
-  for (int i0 = 0; i0 < m; i0 += SEG_GROUP) {
-    const int g_n = m - i0 < SEG_GROUP ? m - i0 : SEG_GROUP;
-    double acc[SEG_GROUP];
-#pragma unroll
-    for (int g = 0; g < SEG_GROUP; ++g) acc[g] = 0.0;
-    for (int t = threadIdx.x; t < len; t += SEG_THREADS) {
-      const int64_t k = b0 + t;
-      const double wk = wt ? wt[k] : w[k];
-#pragma unroll
-      for (int g = 0; g < SEG_GROUP; ++g) {
-        if (g < g_n) {
-          const double v = V[(int64_t)(i0 + g) * ldv + k];
-          acc[g] += wt ? v * v * wk : v * wk;
-        }
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < SEG_GROUP; ++g) sh[g][threadIdx.x] = acc[g];
-    __syncthreads();
-    for (int s = SEG_THREADS / 2; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) {
-#pragma unroll
-        for (int g = 0; g < SEG_GROUP; ++g) sh[g][threadIdx.x] += sh[g][threadIdx.x + s];
-      }
-      __syncthreads();
-    }
-    if ((int)threadIdx.x < g_n) partial[(int64_t)c * mstride + i0 + threadIdx.x] = sh[threadIdx.x][0];
+// The CGS2 step of the packed instances, one workgroup per reduction chunk, in
+// the four fused launches of the single solve (solver.hip: dots; update and
+// dots; update and norm; scale), each instance on its own chunks.  Partial
+// sums of chunk c are partial[i * nct + c]; a workgroup adds up its own
+// instance's (in chunk order, so the bits depend on the instance only).  An
+// instance of more than CGS_SELF_REDUCE chunks (262,144 dofs) has them added
+// up once, by seg_reduce_big, into sum[inst][i].  With one kernel for every dot,
+// sum, update and norm, 9 launches a step, and 4096-dof chunks, a launch of the
+// dots took 19 us and of the rest 19 us more on average in a batch of ten (8 to
+// 28 cells a side, five operators side by side); these take 13 us and there are
+// four.  1024-dof chunks: a thread then meets four entries, so that the small
+// instances spread over more of the chip.
+struct SegLists {
+  const int64_t* __restrict__ cbeg;
+  const int32_t* __restrict__ clen;
+  const int32_t* __restrict__ clist;        // chunks of the launch, by workgroup
+  const int32_t* __restrict__ chunk_inst;
+  const int32_t* __restrict__ inst_c0;
+  const int32_t* __restrict__ mask;         // 0: the instance sits out
+  int64_t nct;                              // chunks of the group
+  int mstride;
+};
+
+// h[i], i < m, of the workgroup's instance from the partial sums before
+__device__ __forceinline__ void seg_rows(const SegLists& L, int inst, const double* __restrict__ pin,
+                                         const double* __restrict__ sum, int m, double* h) {
+  const int c0 = L.inst_c0[inst], nb = L.inst_c0[inst + 1] - c0;
+  if (nb <= CGS_SELF_REDUCE) {
+    sum_partial_rows(pin + c0, m, nb, L.nct, h);
+  } else {
+    for (int i = threadIdx.x; i < m; i += SEG_THREADS) h[i] = sum[(int64_t)inst * L.mstride + i];
     __syncthreads();
   }
 }
 
-// out[inst][i] = sum of the instance's chunk partials in chunk order
-__global__ void seg_dot_reduce(const double* __restrict__ partial, int m, int mstride,
-                               const int32_t* __restrict__ inst_c0, const int32_t* __restrict__ ilist,
-                               double* __restrict__ out, const int32_t* __restrict__ mask) {
-  const int inst = ilist[blockIdx.x];
-  const int i = threadIdx.x;
-  if (i >= m || (mask && !mask[inst])) return;
-  double acc = 0.0;
-  for (int c = inst_c0[inst]; c < inst_c0[inst + 1]; ++c) acc += partial[(int64_t)c * mstride + i];
-  out[(int64_t)inst * mstride + i] = acc;
+constexpr int SEG_MAX = 64;     // coefficients of one instance (restart + 2 at most)
+
+template <int MG, bool AXPY>
+__global__ void __launch_bounds__(SEG_THREADS)
+seg_pass(SegLists L, const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ w,
+         const double* __restrict__ pin, const double* __restrict__ sum, double* __restrict__ hsave,
+         double* __restrict__ pout) {
+  constexpr int NV = 8 * MG;
+  __shared__ double sh_h[SEG_MAX];
+  __shared__ double sh_w[SEG_THREADS / 64][NV];
+  const int c = L.clist[blockIdx.x], inst = L.chunk_inst[c];
+  if (L.mask && !L.mask[inst]) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if constexpr (AXPY) {
+    seg_rows(L, inst, pin, sum, m, sh_h);
+    if (c == L.inst_c0[inst])
+      for (int i = tid; i < m; i += SEG_THREADS) hsave[(int64_t)inst * L.mstride + i] = sh_h[i];
+  }
+  const int64_t b0 = L.cbeg[c];
+  const int len = L.clen[c];
+  for (int i0 = 0; i0 < m; i0 += NV) {
+    double acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = 0.0;
+    for (int64_t t = b0 + tid; t < b0 + len; t += SEG_THREADS) {
+      double v[NV];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = i0 + i < m ? V[(int64_t)(i0 + i) * ldv + t] : 0.0;
+      double wt = w[t];
+      if (AXPY && i0 == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (i < m) wt -= sh_h[i] * v[i];
+        for (int i = NV; i < m; ++i) wt -= sh_h[i] * V[(int64_t)i * ldv + t];
+        w[t] = wt;
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[i] += v[i] * wt;
+    }
+    const double x = wave_sums<NV>(acc);
+    if (lane % (64 / NV) == 0) sh_w[wave][lane / (64 / NV)] = x;
+    __syncthreads();
+    if (tid < NV && i0 + tid < m) {
+      double y = 0.0;
+#pragma unroll
+      for (int k = 0; k < SEG_THREADS / 64; ++k) y += sh_w[k][tid];
+      pout[(int64_t)(i0 + tid) * L.nct + c] = y;
+    }
+    __syncthreads();
+  }
 }
 
-// w -= sum_i coef[inst][i] V_i   over the active dofs
-__global__ void seg_multiaxpy(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ coef,
-                              int mstride, double* __restrict__ w, const int32_t* __restrict__ el_list,
-                              const int32_t* __restrict__ el_inst, int dpe, int64_t n,
-                              const int32_t* __restrict__ mask) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
-    const int64_t k = active_dof(el_list, t, dpe);
-    const int inst = el_inst[k / dpe];
-    if (mask && !mask[inst]) continue;
-    const double* cf = coef + (int64_t)inst * mstride;
-    double acc = w[k];
-    for (int i = 0; i < m; ++i) acc -= cf[i] * V[(int64_t)i * ldv + k];
-    w[k] = acc;
+// w -= sum_i h_i V_i and the partial sum of w^2; the chunk that begins the
+// instance adds h to the first pass's coefficients: Hessenberg column j
+template <int MG>
+__global__ void __launch_bounds__(SEG_THREADS)
+seg_norm(SegLists L, const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ w,
+         const double* __restrict__ pin, const double* __restrict__ sum, const double* __restrict__ h1,
+         double* __restrict__ H, int R, int j, double* __restrict__ pout) {
+  constexpr int NV = 8 * MG;
+  __shared__ double sh_h[SEG_MAX];
+  __shared__ double sh_w[SEG_THREADS / 64];
+  const int c = L.clist[blockIdx.x], inst = L.chunk_inst[c];
+  if (L.mask && !L.mask[inst]) return;
+  const int tid = threadIdx.x;
+  seg_rows(L, inst, pin, sum, m, sh_h);
+  if (c == L.inst_c0[inst])
+    for (int i = tid; i < m; i += SEG_THREADS)
+      H[(int64_t)inst * (R + 1) * R + (int64_t)i * R + j] = h1[(int64_t)inst * L.mstride + i] + sh_h[i];
+  const int64_t b0 = L.cbeg[c];
+  const int len = L.clen[c];
+  double acc = 0.0;
+  for (int64_t t = b0 + tid; t < b0 + len; t += SEG_THREADS) {
+    double wt = w[t];
+    for (int i0 = 0; i0 < m; i0 += NV) {
+      double v[NV];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = i0 + i < m ? V[(int64_t)(i0 + i) * ldv + t] : 0.0;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (i0 + i < m) wt -= sh_h[i0 + i] * v[i];
+    }
+    w[t] = wt;
+    acc += wt * wt;
+  }
+  acc = wave_sum(acc);
+  if ((tid & 63) == 0) sh_w[tid >> 6] = acc;
+  __syncthreads();
+  if (tid == 0) {
+    double y = 0.0;
+#pragma unroll
+    for (int k = 0; k < SEG_THREADS / 64; ++k) y += sh_w[k];
+    pout[c] = y;
+  }
+}
+
+// partial sum of x^2 (times wt when given)
+__global__ void __launch_bounds__(SEG_THREADS)
+seg_square(SegLists L, const double* __restrict__ x, const double* __restrict__ wt, double* __restrict__ pout) {
+  __shared__ double sh_w[SEG_THREADS / 64];
+  const int c = L.clist[blockIdx.x];
+  if (L.mask && !L.mask[L.chunk_inst[c]]) return;
+  const int64_t b0 = L.cbeg[c];
+  const int len = L.clen[c];
+  double acc = 0.0;
+  for (int64_t t = b0 + threadIdx.x; t < b0 + len; t += SEG_THREADS) {
+    const double v = x[t];
+    acc += wt ? v * v * wt[t] : v * v;
+  }
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) sh_w[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double y = 0.0;
+#pragma unroll
+    for (int k = 0; k < SEG_THREADS / 64; ++k) y += sh_w[k];
+    pout[c] = y;
+  }
+}
+
+// sum[inst][i] = sum of the instance's chunk partials, i = blockIdx.y, for the
+// instances of more than min_chunks chunks
+__global__ void __launch_bounds__(SEG_THREADS)
+seg_reduce(SegLists L, const int32_t* __restrict__ ilist, int min_chunks, const double* __restrict__ partial,
+           double* __restrict__ sum) {
+  __shared__ double sh_w[SEG_THREADS / 64];
+  const int inst = ilist[blockIdx.x];
+  if (L.mask && !L.mask[inst]) return;
+  const int c0 = L.inst_c0[inst], c1 = L.inst_c0[inst + 1];
+  if (c1 - c0 <= min_chunks) return;
+  double acc = 0.0;
+  for (int c = c0 + threadIdx.x; c < c1; c += SEG_THREADS) acc += partial[(int64_t)blockIdx.y * L.nct + c];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) sh_w[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double y = 0.0;
+#pragma unroll
+    for (int k = 0; k < SEG_THREADS / 64; ++k) y += sh_w[k];
+    sum[(int64_t)inst * L.mstride + blockIdx.y] = y;
   }
 }
 
@@ -158,63 +262,71 @@ __global__ void seg_scale(const double* __restrict__ x, double* __restrict__ y, 
 // per-instance GMRES scalars, [inst][GS_*]
 enum { GS_BETA0 = 0, GS_RES = 1, GS_NSCAL = 2 };
 
-// sums of the chunk partials -> coef[inst][i] (the CGS coefficients) and the
-// Hessenberg column j (pass 0 stores, pass 1 adds)
-__global__ void seg_reduce_hcol(const double* __restrict__ partial, int m, int mstride,
-                                const int32_t* __restrict__ inst_c0, const int32_t* __restrict__ ilist,
-                                const int32_t* __restrict__ mask, double* __restrict__ coef, double* __restrict__ H,
-                                int R, int j, int pass) {
-  const int inst = ilist[blockIdx.x];
-  const int i = threadIdx.x;
-  if (i >= m || !mask[inst]) return;
-  double acc = 0.0;
-  for (int c = inst_c0[inst]; c < inst_c0[inst + 1]; ++c) acc += partial[(int64_t)c * mstride + i];
-  coef[(int64_t)inst * mstride + i] = acc;
-  double* h = H + (int64_t)inst * (R + 1) * R + (int64_t)i * R + j;
-  *h = pass ? *h + acc : acc;
-}
-
-// Arnoldi step j done: ||w|| is in seg[inst][0]; apply the previous Givens
-// rotations to column j, form rotation j, update g and the residual estimate,
-// and decide whether the instance keeps iterating.
-__global__ void gmres_finish_step(int nlist, const int32_t* __restrict__ ilist, int32_t* __restrict__ iter,
-                                  int32_t* __restrict__ live, int32_t* __restrict__ total, int32_t* __restrict__ jdone,
-                                  const double* __restrict__ seg, double* __restrict__ coef, int mstride,
-                                  double* __restrict__ H, double* __restrict__ cs, double* __restrict__ sn,
-                                  double* __restrict__ g, double* __restrict__ gs, int R, int j, double rtol,
-                                  double atol, int maxit) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nlist) return;
-  const int inst = ilist[t];
-  if (!iter[inst]) return;
+// Arnoldi step j: w /= ||w|| (from the partial sums of w^2), one workgroup per
+// chunk; the chunk that begins an instance also applies the previous Givens
+// rotations to column j, forms rotation j, updates g and the residual
+// estimate, and decides whether the instance keeps iterating.  (The instance's
+// other workgroups may see it stopped and leave w alone: it is not used then.)
+// The rotations are a serial chain, so the column and the rotations are staged
+// in LDS first.
+__global__ void __launch_bounds__(SEG_THREADS)
+gmres_finish_step(SegLists L, double* __restrict__ w, const double* __restrict__ pin, const double* __restrict__ sum,
+                  int32_t* __restrict__ iter, int32_t* __restrict__ live, int32_t* __restrict__ total,
+                  int32_t* __restrict__ jdone, double* __restrict__ H, double* __restrict__ cs,
+                  double* __restrict__ sn, double* __restrict__ g, double* __restrict__ gs, int R, int j, double rtol,
+                  double atol, int maxit) {
+  __shared__ double sh_h[8], sh_c[SEG_MAX], sh_s[SEG_MAX], sh_col[SEG_MAX];
+  const int c = L.clist[blockIdx.x], inst = L.chunk_inst[c];
+  __shared__ int running;
+  if (threadIdx.x == 0) running = iter[inst];     // one reading for the workgroup
+  __syncthreads();
+  if (!running) return;
+  seg_rows(L, inst, pin, sum, 1, sh_h);
+  const double hn = sqrt(sh_h[0]);
+  const double inv = hn > 0.0 ? 1.0 / hn : 0.0;
+  const int64_t b0 = L.cbeg[c];
+  const int len = L.clen[c];
+  for (int64_t t = b0 + threadIdx.x; t < b0 + len; t += SEG_THREADS) w[t] = inv * w[t];
+  if (c != L.inst_c0[inst]) return;
   double* Hi = H + (int64_t)inst * (R + 1) * R;
   double* ci = cs + (int64_t)inst * R;
   double* si = sn + (int64_t)inst * R;
   double* gi = g + (int64_t)inst * (R + 1);
-  const double hn = sqrt(seg[(int64_t)inst * mstride]);
-  Hi[(j + 1) * R + j] = hn;
-  for (int k = 0; k < j; ++k) {
-    const double a = Hi[k * R + j], b = Hi[(k + 1) * R + j];
-    Hi[k * R + j] = ci[k] * a + si[k] * b;
-    Hi[(k + 1) * R + j] = -si[k] * a + ci[k] * b;
+  for (int k = threadIdx.x; k <= j; k += SEG_THREADS) {
+    sh_col[k] = Hi[k * R + j];
+    if (k < j) {
+      sh_c[k] = ci[k];
+      sh_s[k] = si[k];
+    }
   }
-  const double a = Hi[j * R + j], b = Hi[(j + 1) * R + j];
-  const double r = hypot(a, b);
-  ci[j] = r > 0 ? a / r : 1.0;
-  si[j] = r > 0 ? b / r : 0.0;
-  Hi[j * R + j] = r;
-  Hi[(j + 1) * R + j] = 0.0;
-  gi[j + 1] = -si[j] * gi[j];
-  gi[j] = ci[j] * gi[j];
-  const double res = fabs(gi[j + 1]);
-  gs[(int64_t)inst * GS_NSCAL + GS_RES] = res;
-  total[inst] += 1;
-  jdone[inst] = j + 1;
-  const double tol = fmax(rtol * gs[(int64_t)inst * GS_NSCAL + GS_BETA0], atol);
-  const bool conv = res <= tol || hn == 0.0;
-  if (conv) live[inst] = 0;
-  if (conv || total[inst] >= maxit || j + 1 == R) iter[inst] = 0;
-  coef[(int64_t)inst * mstride] = hn > 0 ? 1.0 / hn : 0.0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double a = sh_col[0];
+    for (int k = 0; k < j; ++k) {
+      const double b = sh_col[k + 1];
+      sh_col[k] = sh_c[k] * a + sh_s[k] * b;
+      a = -sh_s[k] * a + sh_c[k] * b;
+    }
+    const double r = hypot(a, hn);
+    const double cj = r > 0 ? a / r : 1.0, sj = r > 0 ? hn / r : 0.0;
+    ci[j] = cj;
+    si[j] = sj;
+    sh_col[j] = r;
+    const double gj = gi[j];
+    const double res = fabs(-sj * gj);
+    gi[j + 1] = -sj * gj;
+    gi[j] = cj * gj;
+    gs[(int64_t)inst * GS_NSCAL + GS_RES] = res;
+    const int tot = total[inst] + 1;
+    total[inst] = tot;
+    jdone[inst] = j + 1;
+    const double tol = fmax(rtol * gs[(int64_t)inst * GS_NSCAL + GS_BETA0], atol);
+    const bool conv = res <= tol || hn == 0.0;
+    if (conv) live[inst] = 0;
+    if (conv || tot >= maxit || j + 1 == R) iter[inst] = 0;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k <= j; k += SEG_THREADS) Hi[k * R + j] = sh_col[k];
 }
 
 // end of a cycle: y = H^-1 g for the instances that took part -> coef[inst][0..R)
@@ -340,7 +452,8 @@ struct pdes_batch_group {
   int32_t* d_inst_c0 = nullptr;
   int32_t* d_clist = nullptr;        // active chunk list
   int32_t* d_ilist = nullptr;        // active instance list
-  double* d_partial = nullptr;       // [nchunk][mstride]
+  double* d_partial = nullptr;       // two sets of chunk partial sums, [mstride][nchunk] each
+  int max_chunks = 0;                // of one instance
   double* d_seg = nullptr;           // [ninst][mstride]
   double* d_coef = nullptr;          // [ninst][mstride]
   double* h_seg = nullptr;           // pinned
@@ -431,15 +544,62 @@ int set_worklist(pdes_batch_group* g, Pick pick, std::vector<int>& chunks, std::
   return PDES_OK;
 }
 
-// seg[inst][0..m) = V_i . w  (or weighted squares of V_0 when wt) for the listed instances
-int seg_dots(pdes_batch_group* g, const double* V, int m, int64_t ldv, const double* w, const double* wt,
-             int nchunks, int ninst_list, const int32_t* mask = nullptr) {
+SegLists seg_lists(const pdes_batch_group* g, const int32_t* mask) {
+  return SegLists{g->d_cbeg, g->d_clen, g->d_clist, g->d_chunk_inst, g->d_inst_c0, mask, (int64_t)g->h_cbeg.size(),
+                  g->mstride};
+}
+
+// seg[inst][0] = ||x||^2 (weighted by wt when given) for the listed instances
+int seg_squares(pdes_batch_group* g, const double* x, const double* wt, int nchunks, int ninst_list,
+                const int32_t* mask = nullptr) {
   pdes_ctx* c = g->c;
   if (nchunks == 0) return PDES_OK;
-  hipLaunchKernelGGL(seg_dot_partial, dim3(nchunks), dim3(SEG_THREADS), 0, c->stream, V, m, ldv, w, wt, g->d_cbeg,
-                     g->d_clen, g->d_clist, g->d_partial, g->mstride, g->d_chunk_inst, mask);
-  hipLaunchKernelGGL(seg_dot_reduce, dim3(ninst_list), dim3(64), 0, c->stream, g->d_partial, m, g->mstride,
-                     g->d_inst_c0, g->d_ilist, g->d_seg, mask);
+  const SegLists L = seg_lists(g, mask);
+  hipLaunchKernelGGL(seg_square, dim3(nchunks), dim3(SEG_THREADS), 0, c->stream, L, x, wt, g->d_partial);
+  hipLaunchKernelGGL(seg_reduce, dim3(ninst_list), dim3(SEG_THREADS), 0, c->stream, L, g->d_ilist, 0, g->d_partial,
+                     g->d_seg);
+  PDES_HIP(hipGetLastError());
+  return PDES_OK;
+}
+
+// CGS2 of w = V_{j+1} against V_0 .. V_j for the instances with iter set, the
+// scale and the Givens rotations (launches only)
+int seg_cgs2(pdes_batch_group* g, int j, int nch, int ni, int R, double rtol, double atol, int maxit) {
+  hipStream_t sm = g->c->stream;
+  const int64_t ldv = g->c->numDof;
+  const int m = j + 1;
+  double* w = g->d_V + (int64_t)m * ldv;
+  const SegLists L = seg_lists(g, g->d_iter);
+  double* pa = g->d_partial;
+  double* pb = g->d_partial + L.nct * g->mstride;
+  auto big = [&](const double* p, int rows) {
+    if (g->max_chunks > CGS_SELF_REDUCE)
+      hipLaunchKernelGGL(seg_reduce, dim3(ni, rows), dim3(SEG_THREADS), 0, sm, L, g->d_ilist, CGS_SELF_REDUCE, p,
+                         g->d_seg);
+  };
+  auto dots = [&](auto kernel, const double* pin, double* pout) {
+    hipLaunchKernelGGL(kernel, dim3(nch), dim3(SEG_THREADS), 0, sm, L, g->d_V, m, ldv, w, pin, g->d_seg, g->d_coef,
+                       pout);
+  };
+  auto norm = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nch), dim3(SEG_THREADS), 0, sm, L, g->d_V, m, ldv, w, pb, g->d_seg, g->d_coef,
+                       g->d_H, R, j, pa);
+  };
+  const double* none = nullptr;
+  if (m <= 8) dots(seg_pass<1, false>, none, pa);
+  else if (m <= 16) dots(seg_pass<2, false>, none, pa);
+  else dots(seg_pass<4, false>, none, pa);
+  big(pa, m);
+  if (m <= 8) dots(seg_pass<1, true>, pa, pb);
+  else if (m <= 16) dots(seg_pass<2, true>, pa, pb);
+  else dots(seg_pass<4, true>, pa, pb);
+  big(pb, m);
+  if (m <= 8) norm(seg_norm<1>);
+  else if (m <= 16) norm(seg_norm<2>);
+  else norm(seg_norm<4>);
+  big(pa, 1);
+  hipLaunchKernelGGL(gmres_finish_step, dim3(nch), dim3(SEG_THREADS), 0, sm, L, w, pa, g->d_seg, g->d_iter, g->d_live,
+                     g->d_total, g->d_jdone, g->d_H, g->d_cs, g->d_sn, g->d_g, g->d_gs, R, j, rtol, atol, maxit);
   PDES_HIP(hipGetLastError());
   return PDES_OK;
 }
@@ -491,8 +651,7 @@ int batch_residual_norms(pdes_batch_group* g, std::vector<int>& chunks, std::vec
   pdes_ctx* c = g->c;
   int st = launch_residual(c, c->d_q, nullptr, c->d_res, nullptr, c->phys.check_positivity != 0);
   if (st) return st;
-  // weighted squares: seg_dot_partial with wt uses V_0 = res
-  if ((st = seg_dots(g, c->d_res, 1, 0, nullptr, c->d_Minv, (int)chunks.size(), (int)insts.size()))) return st;
+  if ((st = seg_squares(g, c->d_res, c->d_Minv, (int)chunks.size(), (int)insts.size()))) return st;
   if ((st = fetch_seg(g))) return st;
   std::vector<int32_t> flags(g->inst.size(), 0);
   PDES_HIP(hipMemcpyAsync(flags.data(), c->d_flag, flags.size() * 4, hipMemcpyDeviceToHost, c->stream));
@@ -669,8 +828,7 @@ int group_pass(pdes_batch_group* g, const pdes_newton_opts* o) {
       if ((st = apply_op_masked(g, o->jv_mode, g->d_dq, g->d_w, g->d_live))) return st;
       hipLaunchKernelGGL(sub_masked, dim3(grid_n(n)), dim3(256), 0, sm, g->d_rhs, g->d_w, g->d_V, c->d_el_list,
                          c->d_el_inst, g->dpe, n, g->d_live);
-      if ((st = seg_dots(g, g->d_V, 1, ldv, g->d_V, nullptr, (int)chunks.size(), (int)insts.size(), g->d_live)))
-        return st;
+      if ((st = seg_squares(g, g->d_V, nullptr, (int)chunks.size(), (int)insts.size(), g->d_live))) return st;
       hipLaunchKernelGGL(gmres_restart, dim3((unsigned)ceil_div((int64_t)insts.size(), 64)), dim3(64), 0, sm,
                          (int)insts.size(), g->d_ilist, g->d_iter, g->d_live, g->d_part, g->d_total, g->d_jdone,
                          g->d_seg, g->d_coef, ms, g->d_g, g->d_gs, R, o->krylov_reltol, o->krylov_abstol,
@@ -707,7 +865,7 @@ int group_pass(pdes_batch_group* g, const pdes_newton_opts* o) {
       // q += dq, step norms, new residual (and its norms) of these instances
       hipLaunchKernelGGL(seg_scale, dim3(grid_n(n)), dim3(256), 0, sm, g->d_dq, c->d_q, g->d_coef, ms, 1,
                          c->d_el_list, c->d_el_inst, g->dpe, n, (const int32_t*)nullptr);
-      if ((st = seg_dots(g, g->d_dq, 1, 0, g->d_dq, nullptr, (int)fin_chunks.size(), (int)fin.size()))) return st;
+      if ((st = seg_squares(g, g->d_dq, nullptr, (int)fin_chunks.size(), (int)fin.size()))) return st;
       if ((st = fetch_seg(g))) return st;
       for (int i : fin) g->inst[i].rep.step_norm = std::sqrt(g->h_seg[(int64_t)i * ms]);
       if ((st = batch_residual_norms(g, fin_chunks, fin, false))) return st;
@@ -757,25 +915,7 @@ int group_pass(pdes_batch_group* g, const pdes_newton_opts* o) {
       int sst;
       if ((sst = pc_apply_masked(g, Vj, g->d_z, g->d_iter))) return sst;
       if ((sst = apply_op_masked(g, o->jv_mode, g->d_z, Vn, g->d_iter))) return sst;
-      // CGS2: two passes of h = V^T w, w -= V h; H column = sum of both passes
-      for (int pass = 0; pass < 2; ++pass) {
-        hipLaunchKernelGGL(seg_dot_partial, dim3(nch), dim3(SEG_THREADS), 0, sm, g->d_V, j + 1, ldv, Vn,
-                           (const double*)nullptr, g->d_cbeg, g->d_clen, g->d_clist, g->d_partial, ms,
-                           g->d_chunk_inst, g->d_iter);
-        hipLaunchKernelGGL(seg_reduce_hcol, dim3(ni), dim3(64), 0, sm, g->d_partial, j + 1, ms, g->d_inst_c0,
-                           g->d_ilist, g->d_iter, g->d_coef, g->d_H, R, j, pass);
-        hipLaunchKernelGGL(seg_multiaxpy, dim3(grid_n(n)), dim3(256), 0, sm, g->d_V, j + 1, ldv, g->d_coef, ms, Vn,
-                           c->d_el_list, c->d_el_inst, g->dpe, n, g->d_iter);
-      }
-      if ((sst = seg_dots(g, Vn, 1, ldv, Vn, nullptr, nch, ni, g->d_iter))) return sst;
-      hipLaunchKernelGGL(gmres_finish_step, dim3(gi), dim3(64), 0, sm, ni, g->d_ilist, g->d_iter, g->d_live,
-                         g->d_total, g->d_jdone, g->d_seg, g->d_coef, ms, g->d_H, g->d_cs, g->d_sn, g->d_g, g->d_gs,
-                         R, j, o->krylov_reltol, o->krylov_abstol, o->krylov_itermax);
-      // instances that stopped in gmres_finish_step are masked out of the scale
-      hipLaunchKernelGGL(seg_scale, dim3(grid_n(n)), dim3(256), 0, sm, Vn, Vn, g->d_coef, ms, 0, c->d_el_list,
-                         c->d_el_inst, g->dpe, n, g->d_iter);
-      PDES_HIP(hipGetLastError());
-      return PDES_OK;
+      return seg_cgs2(g, j, nch, ni, R, o->krylov_reltol, o->krylov_abstol, o->krylov_itermax);
     };
     // Blocks of 8 steps between flag read-backs.  A block is captured once
     // into a HIP graph and replayed in later cycles while everything its
@@ -987,6 +1127,7 @@ int pdes_batch_create(int ninst, const pdes_mesh_desc* meshes, const pdes_sbp_de
         g->h_cbeg.push_back(d);
         g->h_clen.push_back((int32_t)std::min<int64_t>(CHUNK, d1 - d));
       }
+      g->max_chunks = std::max(g->max_chunks, (int)g->h_cbeg.size() - g->h_inst_c0.back());
       g->h_inst_c0.push_back((int32_t)g->h_cbeg.size());
     }
     g->restart = 30;
@@ -1015,7 +1156,7 @@ int pdes_batch_create(int ninst, const pdes_mesh_desc* meshes, const pdes_sbp_de
     dm((void**)&g->d_inst_c0, (ni + 1) * 4);
     dm((void**)&g->d_clist, nchunk * 4);
     dm((void**)&g->d_ilist, ni * 4);
-    dm((void**)&g->d_partial, nchunk * g->mstride * 8);
+    dm((void**)&g->d_partial, 2 * nchunk * g->mstride * 8);
     dm((void**)&g->d_seg, (size_t)ni * g->mstride * 8);
     dm((void**)&g->d_coef, (size_t)ni * g->mstride * 8);
     dm((void**)&g->d_z, c->numDof * 8);

@@ -333,7 +333,7 @@ int pdes_estimate_bytes(const pdes_mesh_desc* m, const pdes_sbp_desc* s, int fp6
   // basis vector), Newton step and right-hand side
   b += (gmres_restart + 1) * ndof * 8 + 2 * ndof * 8 + (int64_t)(gmres_restart + 1) * 2 * 512 * 8;
   b += 2 * ndof * 8;
-  if (batched) b += 2 * nel * 4 + 2 * ndof * 8 + (ndof / 4096 + 1) * (8 + 4 + 4 + 64 * 8);
+  if (batched) b += 2 * nel * 4 + 2 * ndof * 8 + (ndof / 1024 + 1) * (8 + 4 + 4 + 2 * 64 * 8);
   *bytes = b;
   return PDES_OK;
 }

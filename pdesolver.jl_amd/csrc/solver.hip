@@ -20,6 +20,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "jacobian.hpp"
+#include "krylov_kernels.hpp"
 
 struct pdes_precond {
   int kind = 0;
@@ -1467,66 +1468,12 @@ int pc_setup(pdes_ctx* c, int kind) {
 // second).  Separate kernels for each dot, update and sum (11 launches and a
 // wait of the host a step) took 73 us a step at n = 9,600 with the operator
 // and the preconditioner, these take 38.
-constexpr int CGS_THREADS = 256;
-constexpr int CGS_SELF_REDUCE = 256, CGS_MAX_BLOCKS = 512;
+constexpr int CGS_MAX_BLOCKS = 512;
 
 static int cgs_blocks(int64_t n) {
   const int64_t full = std::max<int64_t>(1, ceil_div(n, CGS_THREADS));
   if (full <= 8 * CGS_SELF_REDUCE) return (int)std::min<int64_t>(CGS_SELF_REDUCE, full);
   return (int)std::min<int64_t>(CGS_MAX_BLOCKS, full);
-}
-
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
-
-// Sums of NV values over the lanes of a wave, NV a power of two up to 64: each
-// exchange halves the values a lane keeps, so NV - 1 of them serve all.  Lane
-// l ends with the sum of value l / (64 / NV).
-template <int NV, int HALF = NV / 2, int OFF = 32>
-__device__ __forceinline__ double wave_sums(double (&v)[NV]) {
-  if constexpr (OFF == 0) {
-    return v[0];
-  } else if constexpr (HALF == 0) {
-    v[0] += __shfl_xor(v[0], OFF, 64);
-    return wave_sums<NV, 0, OFF / 2>(v);
-  } else {
-    const bool up = threadIdx.x & OFF;
-#pragma unroll
-    for (int k = 0; k < HALF; ++k) {
-      const double give = up ? v[k] : v[k + HALF], keep = up ? v[k + HALF] : v[k];
-      v[k] = keep + __shfl_xor(give, OFF, 64);
-    }
-    return wave_sums<NV, HALF / 2, OFF / 2>(v);
-  }
-}
-
-// h[i] = sum of partial[i][0 .. nb), i < m: each wave sums 8 rows at a time
-__device__ __forceinline__ void sum_partial_rows(const double* __restrict__ partial, int m, int nb, double* h) {
-  const int lane = threadIdx.x & 63;
-  for (int i0 = 8 * (threadIdx.x >> 6); i0 < m; i0 += 8 * (CGS_THREADS / 64)) {
-    double x[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = 0.0;
-    // (all of a wave's loads in flight together)
-    double v[8][CGS_SELF_REDUCE / 64];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int k = 0; k < CGS_SELF_REDUCE / 64; ++k) {
-        const int b = lane + 64 * k;
-        v[i][k] = i0 + i < m && b < nb ? partial[(int64_t)(i0 + i) * nb + b] : 0.0;
-      }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int k = 0; k < CGS_SELF_REDUCE / 64; ++k) x[i] += v[i][k];
-    const double y = wave_sums<8>(x);
-    if (lane % 8 == 0 && i0 + lane / 8 < m) h[i0 + lane / 8] = y;
-  }
-  __syncthreads();
 }
 
 // AXPY: h = sums of pin's rows (nb_in each), w -= sum_i h_i V_i (kept in hsave
@@ -1542,7 +1489,7 @@ cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ 
   __shared__ double sh_w[CGS_THREADS / 64][NV];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if constexpr (AXPY) {
-    sum_partial_rows(pin, m, nb_in, sh_h);
+    sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
     if (blockIdx.x == 0)
       for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
   }
@@ -1590,7 +1537,7 @@ cgs_norm(const double* __restrict__ V, int m, int64_t ldv, const double* __restr
   __shared__ double sh_w[CGS_THREADS / 64];
   const int tid = threadIdx.x;
   if (m > 0) {
-    sum_partial_rows(pin, m, nb_in, sh_h);
+    sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
     if (blockIdx.x == 0)
       for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
   }
@@ -1626,7 +1573,7 @@ __global__ void __launch_bounds__(CGS_THREADS)
 cgs_finish(double* __restrict__ w, int64_t n, const double* __restrict__ pin, int nb_in, int m,
            const double* __restrict__ h1, const double* __restrict__ h2, double* __restrict__ host) {
   __shared__ double sh_h[8];
-  sum_partial_rows(pin, 1, nb_in, sh_h);
+  sum_partial_rows(pin, 1, nb_in, nb_in, sh_h);
   const double hn = sqrt(sh_h[0]);
   if (blockIdx.x == 0) {
     for (int i = threadIdx.x; i < m; i += CGS_THREADS) host[i] = h1[i] + h2[i];
