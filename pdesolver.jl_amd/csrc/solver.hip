@@ -689,8 +689,6 @@ __host__ __device__ constexpr int ilu_dep_chunk(int n, bool diage) {
   return 256 / (n * ilu_dep_lanes(n, diage)) >= 4 ? 4 : 256 / (n * ilu_dep_lanes(n, diage));
 }
 
-__global__ void ilu_sweep_begin(int32_t* __restrict__ sync) { sync[ILU_SYNC_TICKET] = 0; }
-
 __global__ void ilu_pending_fill(double* __restrict__ y, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = __longlong_as_double((long long)ILU_PENDING);
@@ -705,6 +703,15 @@ __device__ __forceinline__ double x_load(const double* p) {
 }
 __device__ __forceinline__ void x_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// the value that lane L of this lane's group of four holds
+template <int L>
+__device__ __forceinline__ double quad_lane(double x) {
+  const int64_t b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, L * 0x55, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), L * 0x55, 0xf, 0xf, false);
+  return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
 }
 
 // in: the right-hand side (forward: b; backward: y); out: the result, which
@@ -723,13 +730,22 @@ ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restric
   constexpr int TPE = N * LPR;
   static_assert(CH * TPE <= 256, "a chunk's rows must fit a workgroup");
   // neighbour blocks of one row on one side: at most one per face with
-  // diagonal-E faces, the face stencil per face otherwise; this lane's share
-  // is loaded before the neighbours' values are awaited
+  // diagonal-E faces, all nodes of the neighbour per face otherwise; this
+  // lane's share is loaded before the neighbours' values are awaited
   constexpr int NFACES = (ND == 4) ? 3 : 4;
   constexpr int MAXB = DIAGE ? NFACES : (NFACES * NS + LPR - 1) / LPR;
+  // the neighbours' unknowns: each is loaded, and waited for, by one lane.
+  // Diagonal-E: lane (node, a) has component a of its node's blocks, and the
+  // four lanes of a node exchange them by lane permutation.  Dense faces: the
+  // rows of an element have the same columns, so lane u has value u of them,
+  // exchanged through LDS.
+  static_assert(DIAGE || NS == NP, "dense faces couple all nodes of both elements");
+  static_assert(DIAGE ? (LPR == 1 && ND == 4) : NFACES * NS * ND <= TPE, "one awaited value per lane");
+  constexpr int NX = DIAGE ? 1 : NFACES * NS * ND;
   __shared__ double tp[CH][N][LPR];
   __shared__ float yp[CH][N][LPR];
   __shared__ float v[CH][N];
+  __shared__ double xs[CH][NX];
   __shared__ int64_t sh_e[CH];
   __shared__ int sh_any;
   const int t = threadIdx.x;
@@ -738,7 +754,8 @@ ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restric
   const int r = tt / LPR, l = tt - r * LPR;
   const int32_t max_polls = sync[ILU_SYNC_POLLS] > 0 ? sync[ILU_SYNC_POLLS] : ILU_WAIT_POLLS;
   if (t == 0) {
-    const int64_t tk = __hip_atomic_fetch_add(&sync[ILU_SYNC_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (the counter wraps to 0 with the last of the launch's workgroups)
+    const int64_t tk = atomicInc(reinterpret_cast<unsigned*>(&sync[ILU_SYNC_TICKET]), (unsigned)nchunks - 1u);
     const int64_t ch = tk < nchunks ? (chunks ? (int64_t)chunks[tk] : tk) : -1;
     int any = 0;
     for (int sl = 0; sl < CH; ++sl) {
@@ -759,89 +776,90 @@ ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restric
   // everything that does not depend on the neighbours' values: this lane's
   // entries of D'_e^-1 (columns l, l + LPR, ...; the first 32 when there are
   // more than 72), the right-hand side, and this lane's neighbour blocks and
-  // their columns
+  // the places of its awaited values
   constexpr int NC = (N + LPR - 1) / LPR;
   constexpr int PF = NC <= 72 ? NC : 32;
+  constexpr int NW = DIAGE ? NFACES : 1;         // values this lane waits for
   float mrow[PF];
   BT pre[MAXB][ND];
-  int32_t pcol[MAXB];
+  int64_t xat[NW];                               // -1: none
   double bval = 0.0;
   const float* Mi = inv + (act ? e : 0) * N * N;
   int64_t q0 = 0, q1 = 0;
-  if (act) {
 #pragma unroll
-    for (int k = 0; k < PF; ++k)
-      if (l + k * LPR < N) mrow[k] = Mi[(l + k * LPR) * N + r];
-    if (l == 0) bval = in[e * N + r];
+  for (int u = 0; u < NW; ++u) xat[u] = -1;
+  if (act) {
     const int i = r / ND, a = r - i * ND;
     const int64_t row = e * NP + i;
     const int64_t p0 = rowptr[row], p1 = rowptr[row + 1];
     q0 = forward ? p0 : p0 + own[row] + NP;
     q1 = forward ? p0 + own[row] : p1;
+    if constexpr (DIAGE) {
+#pragma unroll
+      for (int u = 0; u < NW; ++u)
+        if (q0 + u < q1) xat[u] = (int64_t)colind[q0 + u] * ND + a;
+    } else {
+      // (rows of one element: the same number of neighbour blocks)
+      if (tt < (q1 - q0) * ND) xat[0] = (int64_t)colind[q0 + tt / ND] * ND + tt % ND;
+    }
+#pragma unroll
+    for (int k = 0; k < PF; ++k)
+      if (l + k * LPR < N) mrow[k] = Mi[(l + k * LPR) * N + r];
+    if (l == 0) bval = in[e * N + r];
 #pragma unroll
     for (int u = 0; u < MAXB; ++u) {
       const int64_t p = q0 + l + (int64_t)u * LPR;
-      pcol[u] = p < q1 ? colind[p] : 0;
 #pragma unroll
       for (int c = 0; c < ND; ++c) pre[u][c] = p < q1 ? vals[p * ND * ND + a * ND + c] : BT(0);
     }
   }
-  double acc = 0.0;
-  if (act) {
-    const int a = r % ND;
-    // the neighbours' values: all loads issued at once, then the pending
-    // ones polled again until every one has arrived
-    double xv[MAXB][ND];
+  // all loads issued at once, then the pending ones polled again until every
+  // one has arrived
+  double xw[NW];
 #pragma unroll
-    for (int u = 0; u < MAXB; ++u)
+  for (int u = 0; u < NW; ++u) xw[u] = xat[u] >= 0 ? x_load(out + xat[u]) : 0.0;
+  int polls = 0;
+  while (true) {
+    bool pending = false;
 #pragma unroll
-      for (int c = 0; c < ND; ++c)
-        xv[u][c] = q0 + l + (int64_t)u * LPR < q1 ? x_load(out + (int64_t)pcol[u] * ND + c) : 0.0;
-    int polls = 0;
-    while (true) {
-      bool pending = false;
-#pragma unroll
-      for (int u = 0; u < MAXB; ++u)
-#pragma unroll
-        for (int c = 0; c < ND; ++c) pending |= ilu_is_pending(xv[u][c]);
-      if (!pending) break;
-      if (++polls > max_polls) {
-        __hip_atomic_store(&sync[ILU_SYNC_ERR], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-      for (int u = 0; u < MAXB; ++u)
-#pragma unroll
-        for (int c = 0; c < ND; ++c)
-          if (ilu_is_pending(xv[u][c])) xv[u][c] = x_load(out + (int64_t)pcol[u] * ND + c);
+    for (int u = 0; u < NW; ++u) pending |= ilu_is_pending(xw[u]);
+    if (!pending) break;
+    if (++polls > max_polls) {
+      __hip_atomic_store(&sync[ILU_SYNC_ERR], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      break;
     }
+    __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+      if (ilu_is_pending(xw[u])) xw[u] = x_load(out + xat[u]);
+  }
+  double acc = 0.0;
+  if constexpr (DIAGE) {
 #pragma unroll
     for (int u = 0; u < MAXB; ++u) {
-      if (q0 + l + (int64_t)u * LPR < q1) {
-#pragma unroll
-        for (int c = 0; c < ND; ++c) acc += (double)pre[u][c] * xv[u][c];
+      const double x0 = quad_lane<0>(xw[u]), x1 = quad_lane<1>(xw[u]), x2 = quad_lane<2>(xw[u]),
+                   x3 = quad_lane<3>(xw[u]);
+      if (q0 + u < q1) {
+        acc += (double)pre[u][0] * x0;
+        acc += (double)pre[u][1] * x1;
+        acc += (double)pre[u][2] * x2;
+        acc += (double)pre[u][3] * x3;
       }
     }
-    for (int64_t p = q0 + l + (int64_t)MAXB * LPR; p < q1; p += LPR) {
-      const int32_t col = colind[p];
-      const BT* blk = vals + p * ND * ND + a * ND;
-      const double* xc = out + (int64_t)col * ND;
+  } else {
+    if (xat[0] >= 0) xs[slot][tt] = xw[0];
+    __syncthreads();
+    if (act) {
 #pragma unroll
-      for (int c = 0; c < ND; ++c) {
-        double xcv = x_load(xc + c);
-        while (ilu_is_pending(xcv)) {
-          if (++polls > max_polls) {
-            __hip_atomic_store(&sync[ILU_SYNC_ERR], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-          xcv = x_load(xc + c);
+      for (int u = 0; u < MAXB; ++u) {
+        const int p = l + u * LPR;
+        if (q0 + p < q1) {
+#pragma unroll
+          for (int c = 0; c < ND; ++c) acc += (double)pre[u][c] * xs[slot][p * ND + c];
         }
-        acc += (double)blk[c] * xcv;
       }
+      tp[slot][r][l] = acc;
     }
-    if constexpr (LPR > 1) tp[slot][r][l] = acc;
   }
   if constexpr (LPR == 1) {
     // one lane per row: the row sums need no reduction over lanes, so one
@@ -1174,7 +1192,6 @@ static int ilu_apply(pdes_ctx* c, const double* b, double* x) {
       const double* in = pass == 0 ? b : p->d_y;
       double* out = pass == 0 ? p->d_y : x;
       double* reset = pass == 0 ? x : p->d_y;
-      hipLaunchKernelGGL(ilu_sweep_begin, dim3(1), dim3(1), 0, c->stream, p->d_sync);
       if (j->fp64)
         hipLaunchKernelGGL((ilu_sweep_dep_kernel<NP, ND, NS, DIAGE, double, LPR, CH>), dim3((unsigned)nch),
                            dim3(CH * N * LPR), 0, c->stream, order, chunks, nch, j->d_rowptr, j->d_colind, p->d_own,
