@@ -1107,6 +1107,7 @@ int pdes_batch_create(int ninst, const pdes_mesh_desc* meshes, const pdes_sbp_de
       for (int64_t e = el_start[i]; e < el_start[i + 1]; ++e) g->h_el_inst[e] = i;
       B->where[ids[i]] = {(int)gi, i};
     }
+    c->h_inst_of = g->h_el_inst;
     // per-instance physics and boundary records tagged with the instance
     std::vector<PhysConst> ip(ni);
     for (int i = 0; i < ni; ++i) {

@@ -321,13 +321,12 @@ int pdes_estimate_bytes(const pdes_mesh_desc* m, const pdes_sbp_desc* s, int fp6
   const int64_t nnzb = nel * Np * Np + 2 * nI * cpl;
   b += (nel * Np + 1) * 8 + nnzb * 4 + nnzb * nd * nd * (fp64_blocks ? 8 : 4) + 4;
   // preconditioner: one FP32 inverse per element (block-Jacobi and ILU(0))
-  if (pc_kind != PDES_PC_NONE) b += nel * (Np * nd) * (Np * nd) * 4;
+  if (pc_kind != PDES_PC_NONE) b += nel * pc_block_floats((int)(Np * nd)) * 4;
   if (pc_kind == PDES_PC_ILU0) {
     b += 2 * nel * 4 + 2 * ndof * 8;   // level lists, graph staging
-    // own-block offsets per node row, the padded chunk lists (a level padded
-    // to whole chunks of at most 4 elements: at most 4 entries per element)
-    // and the dependency-driven sweeps' vector
-    b += nel * Np * 4 + 2 * 4 * nel * 4 + ndof * 8;
+    // own-block offsets per node row, the sets of both sweeps (order, places and
+    // at most one start per element) and the dependency-driven sweeps' vector
+    b += nel * Np * 4 + 2 * 3 * nel * 4 + ndof * 8;
   }
   // GMRES basis and vectors (two sets of block partials, 512 workgroups per
   // basis vector), Newton step and right-hand side

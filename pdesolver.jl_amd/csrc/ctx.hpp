@@ -51,6 +51,7 @@ struct pdes_ctx {
   int32_t* d_el_list = nullptr;
   int32_t nlist = -1;           // < 0: no list, every element is processed
   int32_t* d_el_inst = nullptr;
+  std::vector<int32_t> h_inst_of;   // host copy of d_el_inst (packed batches)
   pdes::PhysConst* d_inst_phys = nullptr;
   int ninst = 1;
   // implicit-Euler globalization: per node M (1 + sqrt(jac)), per instance 1/tau
@@ -113,5 +114,7 @@ int launch_wnorm2(pdes_ctx* c, const double* x, const double* w, int64_t n, doub
 int sync_check_flag(pdes_ctx* c);
 int jacobian_free(pdes_ctx* c);
 int precond_free(pdes_ctx* c);
+// floats that the inverse of an element block of n unknowns takes
+int64_t pc_block_floats(int n);
 int bc_state_setup(pdes_ctx* c);
 }  // namespace pdes

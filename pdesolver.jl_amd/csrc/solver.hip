@@ -25,7 +25,7 @@
 struct pdes_precond {
   int kind = 0;
   int n = 0;                 // block size Np*nd
-  float* d_inv = nullptr;    // [numEl][n][n] column-major inverse of each (modified) element block
+  float* d_inv = nullptr;    // inverse of each (modified) element block, laid out by InvLayout
   bool factored = false;
   // ILU(0): elements grouped by dependency level of the forward (lower
   // neighbours first) and backward (upper neighbours first) sweeps
@@ -43,14 +43,15 @@ struct pdes_precond {
   // (PDES_ILU_LEVELS set), 2 always dependency-driven (PDES_ILU_DEP set)
   int force = 0;
   std::vector<int32_t> h_fl, h_bl;   // forward / backward level of each element
-  // the dependency-driven sweeps' level-ordered lists, every level padded
-  // with -1 to whole chunks of `chunk` elements, and their chunk counts
-  int chunk = 1;
-  int32_t* d_fpad = nullptr;
-  int32_t* d_bpad = nullptr;
-  int64_t fpad_n = 0, bpad_n = 0;
-  // the chunks holding elements of selected instances (packed batches), their
-  // counts, the selection flags and the select's work space
+  // the dependency-driven sweeps' sets: the elements set by set, where each
+  // set starts, and each element's place in that list
+  struct Sets {
+    int32_t* d_order = nullptr;
+    int32_t* d_start = nullptr;
+    int32_t* d_place = nullptr;
+    int64_t n = 0;
+  } fset, bset;
+  // the sets of selected instances (packed batches), their counts, the selection flags and the select's work space
   int32_t* d_fsel = nullptr;
   int32_t* d_bsel = nullptr;
   int64_t sel_nf = 0, sel_nb = 0;
@@ -87,8 +88,9 @@ int precond_free(pdes_ctx* c) {
   if (c->pc_obj->d_bel) hipFree(c->pc_obj->d_bel);
   if (c->pc_obj->d_own) hipFree(c->pc_obj->d_own);
   if (c->pc_obj->d_y) hipFree(c->pc_obj->d_y);
-  if (c->pc_obj->d_fpad) hipFree(c->pc_obj->d_fpad);
-  if (c->pc_obj->d_bpad) hipFree(c->pc_obj->d_bpad);
+  for (auto* k : {&c->pc_obj->fset, &c->pc_obj->bset})
+    for (int32_t* p : {k->d_order, k->d_start, k->d_place})
+      if (p) hipFree(p);
   if (c->pc_obj->d_fsel) hipFree(c->pc_obj->d_fsel);
   if (c->pc_obj->d_bsel) hipFree(c->pc_obj->d_bsel);
   if (c->pc_obj->d_inst_sel) hipFree(c->pc_obj->d_inst_sel);
@@ -103,11 +105,56 @@ int precond_free(pdes_ctx* c) {
   return PDES_OK;
 }
 
+// lanes per row of the sweeps.  A wave holds 64 / lanes whole rows, so an
+// element of N rows takes ilu_waves() waves; the lanes are chosen so that a
+// lane's share of a row (N / lanes inverse entries and its neighbour blocks)
+// leaves room for a few elements' shares in registers, and small elements fit
+// one wave.  Dense faces (up to 45 neighbour blocks a row) need more lanes than
+// diagonal-E ones (at most 3).  3D p=2 (50 rows): with four lanes the sweep
+// spilled, 276 us for both triangles of a 10^3 cube, five take 212 us.
+template <int N, bool DIAGE>
+constexpr int ilu_lanes() {
+  if (DIAGE) return N <= 28 ? 2 : N <= 64 ? 1 : 2;
+  return N <= 12 ? 5 : N <= 20 ? 3 : N <= 24 ? 2 : N <= 40 ? 3 : N <= 50 ? 5 : 4;
+}
+template <int N, bool DIAGE>
+constexpr int ilu_waves() {
+  return (N + 64 / ilu_lanes<N, DIAGE>() - 1) / (64 / ilu_lanes<N, DIAGE>());
+}
+
+// whether the blocks of size n belong to a diagonal-E operator
+constexpr bool diage_block(int n) {
+  bool diage = false;
+#define PDES_DIAGE_BLOCK(D_, NP_, NF_, NS_, DE_) \
+  if (NP_ * (D_ + 2) == n) diage = DE_;
+  PDES_FOR_EACH_SHAPE(PDES_DIAGE_BLOCK)
+#undef PDES_DIAGE_BLOCK
+  return diage;
+}
+
+// Where entry (r, c) of an element's inverse is stored.  Dense-face operators:
+// column-major.  Diagonal-E: four of a sweep lane's columns (l, l + LPR, ...)
+// together, [column / (4 LPR)][row][lane][4], so that a lane reads its share of
+// a row 16 bytes at a time and a wave reads them in order: the sweeps keep a
+// few elements' shares in flight, and a wave can have 63 loads outstanding,
+// which 48 to 108 single entries an element would use up.
+template <int N>
+struct InvLayout {
+  static constexpr bool VEC4 = diage_block(N);
+  static constexpr int LPR = ilu_lanes<N, VEC4>();
+  static constexpr int NC = (N + LPR - 1) / LPR;              // columns per lane
+  static constexpr int NCP = VEC4 ? (NC + 3) / 4 * 4 : NC;    // and with the padding
+  static constexpr int SIZE = VEC4 ? NCP * LPR * N : N * N;
+  static __host__ __device__ constexpr int at(int r, int c) {
+    return VEC4 ? (c / (4 * LPR) * (N * LPR) + r * LPR + c % LPR) * 4 + c / LPR % 4 : c * N + r;
+  }
+};
+
 // ---------------------------------------------------------------------------
 // block-Jacobi setup: each element's block is gathered from the BSR matrix
 // (FP32) and inverted in place by Gauss-Jordan elimination with partial (row)
-// pivoting; the inverse is stored column-major so that the apply is a
-// coalesced matrix-vector product.
+// pivoting; the inverse is stored so that the apply is a coalesced
+// matrix-vector product (InvLayout).
 //
 // A chain of N pivots, so what bounds it is the latency of one step, not its
 // flops.  The block lives in registers: G x G threads, thread (tr, tc) holds
@@ -150,7 +197,7 @@ struct GjSmem {
 };
 
 // Inverts the block held in a (thread (tr, tc), see above; zero beyond N) and
-// stores it column-major.  Every thread of the workgroup calls it.
+// stores it.  Every thread of the workgroup calls it.
 template <int N>
 __device__ __forceinline__ void gauss_jordan_inverse(float (&a)[GjShape<N>::R][GjShape<N>::R], GjSmem<N>& sh,
                                                      float* __restrict__ out, int32_t* __restrict__ err) {
@@ -273,7 +320,7 @@ __device__ __forceinline__ void gauss_jordan_inverse(float (&a)[GjShape<N>::R][G
     const int col = sh.row_at[tc + G * j];
 #pragma unroll
     for (int i = 0; i < R; ++i)
-      if (tr + G * i < N) out[col * N + sh.pos[tr + G * i]] = a[i][j];
+      if (tr + G * i < N) out[InvLayout<N>::at(sh.pos[tr + G * i], col)] = a[i][j];
   }
 }
 
@@ -306,12 +353,12 @@ bjacobi_factor_kernel(const int32_t* __restrict__ el_list, const int64_t* __rest
   __syncthreads();
   float a[GjShape<N>::R][GjShape<N>::R];
   load_own_block<NP, ND>(vals, run, a);
-  gauss_jordan_inverse<N>(a, sh, inv + e * N * N, err);
+  gauss_jordan_inverse<N>(a, sh, inv + e * InvLayout<N>::SIZE, err);
 }
 
 // block-Jacobi apply: x_e = inv_e b_e; EPB = 256 / N elements per block, thread
-// (element slot, row r) forms one row of the product from the column-major
-// inverse (consecutive rows read consecutive floats).
+// (element slot, row r) forms one row of the product (consecutive rows read
+// consecutive words of the inverse).
 template <int NP, int ND>
 __global__ void __launch_bounds__(256)
 bjacobi_apply_kernel(const int32_t* __restrict__ el_list, int64_t nel, const float* __restrict__ inv,
@@ -332,10 +379,10 @@ bjacobi_apply_kernel(const int32_t* __restrict__ el_list, int64_t nel, const flo
   if (act) v[slot][r] = (float)b[e * N + r];
   __syncthreads();
   if (!act) return;
-  const float* M = inv + e * N * N;
+  const float* M = inv + e * InvLayout<N>::SIZE;
   float acc = 0.0f;
 #pragma unroll
-  for (int cc = 0; cc < N; ++cc) acc += M[cc * N + r] * v[slot][cc];
+  for (int cc = 0; cc < N; ++cc) acc += M[InvLayout<N>::at(r, cc)] * v[slot][cc];
   x[e * N + r] = (double)acc;
 }
 
@@ -415,7 +462,7 @@ ilu_factor_level_kernel(const int32_t* __restrict__ lev_el, const int64_t* __res
     }
     __syncthreads();
     // B1 = [D'_k^-1](Rk,Rk), B2 = S_ke = A(k rows Rk, e cols Ce), B4 = S_ek = A(e rows Ce, k cols Rk)
-    const float* Ik = inv + k * N * N;
+    const float* Ik = inv + k * InvLayout<N>::SIZE;
     float v1[LM], v2[LM], v4[LM];
 #pragma unroll
     for (int u = 0; u < LM; ++u) {
@@ -424,7 +471,7 @@ ilu_factor_level_kernel(const int32_t* __restrict__ lev_el, const int64_t* __res
       if (t < M * M) {
         const int r1 = t / M, c1 = t - r1 * M;
         const int s1 = r1 / ND, x = r1 - s1 * ND, s2 = c1 / ND, y = c1 - s2 * ND;
-        v1[u] = Ik[(Rk[s1] * ND + x) * N + Rk[s2] * ND + y];   // transposed: lanes along a stored column
+        v1[u] = Ik[InvLayout<N>::at(Rk[s2] * ND + y, Rk[s1] * ND + x)];   // transposed: lanes along a column
         const int64_t q2 = at_ke[s1][DIAGE ? s2 : 0], q4 = at_ek[s1][DIAGE ? s2 : 0];
         if (q2 >= 0) v2[u] = (float)vals[(q2 + (DIAGE ? 0 : Ce[s2])) * (ND * ND) + x * ND + y];
         if (q4 >= 0) v4[u] = (float)vals[(q4 + (DIAGE ? 0 : Rk[s2])) * (ND * ND) + x * ND + y];
@@ -495,7 +542,28 @@ ilu_factor_level_kernel(const int32_t* __restrict__ lev_el, const int64_t* __res
         if (ri[i] >= 0 && cj[j] >= 0) a[i][j] -= upd[i][j];
     __syncthreads();
   }
-  gauss_jordan_inverse<N>(a, sh, inv + e * N * N, err);
+  gauss_jordan_inverse<N>(a, sh, inv + e * InvLayout<N>::SIZE, err);
+}
+
+// The two sums of a sweep's row, in the order that every sweep kernel uses: a
+// neighbour block's product first on its own, then added to the row's (short
+// chains of dependent operations), and the row of the inverse over four partial
+// sums.
+template <int ND, class BT>
+__device__ __forceinline__ double block_dot(const BT* blk, const double* x) {
+  double d = (double)blk[0] * x[0];
+#pragma unroll
+  for (int c = 1; c < ND; ++c) d += (double)blk[c] * x[c];
+  return d;
+}
+// sum over u < NC of m(u) * v(u); u past the row's end is skipped by `in`
+template <int NC, class FM, class FV, class FI>
+__device__ __forceinline__ float row_dot(FM m, FV v, FI in) {
+  float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int u = 0; u < NC; ++u)
+    if (in(u)) y[u & 3] += m(u) * v(u);
+  return (y[0] + y[1]) + (y[2] + y[3]);
 }
 
 // One level of a sweep.  Forward: x_e = D'_e^-1 (b_e - sum_{k<e} A_ek x_k).
@@ -529,9 +597,9 @@ ilu_sweep_level_kernel(const int32_t* __restrict__ lev_el, int64_t count, const 
   }
   float mrow[PF];
   if (act) {
-    const float* Mi = inv + e * N * N;
+    const float* Mi = inv + e * InvLayout<N>::SIZE;
 #pragma unroll
-    for (int cc = 0; cc < PF; ++cc) mrow[cc] = Mi[cc * N + r];
+    for (int cc = 0; cc < PF; ++cc) mrow[cc] = Mi[InvLayout<N>::at(r, cc)];
   }
   if (act) {
     const int i = r / ND, a = r - i * ND;
@@ -545,24 +613,16 @@ ilu_sweep_level_kernel(const int32_t* __restrict__ lev_el, int64_t count, const 
     const int64_t q1 = forward ? p0 + own[row] : p1;
     double t = 0.0;
 #pragma unroll 4
-    for (int64_t p = q0; p < q1; ++p) {
-      const int32_t col = colind[p];
-      const BT* blk = vals + p * ND * ND + a * ND;
-      const double* xc = x + (int64_t)col * ND;
-#pragma unroll
-      for (int c = 0; c < ND; ++c) t += (double)blk[c] * xc[c];
-    }
+    for (int64_t p = q0; p < q1; ++p)
+      t += block_dot<ND>(vals + p * ND * ND + a * ND, x + (int64_t)colind[p] * ND);
     acc = forward ? acc - t : acc + t;
     v[slot][r] = (float)acc;
   }
   __syncthreads();
   if (!act) return;
-  const float* Mi = inv + e * N * N;
-  float y = 0.0f;
-#pragma unroll
-  for (int cc = 0; cc < PF; ++cc) y += mrow[cc] * v[slot][cc];
-#pragma unroll
-  for (int cc = PF; cc < N; ++cc) y += Mi[cc * N + r] * v[slot][cc];
+  const float* Mi = inv + e * InvLayout<N>::SIZE;
+  const float y = row_dot<N>([&](int u) { return u < PF ? mrow[u < PF ? u : 0] : Mi[InvLayout<N>::at(r, u)]; },
+                             [&](int u) { return v[slot][u]; }, [](int) { return true; });
   if (forward) x[e * N + r] = (double)y;
   else x[e * N + r] -= (double)y;
 }
@@ -605,10 +665,10 @@ ilu_sweep_level_ml_kernel(const int32_t* __restrict__ lev_el, int64_t count, con
   float mrow[NC];
   double bval = 0.0;
   if (act) {
-    const float* Mi = inv + e * N * N;
+    const float* Mi = inv + e * InvLayout<N>::SIZE;
 #pragma unroll
     for (int k = 0; k < NC; ++k)
-      if (l + k * LPR < N) mrow[k] = Mi[(l + k * LPR) * N + r];
+      if (l + k * LPR < N) mrow[k] = Mi[InvLayout<N>::at(r, l + k * LPR)];
     if (forward && l == 0) bval = b[e * N + r];
   }
   if (act) {
@@ -619,13 +679,8 @@ ilu_sweep_level_ml_kernel(const int32_t* __restrict__ lev_el, int64_t count, con
     const int64_t q1 = forward ? p0 + own[row] : p1;
     double acc = 0.0;
 #pragma unroll 2
-    for (int64_t p = q0 + l; p < q1; p += LPR) {
-      const int32_t col = colind[p];
-      const BT* blk = vals + p * ND * ND + a * ND;
-      const double* xc = x + (int64_t)col * ND;
-#pragma unroll
-      for (int c = 0; c < ND; ++c) acc += (double)blk[c] * xc[c];
-    }
+    for (int64_t p = q0 + l; p < q1; p += LPR)
+      acc += block_dot<ND>(vals + p * ND * ND + a * ND, x + (int64_t)colind[p] * ND);
     tp[slot][r][l] = acc;
   }
   __syncthreads();
@@ -637,11 +692,8 @@ ilu_sweep_level_ml_kernel(const int32_t* __restrict__ lev_el, int64_t count, con
   }
   __syncthreads();
   if (act) {
-    float y = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NC; ++k)
-      if (l + k * LPR < N) y += mrow[k] * v[slot][l + k * LPR];
-    yp[slot][r][l] = y;
+    yp[slot][r][l] = row_dot<NC>([&](int u) { return mrow[u]; }, [&](int u) { return v[slot][l + u * LPR]; },
+                                 [&](int u) { return l + u * LPR < N; });
   }
   __syncthreads();
   if (act && l == 0) {
@@ -655,39 +707,59 @@ ilu_sweep_level_ml_kernel(const int32_t* __restrict__ lev_el, int64_t count, con
 
 // ---------------------------------------------------------------------------
 // Dependency-driven sweeps: one launch per triangle instead of one per level.
-// The level-ordered element list is cut into chunks of ILU_CHUNK elements of
-// one level each (every level padded to whole chunks with -1), so the
-// elements of a chunk never depend on each other.  Each workgroup takes one
-// chunk, in ticket order: an atomic counter hands out chunk positions, so
-// every element that a chunk's elements depend on (their lower neighbours in
-// the forward sweep, their upper ones in the backward sweep) sits in a chunk
-// with a smaller ticket, which already runs on the device or is done.  A
-// sweep's output holds ILU_PENDING (a signalling-NaN bit pattern, which no
+// The elements are cut into sets that take one or two elements of a level
+// each: an element joins the set of its latest-begun neighbour when it can, so
+// that most of the dependences run inside a set (ilu_sets).  A workgroup takes
+// one set and walks it, so a value needed by the set's next elements is handed
+// on in LDS (a step takes about 0.75 us); only values from other sets go
+// through memory (1.3 us and more from result to use).  An element depends on
+// its own set and on sets begun before it only, and sets are handed out in that
+// order by an atomic counter, so everything a workgroup waits for belongs to a
+// workgroup that already runs or is done.
+//
+// A sweep's output holds ILU_PENDING (a signalling-NaN bit pattern, which no
 // arithmetic produces: a NaN result is quiet) wherever it is not yet
-// computed, so a workgroup waits for its neighbours by loading their values
-// until none is pending, then computes x_e as the level kernels do (same
-// lanes, same order of operations: the same bits) and stores it.  Values are
-// loaded and stored with device-scope atomics (an 8-byte store is seen whole
-// or not at all), so no stale copy in another XCD's L2 is ever read.  The
-// forward sweep writes y = L^-1 b into d_y and sets its elements' rows of x
-// pending (after reading b: x may be b); the backward sweep reads its own y,
-// writes x and sets its rows of y pending again, so d_y is pending between
-// applications (each factorization sets it so).  A wait gives up after a bounded number of
-// polls, sets the error word and carries on, so every launch ends.
+// computed, so waiting for a neighbour is loading its values until none is
+// pending.  Values are loaded and stored with device-scope atomics (an 8-byte
+// store is seen whole or not at all), so no stale copy in another XCD's L2 is
+// ever read.  The forward sweep writes y = L^-1 b into d_y and sets its
+// elements' rows of x pending (after reading b: x may be b); the backward
+// sweep reads its own y, writes x and sets its rows of y pending again, so
+// d_y is pending between applications (each factorization sets it so).  A
+// wait gives up after a bounded number of polls, sets the error word and
+// carries on, so every launch ends.
+//
+// What bounds a step is the latency from the last value's arrival to the next
+// element's first use of the result, so nothing else is done in between.  Two
+// waves of a workgroup only wait: they poll the other sets' values for the
+// elements ahead, in turn, and put them in a ring in LDS.  The other waves form
+// G groups that take the set's elements in turn: a group loads its next
+// element's matrix into registers while the others compute (a wave that loaded
+// for the element after next before it computed put 20 to 60 loads and their
+// addresses into every step, 1.1 us on an n x n annulus).
+// Both triangles, against one workgroup per level's four elements with every
+// value through memory (MI355X): 2D diagonal-E p=2 on an n x n annulus n=24 115
+// -> 75 us, n=123 653 -> 417 us; 2D Omega p=2 n=48 325 -> 171 us; 2D Omega p=1
+// n=200 1097 -> 539 us; 3D Omega p=2 n=10 240 -> 212 us, p=1 n=24 1920 -> 618 us.
+// The lanes, the order of operations and so the bits are the level kernels'.
 // ---------------------------------------------------------------------------
 constexpr int ILU_WAIT_POLLS = 1 << 18;
 constexpr unsigned long long ILU_PENDING = 0x7FF4DEADBEEF0001ull;
 // sync words: ticket counter, error word, poll limit (0: ILU_WAIT_POLLS)
 enum { ILU_SYNC_TICKET = 0, ILU_SYNC_ERR = 1, ILU_SYNC_POLLS = 2, ILU_SYNC_WORDS = 3 };
 
-// elements per chunk for a row block of n unknowns: as many element row
-// blocks as fill a workgroup of at most 256 threads, at most 4
-__host__ __device__ constexpr int ilu_dep_lanes(int n, bool diage) {
-  return diage ? 1 : (256 / n >= 8 ? 8 : 256 / n);
-}
-__host__ __device__ constexpr int ilu_dep_chunk(int n, bool diage) {
-  return 256 / (n * ilu_dep_lanes(n, diage)) >= 4 ? 4 : 256 / (n * ilu_dep_lanes(n, diage));
-}
+// Groups of computing waves (w waves each) in a workgroup: 8 of one wave, 5 of
+// two, 3 of three, 2 of four.  More make it slower (12 one-wave groups: 93
+// instead of 64 us a triangle on a 40 x 40 annulus, 2D diagonal-E p=2): the
+// waiting groups poll the LDS that the computing one needs.
+constexpr int ilu_groups(int w) { return 10 / w > 8 ? 8 : 10 / w > 2 ? 10 / w : 2; }
+// Elements of one level that a set takes: two where there are groups enough to
+// compute them side by side and load ahead (two instead of one: 2D Omega p=2 82
+// -> 72 us, three: 99 us), more where the sets would otherwise outnumber the
+// CUs (about one workgroup fits a CU, and the sets beyond wait for the first
+// ones to end).
+constexpr int ilu_set_width(int w) { return ilu_groups(w) >= 5 ? 2 : 1; }
+constexpr int ILU_WIDTH_MAX = 8, ILU_CUS = 256;
 
 __global__ void ilu_pending_fill(double* __restrict__ y, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -705,220 +777,358 @@ __device__ __forceinline__ void x_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the value that lane L of this lane's group of four holds
-template <int L>
-__device__ __forceinline__ double quad_lane(double x) {
-  const int64_t b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, L * 0x55, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), L * 0x55, 0xf, 0xf, false);
-  return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
+// LDS words that the waves of a workgroup signal each other with, and the
+// wait that orders a wave's LDS accesses around them
+__device__ __forceinline__ int lds_get(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void lds_set(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_add(int* p, int v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <int NP, int ND, int NS, bool DIAGE, class BT>
+struct IluSet {
+  static constexpr int N = NP * ND, NFACES = ND - 1;
+  static constexpr int LPR = ilu_lanes<N, DIAGE>(), W = ilu_waves<N, DIAGE>(), RW = (N + W - 1) / W;
+  // a lane's share of a row: inverse entries and neighbour blocks
+  static constexpr int NC = InvLayout<N>::NC, NCP = InvLayout<N>::NCP;
+  static constexpr int MAXB = ((DIAGE ? NFACES : NFACES * NS) + LPR - 1) / LPR;
+  static constexpr int G = ilu_groups(W), POLLERS = 2;
+  static constexpr int RING = 2 * ((G + 1) / 2) + 2;
+  static constexpr int THREADS = 64 * (G * W + POLLERS);
+  // largest set: what 64 KB of LDS hold, the reach of an LDS instruction's
+  // offset (beyond it every access computes its address: 12% on 3D Omega p=2)
+  static constexpr int PER_ELEMENT = 8 * N + 8 * NP + 4 + 3 * 4 * NFACES + 8;
+  static constexpr int FIXED = 8 * RING * NFACES * N + 4 * G * (W > 1 ? 2 : 1) * N + 64;
+  static constexpr int KMAX = (65536 - FIXED) / PER_ELEMENT < 384 ? (65536 - FIXED) / PER_ELEMENT : 384;
+  static constexpr int LOCAL = KMAX * N;
+  double xl[LOCAL + RING * NFACES * N];   // the set's values, then a ring of other sets' values
+  // right-hand sides; two a group, as its waves can be one element apart
+  alignas(16) float v[G][W > 1 ? 2 : 1][N];
+  int64_t q[KMAX][NP];                    // per node row: first neighbour block << 8 | blocks
+  int32_t el[KMAX];
+  int32_t nb[KMAX][NFACES];               // neighbour elements of the sweep's side, ascending, -1 beyond
+  int32_t at[KMAX][NFACES];               // where their values are in xl
+  int32_t dep[KMAX][NFACES];              // and their places in the set, KMAX for others
+  int done[KMAX + 1], rows[KMAX];         // waves that have finished the element / written its rows of v
+  int ready[POLLERS];                     // elements whose outside values have come, per waiting wave
+  int64_t set;
+};
 
 // in: the right-hand side (forward: b; backward: y); out: the result, which
 // the neighbours' values are read from (forward: y; backward: x); reset: the
 // vector whose rows of this element become pending after use (forward: x;
 // backward: y).  in may alias reset.
-template <int NP, int ND, int NS, bool DIAGE, class BT, int LPR, int CH>
-__global__ void __launch_bounds__(256)
-ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restrict__ chunks, int64_t nchunks,
-                     const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
-                     const int32_t* __restrict__ own, const BT* __restrict__ vals, const float* __restrict__ inv,
+template <int NP, int ND, int NS, bool DIAGE, class BT>
+__global__ void __launch_bounds__((IluSet<NP, ND, NS, DIAGE, BT>::THREADS))
+ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restrict__ start,
+                     const int32_t* __restrict__ place, const int32_t* __restrict__ sets, int64_t nsets,
+                     const pdes::ElFace* __restrict__ elface, const int64_t* __restrict__ rowptr,
+                     const int32_t* colind, const int32_t* __restrict__ own, const BT* vals, const float* inv,
                      const double* in, double* out, double* reset, int forward,
                      const int32_t* __restrict__ el_inst, const int32_t* __restrict__ mask,
                      const int32_t* __restrict__ inst_active, int32_t* __restrict__ sync) {
-  constexpr int N = NP * ND;
-  constexpr int TPE = N * LPR;
-  static_assert(CH * TPE <= 256, "a chunk's rows must fit a workgroup");
-  // neighbour blocks of one row on one side: at most one per face with
-  // diagonal-E faces, all nodes of the neighbour per face otherwise; this
-  // lane's share is loaded before the neighbours' values are awaited
-  constexpr int NFACES = (ND == 4) ? 3 : 4;
-  constexpr int MAXB = DIAGE ? NFACES : (NFACES * NS + LPR - 1) / LPR;
-  // the neighbours' unknowns: each is loaded, and waited for, by one lane.
-  // Diagonal-E: lane (node, a) has component a of its node's blocks, and the
-  // four lanes of a node exchange them by lane permutation.  Dense faces: the
-  // rows of an element have the same columns, so lane u has value u of them,
-  // exchanged through LDS.
+  using C = IluSet<NP, ND, NS, DIAGE, BT>;
+  constexpr int N = C::N, NFACES = C::NFACES, LPR = C::LPR, W = C::W, RW = C::RW, NC = C::NC, MAXB = C::MAXB;
   static_assert(DIAGE || NS == NP, "dense faces couple all nodes of both elements");
-  static_assert(DIAGE ? (LPR == 1 && ND == 4) : NFACES * NS * ND <= TPE, "one awaited value per lane");
-  constexpr int NX = DIAGE ? 1 : NFACES * NS * ND;
-  __shared__ double tp[CH][N][LPR];
-  __shared__ float yp[CH][N][LPR];
-  __shared__ float v[CH][N];
-  __shared__ double xs[CH][NX];
-  __shared__ int64_t sh_e[CH];
-  __shared__ int sh_any;
-  const int t = threadIdx.x;
-  const int slot = t / TPE;
-  const int tt = t - slot * TPE;
-  const int r = tt / LPR, l = tt - r * LPR;
-  const int32_t max_polls = sync[ILU_SYNC_POLLS] > 0 ? sync[ILU_SYNC_POLLS] : ILU_WAIT_POLLS;
-  if (t == 0) {
+  __shared__ C sm;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (tid == 0) {
     // (the counter wraps to 0 with the last of the launch's workgroups)
-    const int64_t tk = atomicInc(reinterpret_cast<unsigned*>(&sync[ILU_SYNC_TICKET]), (unsigned)nchunks - 1u);
-    const int64_t ch = tk < nchunks ? (chunks ? (int64_t)chunks[tk] : tk) : -1;
-    int any = 0;
-    for (int sl = 0; sl < CH; ++sl) {
-      int64_t e = ch >= 0 ? (int64_t)order[ch * CH + sl] : -1;
-      if (e >= 0) {
-        const int inst = el_inst ? el_inst[e] : 0;
-        if ((mask && !mask[inst]) || (inst_active && !inst_active[inst])) e = -1;   // no element waits on it
-      }
-      sh_e[sl] = e;
-      any |= e >= 0;
+    const int64_t tk = atomicInc(reinterpret_cast<unsigned*>(&sync[ILU_SYNC_TICKET]), (unsigned)nsets - 1u);
+    int64_t set = tk < nsets ? (sets ? (int64_t)sets[tk] : tk) : -1;
+    if (set >= 0) {
+      const int inst = el_inst ? el_inst[order[start[set]]] : 0;   // a set stays within an instance
+      if ((mask && !mask[inst]) || (inst_active && !inst_active[inst])) set = -1;   // no element waits on it
     }
-    sh_any = any;
+    sm.set = set;
+    for (int p = 0; p < C::POLLERS; ++p) sm.ready[p] = 0;
+  }
+  for (int k = tid; k < C::KMAX; k += C::THREADS) sm.done[k] = sm.rows[k] = 0;
+  if (tid == 0) sm.done[C::KMAX] = W;
+  __syncthreads();
+  if (sm.set < 0) return;   // uniform over the workgroup
+  const int base = start[sm.set], K = start[sm.set + 1] - base;
+  // what the walk needs to know about the set's elements
+  for (int k = tid; k < K; k += C::THREADS) {
+    const int e = order[base + k];
+    sm.el[k] = e;
+    int id[NFACES];
+#pragma unroll
+    for (int f = 0; f < NFACES; ++f) {
+      const int n = elface[(int64_t)e * NFACES + f].x;
+      id[f] = n >= 0 && (forward ? n < e : n > e) ? n : 0x7fffffff;
+    }
+#pragma unroll
+    for (int i = 0; i < NFACES; ++i)
+#pragma unroll
+      for (int f = 0; f + 1 < NFACES - i; ++f)
+        if (id[f + 1] < id[f]) { const int t = id[f]; id[f] = id[f + 1]; id[f + 1] = t; }
+#pragma unroll
+    for (int f = 0; f < NFACES; ++f) {
+      const bool has = id[f] != 0x7fffffff;
+      const int pl = has ? place[id[f]] - base : -1;
+      const bool local = pl >= 0 && pl < K;
+      sm.nb[k][f] = has ? id[f] : -1;
+      sm.at[k][f] = local ? pl * N : C::LOCAL + ((k % C::RING) * NFACES + f) * N;
+      sm.dep[k][f] = local ? pl : C::KMAX;
+    }
+  }
+  for (int t = tid; t < K * NP; t += C::THREADS) {
+    const int64_t row = (int64_t)order[base + t / NP] * NP + t % NP;
+    const int64_t p0 = rowptr[row], o = own[row];
+    const int64_t b = forward ? p0 : p0 + o + NP, n = forward ? o : rowptr[row + 1] - b;
+    sm.q[t / NP][t % NP] = b << 8 | n;
   }
   __syncthreads();
-  if (!sh_any) return;   // uniform over the block
-  const int64_t e = slot < CH ? sh_e[slot] : -1;
-  const bool act = e >= 0;
-  // everything that does not depend on the neighbours' values: this lane's
-  // entries of D'_e^-1 (columns l, l + LPR, ...; the first 32 when there are
-  // more than 72), the right-hand side, and this lane's neighbour blocks and
-  // the places of its awaited values
-  constexpr int NC = (N + LPR - 1) / LPR;
-  constexpr int PF = NC <= 72 ? NC : 32;
-  constexpr int NW = DIAGE ? NFACES : 1;         // values this lane waits for
-  float mrow[PF];
-  BT pre[MAXB][ND];
-  int64_t xat[NW];                               // -1: none
-  double bval = 0.0;
-  const float* Mi = inv + (act ? e : 0) * N * N;
-  int64_t q0 = 0, q1 = 0;
+
+  if (wave >= C::G * W) {
+    // a waiting wave
+    const int wp = wave - C::G * W;
+    __builtin_amdgcn_s_setprio(2);
+    const int max_polls = sync[ILU_SYNC_POLLS] > 0 ? sync[ILU_SYNC_POLLS] : ILU_WAIT_POLLS;
+    constexpr int NL = (N + 63) / 64;
+    for (int k = wp; k < K; k += C::POLLERS) {
+      if (k >= C::RING)
+        while (lds_get(&sm.done[k - C::RING]) < W) __builtin_amdgcn_s_sleep(1);   // its ring slot is free
+      const double* from[NFACES];
+      double x[NFACES][NL];
 #pragma unroll
-  for (int u = 0; u < NW; ++u) xat[u] = -1;
-  if (act) {
-    const int i = r / ND, a = r - i * ND;
-    const int64_t row = e * NP + i;
-    const int64_t p0 = rowptr[row], p1 = rowptr[row + 1];
-    q0 = forward ? p0 : p0 + own[row] + NP;
-    q1 = forward ? p0 + own[row] : p1;
-    if constexpr (DIAGE) {
+      for (int f = 0; f < NFACES; ++f) {
+        const int n = sm.nb[k][f];
+        from[f] = n >= 0 && sm.at[k][f] >= C::LOCAL ? out + (int64_t)n * N : nullptr;
 #pragma unroll
-      for (int u = 0; u < NW; ++u)
-        if (q0 + u < q1) xat[u] = (int64_t)colind[q0 + u] * ND + a;
-    } else {
-      // (rows of one element: the same number of neighbour blocks)
-      if (tt < (q1 - q0) * ND) xat[0] = (int64_t)colind[q0 + tt / ND] * ND + tt % ND;
-    }
-#pragma unroll
-    for (int k = 0; k < PF; ++k)
-      if (l + k * LPR < N) mrow[k] = Mi[(l + k * LPR) * N + r];
-    if (l == 0) bval = in[e * N + r];
-#pragma unroll
-    for (int u = 0; u < MAXB; ++u) {
-      const int64_t p = q0 + l + (int64_t)u * LPR;
-#pragma unroll
-      for (int c = 0; c < ND; ++c) pre[u][c] = p < q1 ? vals[p * ND * ND + a * ND + c] : BT(0);
-    }
-  }
-  // all loads issued at once, then the pending ones polled again until every
-  // one has arrived
-  double xw[NW];
-#pragma unroll
-  for (int u = 0; u < NW; ++u) xw[u] = xat[u] >= 0 ? x_load(out + xat[u]) : 0.0;
-  int polls = 0;
-  while (true) {
-    bool pending = false;
-#pragma unroll
-    for (int u = 0; u < NW; ++u) pending |= ilu_is_pending(xw[u]);
-    if (!pending) break;
-    if (++polls > max_polls) {
-      __hip_atomic_store(&sync[ILU_SYNC_ERR], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      break;
-    }
-    __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-    for (int u = 0; u < NW; ++u)
-      if (ilu_is_pending(xw[u])) xw[u] = x_load(out + xat[u]);
-  }
-  double acc = 0.0;
-  if constexpr (DIAGE) {
-#pragma unroll
-    for (int u = 0; u < MAXB; ++u) {
-      const double x0 = quad_lane<0>(xw[u]), x1 = quad_lane<1>(xw[u]), x2 = quad_lane<2>(xw[u]),
-                   x3 = quad_lane<3>(xw[u]);
-      if (q0 + u < q1) {
-        acc += (double)pre[u][0] * x0;
-        acc += (double)pre[u][1] * x1;
-        acc += (double)pre[u][2] * x2;
-        acc += (double)pre[u][3] * x3;
+        for (int u = 0; u < NL; ++u)
+          x[f][u] = from[f] && lane + 64 * u < N ? x_load(from[f] + lane + 64 * u) : 0.0;
       }
-    }
-  } else {
-    if (xat[0] >= 0) xs[slot][tt] = xw[0];
-    __syncthreads();
-    if (act) {
+      int polls = 0;
+      while (true) {
+        bool pending = false;
 #pragma unroll
-      for (int u = 0; u < MAXB; ++u) {
-        const int p = l + u * LPR;
-        if (q0 + p < q1) {
+        for (int f = 0; f < NFACES; ++f)
 #pragma unroll
-          for (int c = 0; c < ND; ++c) acc += (double)pre[u][c] * xs[slot][p * ND + c];
+          for (int u = 0; u < NL; ++u) pending |= ilu_is_pending(x[f][u]);
+        if (!__any(pending)) break;
+        if (++polls > max_polls) {
+          __hip_atomic_store(&sync[ILU_SYNC_ERR], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
         }
+#pragma unroll
+        for (int f = 0; f < NFACES; ++f)
+#pragma unroll
+          for (int u = 0; u < NL; ++u)
+            if (ilu_is_pending(x[f][u])) x[f][u] = x_load(from[f] + lane + 64 * u);
       }
-      tp[slot][r][l] = acc;
+#pragma unroll
+      for (int f = 0; f < NFACES; ++f)
+        if (from[f]) {
+#pragma unroll
+          for (int u = 0; u < NL; ++u)
+            if (lane + 64 * u < N) sm.xl[sm.at[k][f] + lane + 64 * u] = x[f][u];
+        }
+      lds_fence();
+      if (lane == 0) lds_set(&sm.ready[wp], k + 1);
     }
+    return;
   }
-  if constexpr (LPR == 1) {
-    // one lane per row: the row sums need no reduction over lanes, so one
-    // barrier (for the rows of v) instead of three; the sums keep the
-    // lane-reduced form 0 + acc, 0 + y, so the bits are the same
-    if (act) {
-      const double sum = 0.0 + acc;
-      v[slot][r] = (float)(forward ? bval - sum : sum);
+
+  // the computing waves: lane l of row r, elements g, g + G, ... of the set
+  const int g = wave / W, gw = wave - g * W;
+  const int l = lane % LPR, first = lane - l;
+  const bool has_row = lane / LPR < RW && gw * RW + lane / LPR < N;
+  const int r = has_row ? gw * RW + lane / LPR : N - 1;
+  const int i = r / ND, a = r - i * ND;
+  for (int k = g; k < K; k += C::G) {
+    // this lane's share: entries l, l + LPR, ... of its row of D'_e^-1, row a
+    // of the neighbour blocks l, l + LPR, ... (a valid block where there is
+    // none), the places of their values, the right-hand side
+    const int64_t e = sm.el[k];
+    const int64_t q = sm.q[k][i];
+    const int64_t p0 = q >> 8;
+    const int n = (int)(q & 255);
+    float m[C::NCP];
+    // (in FP64 already where the share is small)
+    using KT = std::conditional_t<(MAXB <= 3), double, BT>;
+    KT blk[MAXB][ND];
+    int off[MAXB];
+    const float* Mi = inv + e * InvLayout<N>::SIZE;
+    if constexpr (InvLayout<N>::VEC4) {
+#pragma unroll
+      for (int u = 0; u < C::NCP; u += 4) {
+        const float4 m4 = *reinterpret_cast<const float4*>(Mi + (u / 4 * (N * LPR) + r * LPR + l) * 4);
+        m[u] = m4.x;
+        m[u + 1] = m4.y;
+        m[u + 2] = m4.z;
+        m[u + 3] = m4.w;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NC; ++u) m[u] = Mi[InvLayout<N>::at(r, l + u * LPR < N ? l + u * LPR : N - 1)];
     }
-    __syncthreads();
-    if (act) {
-      float y = 0.0f;
 #pragma unroll
-      for (int k = 0; k < PF; ++k)
-        if (k < N) y += mrow[k] * v[slot][k];
+    for (int u = 0; u < MAXB; ++u) {
+      const int p = l + u * LPR;
+      // (a row without blocks on this side: its first or last own block)
+      const int64_t pp = p < n ? p0 + p : forward ? p0 : p0 - 1;
 #pragma unroll
-      for (int k = PF; k < NC; ++k)
-        if (k < N) y += Mi[k * N + r] * v[slot][k];
-      const float ys = 0.0f + y;
-      x_store(out + e * N + r, forward ? (double)ys : bval - (double)ys);
-      // this thread read the row of `in` (which `reset` may alias) above
-      x_store(reset + e * N + r, __longlong_as_double((long long)ILU_PENDING));
+      for (int c = 0; c < ND; ++c) blk[u][c] = (KT)vals[pp * (ND * ND) + a * ND + c];
+      off[u] = 0;
+      if constexpr (DIAGE) {
+        const int col = colind[pp];
+#pragma unroll
+        for (int f = 0; f < NFACES; ++f) {
+          const int d = col - sm.nb[k][f] * NP;
+          if (sm.nb[k][f] >= 0 && d >= 0 && d < NP) off[u] = sm.at[k][f] + d * ND;
+        }
+      } else {
+        if (p < NFACES * NP) off[u] = sm.at[k][p / NP] + (p % NP) * ND;
+      }
     }
-  } else {
-    __syncthreads();
-    if (act && l == 0) {
-      double sum = 0.0;
+    const double bval = in[e * N + r];
+    if constexpr (MAXB <= 3) {
 #pragma unroll
-      for (int k = 0; k < LPR; ++k) sum += tp[slot][r][k];
-      v[slot][r] = (float)(forward ? bval - sum : sum);
+      for (int u = 0; u < MAXB; ++u)
+#pragma unroll
+        for (int c = 0; c < ND; ++c) asm volatile("" : "+v"(blk[u][c]));   // converted before the wait
     }
-    __syncthreads();
-    if (act) {
-      float y = 0.0f;
+    // its turn: the set's elements that it depends on are done and the values
+    // from outside are here
+    int dep[NFACES];
 #pragma unroll
-      for (int k = 0; k < PF; ++k)
-        if (l + k * LPR < N) y += mrow[k] * v[slot][l + k * LPR];
+    for (int f = 0; f < NFACES; ++f) dep[f] = sm.dep[k][f];
+    while (true) {
+      int have = W;
 #pragma unroll
-      for (int k = PF; k < NC; ++k)
-        if (l + k * LPR < N) y += Mi[(l + k * LPR) * N + r] * v[slot][l + k * LPR];
-      yp[slot][r][l] = y;
+      for (int f = 0; f < NFACES; ++f) {
+        const int d = lds_get(&sm.done[dep[f]]);
+        have = d < have ? d : have;
+      }
+      if (lds_get(&sm.ready[k % C::POLLERS]) > k && have == W) break;
     }
-    __syncthreads();
-    if (act && l == 0) {
-      float y = 0.0f;
+    __builtin_amdgcn_s_setprio(3);
+    lds_fence();
+    // (a few blocks' values are read together: one LDS latency for all; fewer
+    // where the share leaves no registers for four)
+    constexpr int BG = MAXB * ND * (int)(sizeof(BT) / 4) > 40 ? 2 : MAXB < 4 ? MAXB : 4;
+    double acc = 0.0;
 #pragma unroll
-      for (int k = 0; k < LPR; ++k) y += yp[slot][r][k];
-      x_store(out + e * N + r, forward ? (double)y : bval - (double)y);
-      // this thread read the row of `in` (which `reset` may alias) above
-      x_store(reset + e * N + r, __longlong_as_double((long long)ILU_PENDING));
+    for (int u0 = 0; u0 < MAXB; u0 += BG) {
+      double x[BG][ND];
+#pragma unroll
+      for (int u = 0; u < BG; ++u)
+#pragma unroll
+        for (int c = 0; c < ND; ++c)
+          if (u0 + u < MAXB) x[u][c] = sm.xl[off[u0 + u < MAXB ? u0 + u : 0] + c];
+#pragma unroll
+      for (int u = 0; u < BG; ++u)
+        if (u0 + u < MAXB) {
+          const double d = block_dot<ND>(blk[u0 + u < MAXB ? u0 + u : 0], x[u]);
+          if (l + (u0 + u) * LPR < n) acc += d;
+        }
     }
+    double sum = 0.0;
+    if constexpr (LPR == 1) {
+      sum += acc;
+    } else {
+#pragma unroll
+      for (int u = 0; u < LPR; ++u) sum += __shfl(acc, first + u, 64);
+    }
+    float* const v = sm.v[g][W > 1 ? k / C::G % 2 : 0];
+    if (has_row && l == 0) v[r] = (float)(forward ? bval - sum : sum);
+    if constexpr (W == 1) {
+      asm volatile("" ::: "memory");   // (a wave's LDS accesses keep their order)
+    } else {
+      lds_fence();
+      if (lane == 0) lds_add(&sm.rows[k], 1);
+      while (lds_get(&sm.rows[k]) < W) {}
+      lds_fence();
+    }
+    const float y = row_dot<NC>([&](int u) { return m[u]; }, [&](int u) { return v[l + u * LPR]; },
+                                [&](int u) { return l + u * LPR < N; });
+    float ys = 0.0f;
+    if constexpr (LPR == 1) {
+      ys += y;
+    } else {
+#pragma unroll
+      for (int u = 0; u < LPR; ++u) ys += __shfl(y, first + u, 64);
+    }
+    const double xe = forward ? (double)ys : bval - (double)ys;
+    if (has_row && l == 0) {
+      sm.xl[k * N + r] = xe;
+      x_store(out + e * N + r, xe);
+    }
+    lds_fence();
+    if (lane == 0) lds_add(&sm.done[k], 1);
+    __builtin_amdgcn_s_setprio(0);
+    // (this row of `in`, which `reset` may alias, is in bval)
+    if (has_row && l == 0) x_store(reset + e * N + r, __longlong_as_double((long long)ILU_PENDING));
   }
 }
 
-// lanes per row of the sweeps: 1 for diagonal-E operators (a row meets at
-// most one neighbour node per face), up to 8 for dense face stencils
-template <int N, bool DIAGE>
-constexpr int ilu_lanes() {
-  return DIAGE ? 1 : (256 / N >= 8 ? 8 : 256 / N);
+// least width and largest size of a set
+static void ilu_set_shape(const pdes_ctx* c, int* width, int* kmax) {
+  *width = *kmax = 1;
+#define PDES_ILU_SET(D_, NP_, NF_, NS_, DE_)                              \
+  if (c->dim == D_ && c->Np == NP_ && (c->diag_e != 0) == DE_) {          \
+    using C = IluSet<NP_, D_ + 2, NS_, DE_, float>;                     \
+    static_assert(sizeof(C) <= 65536, "a set's LDS");                     \
+    *width = ilu_set_width(C::W);                                         \
+    *kmax = C::KMAX;                                                      \
+  }
+  PDES_FOR_EACH_SHAPE(PDES_ILU_SET)
+#undef PDES_ILU_SET
+}
+
+// The sets of one triangle (host): elements in level order (lv, els), each
+// joining the set of its latest-begun neighbour of the sweep's side, else the
+// set begun last, if it has room (ilu_set_shape, ILU_CUS), else beginning one.  Dependences then go to the own
+// set or to sets begun before.
+static void ilu_sets(const pdes_ctx* c, bool forward, const std::vector<int32_t>& lv, const std::vector<int32_t>& els,
+                     std::vector<int32_t>& order, std::vector<int32_t>& start, std::vector<int32_t>& place) {
+  const int nel = c->numEl, nf = c->nfaces, levels = els.empty() ? 1 : lv[els.back()] + 1;
+  int width, kmax;
+  ilu_set_shape(c, &width, &kmax);
+  width = std::max(width, (int)std::min<int64_t>(ILU_WIDTH_MAX, ceil_div(nel, (int64_t)levels * ILU_CUS)));
+  std::vector<int32_t> set(nel, -1), len, last, at_last;   // per set: elements, latest level, elements of it
+  // (packed batches: a set stays within an instance, whose elements share no
+  // face with the others': join the set begun last only from the same side)
+  auto inst_of = [&](int e) { return c->h_inst_of.empty() ? 0 : c->h_inst_of[e]; };
+  std::vector<int32_t> newest;                             // per instance: the set begun last
+  for (int e : els) {
+    const int in = inst_of(e);
+    if ((int)newest.size() <= in) newest.resize(in + 1, -1);
+    int32_t best = -1;
+    for (int f = 0; f < nf; ++f) {
+      const int k = c->h_elface[(size_t)e * nf + f].x;
+      if (k >= 0 && (forward ? k < e : k > e)) best = std::max(best, set[k]);
+    }
+    auto room = [&](int32_t t) { return t >= 0 && len[t] < kmax && (last[t] < lv[e] || at_last[t] < width); };
+    int32_t to = room(best) ? best : newest[in] >= best && room(newest[in]) ? newest[in] : -1;
+    if (to < 0) {
+      to = (int32_t)len.size();
+      len.push_back(0);
+      last.push_back(-1);
+      at_last.push_back(0);
+      newest[in] = to;
+    }
+    set[e] = to;
+    ++len[to];
+    at_last[to] = last[to] == lv[e] ? at_last[to] + 1 : 1;
+    last[to] = lv[e];
+  }
+  start.assign(len.size() + 1, 0);
+  for (size_t k = 0; k < len.size(); ++k) start[k + 1] = start[k] + len[k];
+  std::vector<int32_t> pos(start.begin(), start.end() - 1);
+  order.resize(nel);
+  place.resize(nel);
+  for (int e : els) {
+    place[e] = pos[set[e]]++;
+    order[place[e]] = e;
+  }
 }
 
 // dependency levels of the natural-order sweeps (host, once per context)
@@ -977,32 +1187,30 @@ static int ilu_structure(pdes_ctx* c, pdes_precond* p) {
   }
   PDES_HIP(hipMemcpyAsync(p->d_fel, fel.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
   PDES_HIP(hipMemcpyAsync(p->d_bel, bel.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  {
-    // chunked, padded copies for the dependency-driven sweeps
-    const int C = ilu_dep_chunk(c->Np * c->nd, c->diag_e != 0);
-    auto pad = [&](const std::vector<int64_t>& ptr, const std::vector<int32_t>& el, std::vector<int32_t>& out) {
-      out.clear();
-      for (size_t lv = 0; lv + 1 < ptr.size(); ++lv) {
-        for (int64_t q = ptr[lv]; q < ptr[lv + 1]; ++q) out.push_back(el[q]);
-        while (out.size() % C) out.push_back(-1);
+  bool twice = false;   // an element that meets a neighbour at two faces (its rows then hold a column twice)
+  for (int e = 0; e < nel && !twice; ++e)
+    for (int f = 0; f < nf; ++f)
+      for (int g = f + 1; g < nf; ++g) {
+        const int k = c->h_elface[(size_t)e * nf + f].x;
+        twice = twice || (k >= 0 && k == c->h_elface[(size_t)e * nf + g].x);
       }
-    };
-    std::vector<int32_t> fpad, bpad;
-    pad(p->fptr, fel, fpad);
-    pad(p->bptr, bel, bpad);
-    p->chunk = C;
-    p->fpad_n = (int64_t)fpad.size() / C;
-    p->bpad_n = (int64_t)bpad.size() / C;
-    if (hipMalloc((void**)&p->d_fpad, std::max<size_t>(1, fpad.size()) * sizeof(int32_t)) != hipSuccess ||
-        hipMalloc((void**)&p->d_bpad, std::max<size_t>(1, bpad.size()) * sizeof(int32_t)) != hipSuccess) {
-      set_error("device allocation of the ILU chunk lists failed");
+  for (int pass = 0; pass < 2; ++pass) {
+    std::vector<int32_t> order, start, place;
+    ilu_sets(c, pass == 0, pass == 0 ? fl : bl, pass == 0 ? fel : bel, order, start, place);
+    pdes_precond::Sets& k = pass == 0 ? p->fset : p->bset;
+    k.n = (int64_t)start.size() - 1;
+    if (hipMalloc((void**)&k.d_order, std::max(1, nel) * sizeof(int32_t)) != hipSuccess ||
+        hipMalloc((void**)&k.d_start, start.size() * sizeof(int32_t)) != hipSuccess ||
+        hipMalloc((void**)&k.d_place, std::max(1, nel) * sizeof(int32_t)) != hipSuccess) {
+      set_error("device allocation of the ILU sets failed");
       return PDES_ERR_NOMEM;
     }
-    PDES_HIP(hipMemcpyAsync(p->d_fpad, fpad.data(), fpad.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-    PDES_HIP(hipMemcpyAsync(p->d_bpad, bpad.data(), bpad.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+    PDES_HIP(hipMemcpyAsync(k.d_order, order.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+    PDES_HIP(hipMemcpyAsync(k.d_start, start.data(), start.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+    PDES_HIP(hipMemcpyAsync(k.d_place, place.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     PDES_HIP(hipStreamSynchronize(c->stream));   // the host vectors go out of scope
   }
-  p->force = std::getenv("PDES_ILU_LEVELS") ? 1 : std::getenv("PDES_ILU_DEP") ? 2 : 0;
+  p->force = twice || std::getenv("PDES_ILU_LEVELS") ? 1 : std::getenv("PDES_ILU_DEP") ? 2 : 0;
   p->h_fl = fl;
   p->h_bl = bl;
   p->blk_per_el = (double)(J->nnzb - (int64_t)nel * c->Np * c->Np) / 2.0 / std::max(1, nel);
@@ -1027,21 +1235,20 @@ static int ilu_structure(pdes_ctx* c, pdes_precond* p) {
   return PDES_OK;
 }
 
-// Which sweeps an application runs (both give the same bits).  A level
-// launch costs at least ILU_LEVEL_FLOOR_US and streams its elements' bytes at
-// ILU_LEVEL_BW; the dependency-driven sweep takes at least ILU_DEP_STEP_US per
-// level of its critical path, ILU_DEP_TICKET_US per chunk, and streams at
-// ILU_DEP_BW (measured on MI355X:
-// 2D diagonal-E p=2 sweeps over 246 levels of 123 elements take 4.8 us per
-// level launch and 1.7 us per dependency step; 3D Omega p=2 sweeps over 96
-// levels of 864 tets stream 2.1 TB/s level by level, 1.7 TB/s dependency-
-// driven).  The elements and levels are those of the instances being solved
-// when the batched solver says so, else the whole mesh.
-constexpr double ILU_LEVEL_FLOOR_US = 4.5, ILU_LEVEL_BW = 2.1e6;   // bytes per us
-constexpr double ILU_DEP_STEP_US = 1.7, ILU_DEP_BW = 1.7e6;
-// and one ticket (a device-scope atomic on one word) per chunk: about 21 ns
-// each, measured as the per-element rate of one-element chunks
-constexpr double ILU_DEP_TICKET_US = 0.021;
+// Which sweeps an application runs (both give the same bits).  The sweeps level
+// by level take ILU_LEVEL_US a launch and stream the blocks at ILU_LEVEL_BW; the
+// dependency-driven ones take ILU_DEP_STEP_US per level of the critical path,
+// ILU_DEP_EL_US per element, or stream at ILU_DEP_BW.  Measured (MI355X, one
+// triangle): natural numbering, hundreds of levels: 2D diagonal-E p=2 n=300 600
+// levels 3131 us level by level, 619 us dependency-driven; 3D Omega p=2 n=20 80
+// levels 842 and 608 us; p=1 n=32 128 levels 919 and 617 us.  The same meshes
+// numbered at random, about 10 levels: diagonal-E n=64 47 and 39 us, n=180 171
+// and 218 us; 2D Omega p=1 n=48 51 and 34 us, n=200 84 and 184 us; 3D Omega p=2
+// n=10 121 and 89 us, n=16 281 and 287 us.  The elements and levels are those of
+// the instances being solved when the batched solver says so, else the whole
+// mesh.
+constexpr double ILU_LEVEL_US = 4.5, ILU_LEVEL_BW = 3.5e6;   // bytes per us
+constexpr double ILU_DEP_STEP_US = 0.85, ILU_DEP_EL_US = 0.0022, ILU_DEP_BW = 2.4e6;
 
 static bool ilu_use_dep(const pdes_ctx* c, const pdes_precond* p) {
   if (p->force) return p->force == 2;
@@ -1053,32 +1260,25 @@ static bool ilu_use_dep(const pdes_ctx* c, const pdes_precond* p) {
   for (int pass = 0; pass < 2; ++pass) {
     const double L = std::max(1, hint ? (pass ? c->ilu_hint_lb : c->ilu_hint_lf)
                                       : (int)(pass ? p->bptr.size() : p->fptr.size()) - 1);
-    lev += L * std::max(ILU_LEVEL_FLOOR_US, nel / L * be / ILU_LEVEL_BW);
-    dep += std::max(std::max(L * ILU_DEP_STEP_US, (nel / p->chunk + L) * ILU_DEP_TICKET_US), nel * be / ILU_DEP_BW);
+    lev += L * ILU_LEVEL_US + nel * be / ILU_LEVEL_BW;
+    dep += std::max({L * ILU_DEP_STEP_US, nel * ILU_DEP_EL_US, nel * be / ILU_DEP_BW});
   }
   return dep < lev;
 }
 
-struct ChunkSelected {
+struct SetSelected {
   const int32_t* order;
-  int chunk;
+  const int32_t* start;
   const int32_t* el_inst;
   const int32_t* sel;
-  __host__ __device__ bool operator()(const int32_t& ch) const {
-    for (int k = 0; k < chunk; ++k) {
-      const int32_t e = order[(int64_t)ch * chunk + k];
-      if (e >= 0 && sel[el_inst[e]]) return true;
-    }
-    return false;
-  }
+  __host__ __device__ bool operator()(const int32_t& set) const { return sel[el_inst[order[start[set]]]] != 0; }
 };
 
 // The batched solver's hint for the ILU(0) applications of its next Arnoldi
 // steps: they touch only the elements of the instances with inst_sel[i] != 0
 // (nel of them, over lf forward and lb backward levels).  When the cost model
-// then picks the dependency-driven sweeps, the level-ordered element lists are
-// compacted to those instances (order kept), so a sweep dispatches and
-// tickets only their elements.  ilu_hint_clear ends the hint.
+// then picks the dependency-driven sweeps, the lists of sets are compacted to
+// those instances (order kept), so a sweep dispatches only their elements.  ilu_hint_clear ends the hint.
 int ilu_hint(pdes_ctx* c, const int32_t* inst_sel, int ninst, int64_t nel, int lf, int lb) {
   pdes_precond* p = c->pc_obj;
   c->ilu_hint_el = nel;
@@ -1086,7 +1286,7 @@ int ilu_hint(pdes_ctx* c, const int32_t* inst_sel, int ninst, int64_t nel, int l
   c->ilu_hint_lb = lb;
   c->ilu_sel = false;
   if (!p || p->kind != PDES_PC_ILU0 || !c->d_el_inst || !ilu_use_dep(c, p)) return PDES_OK;
-  const int64_t nf = p->fpad_n, nb = p->bpad_n;
+  const int64_t nf = p->fset.n, nb = p->bset.n;
   hipcub::CountingInputIterator<int32_t> ids(0);
   if (!p->d_fsel) {
     if (hipMalloc((void**)&p->d_fsel, std::max<int64_t>(1, nf) * sizeof(int32_t)) != hipSuccess ||
@@ -1097,7 +1297,7 @@ int ilu_hint(pdes_ctx* c, const int32_t* inst_sel, int ninst, int64_t nel, int l
     }
     size_t bytes = 0;
     PDES_HIP(hipcub::DeviceSelect::If(nullptr, bytes, ids, p->d_fsel, p->d_nsel, (int)std::max(nf, nb),
-                                      ChunkSelected{p->d_fpad, p->chunk, c->d_el_inst, nullptr}, c->stream));
+                                      SetSelected{p->fset.d_order, p->fset.d_start, c->d_el_inst, nullptr}, c->stream));
     if (hipMalloc(&p->d_select_tmp, std::max<size_t>(bytes, 16)) != hipSuccess) {
       set_error("device allocation of the ILU selection work space failed");
       return PDES_ERR_NOMEM;
@@ -1116,10 +1316,10 @@ int ilu_hint(pdes_ctx* c, const int32_t* inst_sel, int ninst, int64_t nel, int l
   PDES_HIP(hipMemcpyAsync(p->d_inst_sel, inst_sel, ninst * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
   size_t bytes = p->select_tmp_bytes;
   PDES_HIP(hipcub::DeviceSelect::If(p->d_select_tmp, bytes, ids, p->d_fsel, p->d_nsel, (int)nf,
-                                    ChunkSelected{p->d_fpad, p->chunk, c->d_el_inst, p->d_inst_sel}, c->stream));
+                                    SetSelected{p->fset.d_order, p->fset.d_start, c->d_el_inst, p->d_inst_sel}, c->stream));
   bytes = p->select_tmp_bytes;
   PDES_HIP(hipcub::DeviceSelect::If(p->d_select_tmp, bytes, ids, p->d_bsel, p->d_nsel + 1, (int)nb,
-                                    ChunkSelected{p->d_bpad, p->chunk, c->d_el_inst, p->d_inst_sel}, c->stream));
+                                    SetSelected{p->bset.d_order, p->bset.d_start, c->d_el_inst, p->d_inst_sel}, c->stream));
   int32_t cnt[2] = {0, 0};
   PDES_HIP(hipMemcpyAsync(cnt, p->d_nsel, sizeof(cnt), hipMemcpyDeviceToHost, c->stream));
   PDES_HIP(hipStreamSynchronize(c->stream));
@@ -1176,30 +1376,26 @@ static int ilu_apply(pdes_ctx* c, const double* b, double* x) {
   constexpr int LPR = ilu_lanes<N, DIAGE>();
   constexpr int EPB = 256 / (N * LPR);
   if (ilu_use_dep(c, p)) {
-    constexpr int CH = ilu_dep_chunk(N, DIAGE);
-    static_assert(ilu_dep_lanes(N, DIAGE) == LPR, "the dependency-driven and level sweeps split rows alike");
-    if (p->chunk != CH) {
-      set_error("ILU chunk size mismatch");
-      return PDES_ERR_ARG;
-    }
     const bool sel = c->ilu_sel && c->ilu_hint_el >= 0;
     for (int pass = 0; pass < 2; ++pass) {
-      const int32_t* order = pass == 0 ? p->d_fpad : p->d_bpad;
-      const int32_t* chunks = sel ? (pass == 0 ? p->d_fsel : p->d_bsel) : nullptr;
-      const int64_t nch = sel ? (pass == 0 ? p->sel_nf : p->sel_nb) : (pass == 0 ? p->fpad_n : p->bpad_n);
-      if (nch == 0) continue;
+      const pdes_precond::Sets& k = pass == 0 ? p->fset : p->bset;
+      const int32_t* sets = sel ? (pass == 0 ? p->d_fsel : p->d_bsel) : nullptr;
+      const int64_t nsets = sel ? (pass == 0 ? p->sel_nf : p->sel_nb) : k.n;
+      if (nsets == 0) continue;
       // forward: b -> y, x set pending; backward: y -> x, y set pending again
       const double* in = pass == 0 ? b : p->d_y;
       double* out = pass == 0 ? p->d_y : x;
       double* reset = pass == 0 ? x : p->d_y;
       if (j->fp64)
-        hipLaunchKernelGGL((ilu_sweep_dep_kernel<NP, ND, NS, DIAGE, double, LPR, CH>), dim3((unsigned)nch),
-                           dim3(CH * N * LPR), 0, c->stream, order, chunks, nch, j->d_rowptr, j->d_colind, p->d_own,
+        hipLaunchKernelGGL((ilu_sweep_dep_kernel<NP, ND, NS, DIAGE, double>), dim3((unsigned)nsets),
+                           dim3(IluSet<NP, ND, NS, DIAGE, double>::THREADS), 0, c->stream, k.d_order, k.d_start,
+                           k.d_place, sets, nsets, c->d_elface, j->d_rowptr, j->d_colind, p->d_own,
                            (const double*)j->d_vals, p->d_inv, in, out, reset, pass == 0, c->d_el_inst, c->d_mask,
                            c->d_inst_active, p->d_sync);
       else
-        hipLaunchKernelGGL((ilu_sweep_dep_kernel<NP, ND, NS, DIAGE, float, LPR, CH>), dim3((unsigned)nch),
-                           dim3(CH * N * LPR), 0, c->stream, order, chunks, nch, j->d_rowptr, j->d_colind, p->d_own,
+        hipLaunchKernelGGL((ilu_sweep_dep_kernel<NP, ND, NS, DIAGE, float>), dim3((unsigned)nsets),
+                           dim3(IluSet<NP, ND, NS, DIAGE, float>::THREADS), 0, c->stream, k.d_order, k.d_start,
+                           k.d_place, sets, nsets, c->d_elface, j->d_rowptr, j->d_colind, p->d_own,
                            (const float*)j->d_vals, p->d_inv, in, out, reset, pass == 0, c->d_el_inst, c->d_mask,
                            c->d_inst_active, p->d_sync);
     }
@@ -1390,8 +1586,8 @@ int pc_apply(pdes_ctx* c, const double* b, double* x) {
 
 // What a captured sequence of preconditioner applications depends on besides
 // device data: the kind, the factor and matrix buffers, and for ILU(0) the
-// sweep kind and, for the dependency-driven sweeps over compacted chunk
-// lists, their lengths (launch sizes).
+// sweep kind and, for the dependency-driven sweeps over compacted lists of
+// sets, their lengths (launch sizes).
 void pc_graph_key(const pdes_ctx* c, int64_t key[6]) {
   const pdes_precond* p = c->pc_obj;
   for (int i = 0; i < 6; ++i) key[i] = 0;
@@ -1424,6 +1620,15 @@ int pc_check(pdes_ctx* c) {
   return PDES_OK;
 }
 
+// floats that the inverse of an element block of n unknowns takes
+int64_t pc_block_floats(int n) {
+#define PDES_BLOCK_FLOATS(D_, NP_, NF_, NS_, DE_) \
+  if (NP_ * (D_ + 2) == n) return InvLayout<NP_ * (D_ + 2)>::SIZE;
+  PDES_FOR_EACH_SHAPE(PDES_BLOCK_FLOATS)
+#undef PDES_BLOCK_FLOATS
+  return (int64_t)n * n;
+}
+
 int pc_setup(pdes_ctx* c, int kind) {
   PDES_CHECK(kind == PDES_PC_NONE || kind == PDES_PC_BJACOBI || kind == PDES_PC_ILU0, PDES_ERR_UNSUPPORTED,
              "preconditioner kind %d is not available", kind);
@@ -1438,7 +1643,7 @@ int pc_setup(pdes_ctx* c, int kind) {
     for (auto& g : p->graphs) hipGraphExecDestroy(g.exec);
     p->graphs.clear();
     p->n = n;
-    if (hipMalloc((void**)&p->d_inv, (size_t)c->numEl * n * n * sizeof(float)) != hipSuccess) {
+    if (hipMalloc((void**)&p->d_inv, (size_t)c->numEl * pc_block_floats(n) * sizeof(float)) != hipSuccess) {
       set_error("device allocation of the block-Jacobi factors failed");
       return PDES_ERR_NOMEM;
     }
