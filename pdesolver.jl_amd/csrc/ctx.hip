@@ -57,6 +57,27 @@ int bc_state_setup(pdes_ctx* c) {
 
 using namespace pdes;
 
+// Default launch variant of the residual (residual_launch.hpp), from times of
+// all variants on MI355X (us):
+//   split form, diagonal-E: 4 waves per SIMD (2D p=1..3, 18,818 to 131,072
+//     triangles: 44.7, 68.6, 24.9 against 46.6, 70.6, 26.2), but 3 for p=4
+//     (232.7; small blocks 258.1);
+//   split form, dense faces: the small blocks (2D p=2, 45,000 triangles: 89.1
+//     against 106.3; 3D p=2, 16,464 tets: 176.1 against 238.3);
+//   weak form, up to 512 blocks of 192 threads, and 2D Omega p=1: small blocks,
+//     vector ALUs (800 triangles: Omega p=1 5.9 against 6.5 to 7.5, p=3 7.9
+//     against 8.9, diagonal-E p=2 5.8 against 6.0 to 6.4; 3,072 tets p=2 11.6
+//     against 12.1 to 12.5; 131,072 triangles Omega p=1 20.9 against 22.9);
+//   weak form beyond: large blocks, with Q^T F on the matrix cores from 10 nodes
+//     an element (Omega p=4 18.1 against 20.7, 3D p=2, 48,000 tets, 57.3 against
+//     60.1, diagonal-E p=2 45.6 against 48.7) and 4 waves, 3 for the 3D Omega
+//     ones (p=1, 48,000 tets: 20.1 against 23.0).
+static int default_variant(const pdes_ctx* c) {
+  if (c->phys.volume_integral_type == 2) return !c->diag_e ? 2 : c->Np > 18 ? 0 : 1;
+  if ((int64_t)c->numEl * c->Np < 512 * 192 || (c->dim == 2 && c->Np == 3)) return 2;
+  return (c->Np >= 10 ? 4 : 0) + (c->dim == 2 ? 1 : 0);
+}
+
 extern "C" {
 
 const char* pdes_last_error(void) { return g_err; }
@@ -97,14 +118,7 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
   c->pc.rho_free = ph->rho_free;
   c->pc.E_free = ph->p_free / (ph->gamma - 1) + 0.5 * ph->rho_free * ph->Ma * ph->Ma;  // types.jl:252
   c->pc.vortex_Min = ph->vortex_Min;
-  // default launch variants measured on MI355X: the split form at 3 waves per
-  // SIMD; the weak form at 4, with Q^T F on the matrix cores where its product
-  // lays over the flux planes in LDS ((dim - 1) Np >= nfaces Nf), else on the
-  // vector ALUs (the product's own LDS array costs a block per CU)
-  if (ph->volume_integral_type == 2)
-    c->res_variant[0] = c->res_variant[1] = 0;
-  else
-    c->res_variant[0] = c->res_variant[1] = ((c->dim - 1) * c->Np >= c->nfaces * c->Nf) ? 5 : 1;
+  c->res_variant[0] = c->res_variant[1] = default_variant(c);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     set_error("hipStreamCreate failed");
     delete c;
@@ -143,6 +157,7 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
       int node = s->perm[st * nfaces + f];
       if (node < 0 || node >= Np) { set_error("perm entry out of range"); pdes_ctx_destroy(c); return PDES_ERR_ARG; }
       c->h_nodepos[(size_t)node * nfaces + f] = st;
+      c->permbits[f] |= (uint64_t)node << (4 * st);
     }
 
   // element -> face connectivity

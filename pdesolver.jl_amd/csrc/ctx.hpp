@@ -30,6 +30,7 @@ struct pdes_ctx {
   double* d_interp = nullptr;
   int32_t* d_perm = nullptr;
   int32_t* d_nbrperm = nullptr;
+  uint64_t permbits[4] = {0, 0, 0, 0};   // DevSBP::permbits
   int32_t* d_nodepos = nullptr;
   double* d_wface = nullptr;
   double* d_Minv = nullptr;
@@ -100,7 +101,9 @@ struct pdes_ctx {
   int64_t active_count() const { return nlist >= 0 ? nlist : numEl; }
   const int32_t* active_list() const { return nlist >= 0 ? d_el_list : nullptr; }
   pdes::DevSBP devsbp() const {
-    return pdes::DevSBP{d_Q, d_interp, d_perm, d_nbrperm, d_nodepos, d_wface, norient, d_S2c};
+    pdes::DevSBP s{d_Q, d_interp, d_perm, d_nbrperm, d_nodepos, d_wface, norient, d_S2c, {0, 0, 0, 0}};
+    for (int f = 0; f < 4; ++f) s.permbits[f] = permbits[f];
+    return s;
   }
 };
 

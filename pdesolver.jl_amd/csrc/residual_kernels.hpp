@@ -71,6 +71,7 @@ struct DevSBP {
   const double* __restrict__ wface;    // [k]
   int32_t norient;
   const double* __restrict__ S2c;      // [d][dd][a] = Q_d[a][b] - Q_d[b][a], b = a + dd mod Np, dd <= Np/2
+  uint64_t permbits[4];                // dense faces: perm[s][f], four bits a stencil position (node f of 16)
 };
 
 __device__ __forceinline__ int32_t launch_count(const DevMesh& m) { return m.el_list ? m.nlist : m.numEl; }
@@ -173,11 +174,18 @@ struct ResidualSmem {
   // read), which leaves room for one more workgroup per CU
   static constexpr bool Q_LDS = !Op::DIAGE;
   T q[Q_LDS ? EPB : 1][Q_LDS ? NP : 1][ND];
+  // weak form on dense faces, p >= 2: the face records, and the states of both
+  // sides at the face nodes in the (then dead) flux planes; p = 1, where an
+  // element has as many nodes as faces: one thread takes a whole face
+  static constexpr bool FACEWISE = (VOL == VOL_WEAK) && !Op::DIAGE && NP == NFACES;
+  static constexpr bool INTERP = (VOL == VOL_WEAK) && !Op::DIAGE && !FACEWISE;
+  ElFace rec[INTERP ? EPB : 1][NFACES];
   // weak form: volume fluxes; split form: IR z-variables and partner contributions
   // (the F and C arrays are planes of one value per (element, node),
   //  [component][element][node], so that the lanes of a pair round, which
   //  read node i + dd, touch consecutive words)
-  T F[EPB][(VOL == VOL_WEAK) ? DIM * NP * ND : NP * ND];
+  static constexpr int FLUXES = (VOL == VOL_WEAK) ? DIM * NP * ND : NP * ND, FACES = 2 * ND * NFACES * NF;
+  T F[EPB][(INTERP && FACES > FLUXES) ? FACES : FLUXES];
   // split form: partner contributions, two buffers used in alternate rounds
   T C[(VOL == VOL_SPLIT) ? 2 : 1][EPB][(VOL == VOL_SPLIT) ? NP * ND : 1];
   // entropy-stable element face integral (dense faces): own IR entropy
@@ -197,12 +205,14 @@ struct ResidualSmem {
   static constexpr int G_C_BUF = ((NP / 2) + 1) & 1;
   static_assert(!G_IN_F || DIM * NP >= NFACES * NF, "face contributions must fit the weak-form flux planes");
   T G[(G_IN_F || G_IN_C) ? 1 : EPB][NFACES][NF][ND];
-  // weak form on the matrix cores: the volume term of every (element, node)
-  // as planes [component][element][node], laid over the flux planes above
-  // the face contributions where they fit there (the flux planes are dead
-  // once the product is formed), else in an array of their own
-  static constexpr bool RV_IN_F = (DIM - 1) * NP >= NFACES * NF;
+  // weak form on the matrix cores: where the volume term of every (element,
+  // node) goes, as planes [component][element][node].  Dense faces, p >= 2: over
+  // the neighbours' face states, once the numerical fluxes are formed.  Else
+  // over the flux planes above the face contributions where it fits there (the
+  // flux planes are dead once the product is formed), else in an array of its own.
+  static constexpr bool RV_IN_F = INTERP || (DIM - 1) * NP >= NFACES * NF;
   static constexpr int RV_OFF = ND * EPB * NFACES * NF;
+  static_assert(!INTERP || NFACES * NF >= NP, "the volume term must fit the neighbours' face states");
   double Rv[(MF && !RV_IN_F) ? ND : 1][(MF && !RV_IN_F) ? EPB * NP : 1];
 };
 
@@ -321,6 +331,87 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
     }
   }
 
+  // dense weak form, p = 1: the neighbour's nodes at face i (or the boundary
+  // states), the face's normals and the face-node numbers on the other side
+  T xw[Smem::FACEWISE ? ST : 1][ND];
+  double nrmw[Smem::FACEWISE ? NF : 1][DIM];
+  int mw[Smem::FACEWISE ? NF : 1];
+  ElFace recw{-1, 0, 0, 0};
+  if constexpr (Smem::FACEWISE) {
+    if (active) {
+      recw = mesh.elface[e * NFACES + i];
+      const bool inner = recw.x >= 0;
+      const int side = inner ? (recw.z >> 16) & 1 : 0;
+      if (inner) {
+        const int fN = recw.z & 0xff;
+        uint64_t bits = sbp.permbits[0];
+#pragma unroll
+        for (int g = 1; g < NFACES; ++g) bits = fN == g ? sbp.permbits[g] : bits;
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+          for (int c = 0; c < ND; ++c)
+            xw[s][c] = Io<T>::load(qin, vin, ((int64_t)recw.x * NP + (int)(bits >> (4 * s) & 15)) * ND + c);
+      } else {
+#pragma unroll
+        for (int m = 0; m < NF; ++m)
+#pragma unroll
+          for (int c = 0; c < ND; ++c) xw[m][c] = T(mesh.qbc[((int64_t)recw.y * NF + m) * ND + c]);
+      }
+#pragma unroll
+      for (int m = 0; m < NF; ++m) mw[m] = m;
+      if (inner) {
+        const int o = (recw.z >> 8) & 0xff;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) {
+          const int kR = sbp.nbrperm[k * sbp.norient + o];
+#pragma unroll
+          for (int m = 0; m < NF; ++m)
+            if (side ? kR == m : k == m) mw[m] = side ? k : kR;
+        }
+      }
+      const double* nr = (inner ? mesh.nrm_face : mesh.nrm_bndry) + (int64_t)recw.y * (NF * DIM);
+#pragma unroll
+      for (int m = 0; m < NF; ++m)
+#pragma unroll
+        for (int x = 0; x < DIM; ++x) nrmw[m][x] = nr[(side ? mw[m] : m) * DIM + x];
+    }
+  }
+  // dense weak form, p >= 2: task t = (face t / ND, component t % ND) of this element
+  // interpolates that component of both sides to the face nodes.  The
+  // neighbour's nodes (or the boundary states) are issued here, each lane its
+  // own component, so that these dependent loads (record, then state) overlap
+  // with the volume phase and the lanes of a face read consecutive words
+  constexpr int TASKS = Smem::INTERP ? (NFACES * ND + NP - 1) / NP : 1;
+  constexpr int XN = Smem::INTERP ? ST : 1;
+  T xn[TASKS][XN];
+  int bnd[TASKS];
+  if constexpr (Smem::INTERP) {
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int t = i + u * NP;
+      bnd[u] = 0;
+      if (active && t < NFACES * ND) {
+        const int f = t / ND, c = t - f * ND;
+        const ElFace rec = mesh.elface[e * NFACES + f];
+        if (c == 0) sm.rec[el][f] = rec;
+        bnd[u] = rec.x < 0;
+        if (rec.x >= 0) {
+          const int fN = rec.z & 0xff;
+          uint64_t bits = sbp.permbits[0];
+#pragma unroll
+          for (int g = 1; g < NFACES; ++g) bits = fN == g ? sbp.permbits[g] : bits;
+#pragma unroll
+          for (int s = 0; s < ST; ++s)
+            xn[u][s] = Io<T>::load(qin, vin, ((int64_t)rec.x * NP + (int)(bits >> (4 * s) & 15)) * ND + c);
+        } else {
+#pragma unroll
+          for (int m = 0; m < NF; ++m) xn[u][m] = T(mesh.qbc[((int64_t)rec.y * NF + m) * ND + c]);
+        }
+      }
+    }
+  }
+
   T qi[ND];
   if (active) {
 #pragma unroll
@@ -364,6 +455,12 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
   WeakVolumeMfma<DIM, NP, ND, EPB> mfma;
   double* rvpl = nullptr;
   if constexpr (MF) rvpl = Smem::RV_IN_F ? &sm.F[0][0] + Smem::RV_OFF : &sm.Rv[0][0];
+  // dense weak form: the block's face slots (element, face, face node) go over
+  // all its threads; slot t = tid + u * threads
+  constexpr int SLOTS = EPB * NFACES * NF;
+  constexpr int ROUNDS = Smem::INTERP ? (SLOTS + EPB * NP - 1) / (EPB * NP) : 1;
+  double nrmf[ROUNDS][DIM];
+  int kRf[ROUNDS];
 
   if constexpr (VOL == VOL_WEAK) {
     // getEulerFlux: flux in parametric direction d uses nrm = dxidx[d, :, j, e]
@@ -380,6 +477,23 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
       }
     }
     __syncthreads();
+    if constexpr (Smem::INTERP) {
+      // the slots' normals and neighbour face nodes, issued ahead of the volume term
+      const int64_t left = launch_count(mesh) - (eslot - el);
+      const int slots = (int)(left < EPB ? left : EPB) * (NFACES * NF);
+#pragma unroll
+      for (int u = 0; u < ROUNDS; ++u) {
+        const int t = tid + u * (int)blockDim.x;
+        if (t < slots) {
+          const ElFace rec = (&sm.rec[0][0])[t / NF];
+          const int k = t - t / NF * NF;
+          const double* nr = (rec.x < 0 ? mesh.nrm_bndry : mesh.nrm_face) + ((int64_t)rec.y * NF + k) * DIM;
+#pragma unroll
+          for (int x = 0; x < DIM; ++x) nrmf[u][x] = nr[x];
+          kRf[u] = rec.x < 0 ? k : sbp.nbrperm[k * sbp.norient + ((rec.z >> 8) & 0xff)];
+        }
+      }
+    }
     // weakdifferentiate!(trans=true): res_i += sum_d sum_j Q_d[j][i] F_d[j]
     if constexpr (MF) {
       mfma.compute(sm.Q, zpl, tid);
@@ -394,7 +508,7 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
         }
     }
     __syncthreads();   // the face phase writes its contributions into the flux planes
-    if constexpr (MF) mfma.store(rvpl, tid);
+    if constexpr (MF && !Smem::INTERP) mfma.store(rvpl, tid);
   } else {
     // split form (calcVolumeIntegralsSplitFormLinear): per-node IR z-variables in LDS,
     // each unordered node pair evaluated once by the node that starts its circulant distance.
@@ -681,104 +795,117 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
         for (int c = 0; c < ND; ++c) sm.H[el][f][t][c] = h[c];
       }
     }
-  } else
-  {
-  if (active) {
-    for (int slot = i; slot < NFACES * NF; slot += NP) {
-      const int f = slot / NF;
-      const int k = slot - f * NF;
-      const ElFace rec = mesh.elface[e * NFACES + f];
-      T qL[ND], qR[ND], Fk[ND];
-      int m;
-      double sign;
-      if (rec.x < 0) {
-        // boundary: q_b = R q, state from the BC functor, RoeSolver
-        m = k;
-        sign = -1.0;
-        if constexpr (Op::DIAGE) {
-          const int node = sm.perm[k][f];
+  } else if constexpr (Smem::FACEWISE) {
+    // dense faces, weak form, p = 1: thread i takes face i, whose neighbour
+    // nodes it holds: no exchange through LDS, which p >= 2 pays for with
+    // occupancy.  The residual of 131,072 triangles takes 20.9 us (that way 28,
+    // 22.2 with one thread per face node that gathered the nodes here), 800
+    // triangles 5.9 (7.9).
+    static_assert(FLUX == PDES_FLUX_ROE && ST == NP, "dense weak form");
+    if (active) {
+      const bool inner = recw.x >= 0;
+      const int side = inner ? (recw.z >> 16) & 1 : 0;
 #pragma unroll
-          for (int c = 0; c < ND; ++c) qL[c] = sm.q[el][node][c];
-        } else {
+      for (int m = 0; m < NF; ++m) {
+        T qo[ND], qn[ND], qL[ND], qR[ND], Fk[ND];
 #pragma unroll
-          for (int c = 0; c < ND; ++c) qL[c] = 0.0;
-          for (int s = 0; s < ST; ++s) {
-            double r = sm.interp[s][k];
-            const int node = sm.perm[s][f];
+        for (int c = 0; c < ND; ++c) { qo[c] = 0.0; qn[c] = 0.0; }
 #pragma unroll
-            for (int c = 0; c < ND; ++c) qL[c] = qL[c] + r * sm.q[el][node][c];
+        for (int s = 0; s < ST; ++s) {
+          const double ro = sm.interp[s][m], rn = sm.interp[s][mw[m]];
+          const int node = sm.perm[s][i];
+#pragma unroll
+          for (int c = 0; c < ND; ++c) {
+            qo[c] = qo[c] + ro * sm.q[el][node][c];
+            qn[c] = qn[c] + rn * xw[s][c];
           }
         }
-        const int64_t b = rec.y;
-        double qg[ND];
-        bc_state<DIM>(mesh, rec, k, NF, qg);
 #pragma unroll
-        for (int c = 0; c < ND; ++c) qR[c] = qg[c];
-        roe_flux<DIM>(phys, qL, qR, mesh.nrm_bndry + (b * NF + k) * DIM, Fk);
-      } else {
-        const int64_t nb = rec.x;
-        const int fN = rec.z & 0xff;
-        const int o = (rec.z >> 8) & 0xff;
-        const int side = (rec.z >> 16) & 1;
-        const int kR = sbp.nbrperm[k * sbp.norient + o];
-#pragma unroll
-        for (int c = 0; c < ND; ++c) { qL[c] = 0.0; qR[c] = 0.0; }
-        if constexpr (Op::DIAGE) {
-          // SparseFace: R selects the face nodes
-          const int nodeL = sm.perm[k][side == 0 ? f : fN];
-          const int nodeR = sm.perm[kR][side == 0 ? fN : f];
-          if (side == 0) {
-            m = k;
-            sign = -1.0;
-#pragma unroll
-            for (int c = 0; c < ND; ++c) {
-              qL[c] = sm.q[el][nodeL][c];
-              qR[c] = Io<T>::load(qin, vin, (nb * NP + nodeR) * ND + c);
-            }
-          } else {
-            m = kR;
-            sign = 1.0;
-#pragma unroll
-            for (int c = 0; c < ND; ++c) {
-              qL[c] = Io<T>::load(qin, vin, (nb * NP + nodeL) * ND + c);
-              qR[c] = sm.q[el][nodeR][c];
-            }
-          }
-        } else if (side == 0) {
-          // this element is elementL
-          m = k;
-          sign = -1.0;
-          for (int s = 0; s < ST; ++s) {
-            const double rl = sm.interp[s][k], rr = sm.interp[s][kR];
-            const int nodeL = sm.perm[s][f], nodeR = sm.perm[s][fN];
-#pragma unroll
-            for (int c = 0; c < ND; ++c) {
-              qL[c] = qL[c] + rl * sm.q[el][nodeL][c];
-              qR[c] = qR[c] + rr * Io<T>::load(qin, vin, (nb * NP + nodeR) * ND + c);
-            }
-          }
-        } else {
-          m = kR;
-          sign = 1.0;
-          for (int s = 0; s < ST; ++s) {
-            const double rl = sm.interp[s][k], rr = sm.interp[s][kR];
-            const int nodeL = sm.perm[s][fN], nodeR = sm.perm[s][f];
-#pragma unroll
-            for (int c = 0; c < ND; ++c) {
-              qL[c] = qL[c] + rl * Io<T>::load(qin, vin, (nb * NP + nodeL) * ND + c);
-              qR[c] = qR[c] + rr * sm.q[el][nodeR][c];
-            }
-          }
+        for (int c = 0; c < ND; ++c) {
+          const T other = inner ? qn[c] : xw[m][c];
+          qL[c] = side ? other : qo[c];
+          qR[c] = side ? qo[c] : other;
         }
-        const double* nrm = mesh.nrm_face + ((int64_t)rec.y * NF + k) * DIM;
-        if constexpr (FLUX == PDES_FLUX_ROE) roe_flux<DIM>(phys, qL, qR, nrm, Fk);
-        else irslf_flux<DIM>(phys, qL, qR, nrm, Fk);
+        roe_flux<DIM>(phys, qL, qR, nrmw[m], Fk);
+        const double wgt = (side ? 1.0 : -1.0) * sm.wface[m];
+#pragma unroll
+        for (int c = 0; c < ND; ++c) gpl[((c * EPB + el) * NFACES + i) * NF + m] = wgt * Fk[c];
       }
-      const double wgt = sign * sm.wface[m];
-#pragma unroll
-      for (int c = 0; c < ND; ++c) gpl[((c * EPB + el) * NFACES + f) * NF + m] = wgt * Fk[c];
     }
-  }
+  } else {
+    // dense faces, weak form, p >= 2.  What bounds this phase is LDS reads and, before
+    // the neighbours' nodes were loaded ahead, the latency of gathering them:
+    // one thread per (face, component) reads each node's value once for all
+    // face nodes of both sides (the interpolation matrix is the same for every
+    // lane and comes through the scalar cache), instead of every face node's
+    // thread reading every node of both sides.  Residual, before and after:
+    // 3D p=2, 48,000 tets 78 -> 57 us (0.67 TB/s; waves for the numerical flux
+    // and the lift wait, two a SIMD); 2D p=3, 18,818 triangles 19.6 -> 14.0 us,
+    // 800 triangles 12 -> 7.9 us; p=4 23.2 -> 18.1 us; p=2, 131,072 triangles
+    // 48 -> 39.6 us.
+    static_assert(VOL == VOL_WEAK && FLUX == PDES_FLUX_ROE && ST == NP, "dense weak form");
+    typedef const double __attribute__((address_space(4))) uniform_double;
+    uniform_double* const R = (uniform_double*)sbp.interp;
+    T* const npl = gpl + ND * SLOTS;   // own states at [c][el][f][m]: gpl, the neighbours': npl
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int t = i + u * NP;
+      if (active && t < NFACES * ND) {
+        const int f = t / ND, c = t - f * ND;
+        uint64_t bits = sbp.permbits[0];
+#pragma unroll
+        for (int g = 1; g < NFACES; ++g) bits = f == g ? sbp.permbits[g] : bits;
+        T xo[NF], xf[NF];
+#pragma unroll
+        for (int m = 0; m < NF; ++m) { xo[m] = 0.0; xf[m] = 0.0; }
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+          const T qs = sm.q[el][(int)(bits >> (4 * s) & 15)][c];
+#pragma unroll
+          for (int m = 0; m < NF; ++m) {
+            const double r = R[s * NF + m];
+            xo[m] = xo[m] + r * qs;
+            xf[m] = xf[m] + r * xn[u][s];
+          }
+        }
+        const int at = ((c * EPB + el) * NFACES + f) * NF;
+#pragma unroll
+        for (int m = 0; m < NF; ++m) {
+          gpl[at + m] = xo[m];
+          npl[at + m] = bnd[u] ? xn[u][m] : xf[m];
+        }
+      }
+    }
+    __syncthreads();
+    const int64_t left = launch_count(mesh) - (eslot - el);
+    const int slots = (int)(left < EPB ? left : EPB) * (NFACES * NF);
+#pragma unroll
+    for (int u = 0; u < ROUNDS; ++u) {
+      const int t = tid + u * (int)blockDim.x;
+      if (t < slots) {
+        const ElFace rec = (&sm.rec[0][0])[t / NF];
+        const int k = t - t / NF * NF, face = t - k;
+        // elementR (side 1) meets elementL's face node k at its own node kR
+        const int side = rec.x < 0 ? 0 : (rec.z >> 16) & 1;
+        const int m = side ? kRf[u] : k, mn = side ? k : kRf[u];
+        T qL[ND], qR[ND], Fk[ND];
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+          const T qo = gpl[c * SLOTS + face + m], qn = npl[c * SLOTS + face + mn];
+          qL[c] = side ? qn : qo;
+          qR[c] = side ? qo : qn;
+        }
+        roe_flux<DIM>(phys, qL, qR, nrmf[u], Fk);
+        const double wgt = (side ? 1.0 : -1.0) * sm.wface[m];
+        // (this slot alone reads and writes its own state's place)
+#pragma unroll
+        for (int c = 0; c < ND; ++c) gpl[c * SLOTS + face + m] = wgt * Fk[c];
+      }
+    }
+    if constexpr (MF) {
+      __syncthreads();
+      mfma.store(rvpl, tid);
+    }
   }
   __syncthreads();
   if (active) {

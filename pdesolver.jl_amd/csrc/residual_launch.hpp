@@ -1,17 +1,17 @@
 // residual_launch.hpp -- launch-variant interface of the fused residual kernel.
 //
 // Tunable launch variants of the FP64 value kernel (the directional-derivative
-// kernel always uses variant 2's shape with 2 waves):
-//   0: elements per block = 256/Np, 3 waves per SIMD
-//   1: elements per block = 256/Np, 4 waves per SIMD
-//   2: elements per block = 128/Np, 3 waves per SIMD
-//   3: elements per block = 128/Np, 4 waves per SIMD
+// kernel always takes 128 threads, 64 for entropy-stable face integrals, 2 waves):
+//   0: large blocks, 3 waves per SIMD      1: large blocks, 4 waves per SIMD
+//   2: small blocks, 3 waves per SIMD      3: small blocks, 4 waves per SIMD
+// (whole elements in 256 and 128 threads; dense-face weak form 192 and 64;
+// entropy-stable face integrals 128 and 64)
 //   4-7: the weak form only: variants 0-3 with the volume term Q^T F on the
 //        FP64 matrix cores (blocks rounded up to whole waves); the split form
 //        runs variant (v & 3) for these
 // The waves-per-SIMD bound trades registers for occupancy; the choice is
-// made per context by the autotuner (pdes_autotune) or from the default
-// table in residual.hip.
+// made per context by the autotuner (pdes_autotune) or by default_variant
+// (ctx.hip).
 #pragma once
 #include "ctx.hpp"
 

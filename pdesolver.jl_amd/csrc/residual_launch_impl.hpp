@@ -31,12 +31,17 @@ static int launch_cfg(pdes_ctx* c, const double* q, const double* v, double* res
 template <class Op, int VOL, int FLUX, class T>
 static int launch_one(pdes_ctx* c, const double* q, const double* v, double* res, double* jv, int32_t* flag,
                       const RKStage* rk, int variant) {
-  // the entropy-stable face integral stages the neighbours' stencil data in
-  // LDS: half the elements per block
-  constexpr int FULL = (FLUX == PDES_FLUX_ESLF ? 128 : 256) / Op::NP;
-  constexpr int HALF = (FLUX == PDES_FLUX_ESLF ? 64 : 128) / Op::NP;
+  // threads per block.  The entropy-stable face integral stages the neighbours'
+  // stencil data in LDS: half the elements per block.  Dense-face weak form:
+  // three waves where blocks are many (3D p=2, 48,000 tets: 256 threads 63.5 us,
+  // 192 57.7, 128 66.2, 64 67.3; what fits a CU's LDS counts), one where they
+  // are few (2D p=1, 800 triangles: 256 7.0 us, 128 6.2, 64 5.7).
+  constexpr bool DENSE_WEAK = VOL == VOL_WEAK && !Op::DIAGE;
+  constexpr int FULL = (FLUX == PDES_FLUX_ESLF ? 128 : DENSE_WEAK ? 192 : 256) / Op::NP;
+  constexpr int HALF = (FLUX == PDES_FLUX_ESLF || DENSE_WEAK ? 64 : 128) / Op::NP;
   if constexpr (!std::is_same<T, double>::value) {
-    return launch_cfg<Op, VOL, FLUX, T, HALF, 2>(c, q, v, res, jv, flag, nullptr);
+    constexpr int EPB = (FLUX == PDES_FLUX_ESLF ? 64 : 128) / Op::NP;
+    return launch_cfg<Op, VOL, FLUX, T, EPB, 2>(c, q, v, res, jv, flag, nullptr);
   } else {
     if constexpr (VOL == VOL_WEAK) {
       switch (variant) {

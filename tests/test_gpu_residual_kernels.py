@@ -1,0 +1,45 @@
+"""The dense-face weak form of the residual kernel at the edges of its
+workgroups: whole and part-filled last blocks, elements whose neighbours are
+numbered before and after them, every launch variant."""
+import numpy as np
+import pytest
+
+from pdes_amd import abi, euler, problems
+from pdes_amd._lib import check, lib
+from helpers import assert_parity, state_for
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,p", [("vortex", 1), ("vortex", 2), ("vortex", 3), ("vortex", 4), ("cube", 1),
+                                    ("cube", 2)])
+def test_dense_weak_residual_at_block_edges(oracle, kind, p):
+    """Residual and directional derivative on 2, 32 and 128 triangles (6 and 48
+    tets), numbered at random: the oracle's values to 1e-12, the same bits from
+    all eight launch variants, and derivatives that the oracle's complex step
+    gives to 1e-12."""
+    for n in (1, 4, 8) if kind == "vortex" else (1, 2):
+        print(f"case {kind} n={n} p={p}", flush=True)
+        m, op, ph = problems.make_problem(kind, n, p, "omega", "roe")
+        perm = np.random.default_rng(n).permutation(m.numEl)
+        place = np.argsort(perm).astype(m.interfaces.dtype)
+        for a in ("coords", "dxidx", "jac", "vert_coords"):
+            setattr(m, a, np.ascontiguousarray(getattr(m, a)[perm]))
+        m.interfaces[:, :2] = place[m.interfaces[:, :2]]
+        m.bndryfaces[:, 0] = place[m.bndryfaces[:, 0]]
+        b = abi.make_descriptors(m, op, ph)
+        q = state_for(kind, m, ph)
+        ref, scale = oracle.residual(b, q), oracle.residual_scale(b, q)
+        eqn = euler.EulerData(m, op, ph)
+        eqn.set_q(q)
+        first = None
+        for var in range(8):
+            check(lib().pdes_set_launch_variant(eqn.ctx, var, var))
+            euler.evalResidual(m, op, eqn)
+            assert_parity(eqn.res, ref, scale, 1e-12, f"n {n} variant {var}")
+            first = eqn.res.copy() if first is None else first
+            assert np.array_equal(eqn.res, first), f"n {n}: variant {var} differs from variant 0"
+        v = np.random.default_rng(7).standard_normal(q.shape)
+        jv = oracle.jv_complex_step(b, q, v)
+        assert np.abs(euler.evaldRdqProduct(eqn, v) - jv).max() <= 1e-12 * np.abs(jv).max()
+        eqn.free()
