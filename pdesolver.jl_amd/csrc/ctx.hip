@@ -62,8 +62,9 @@ using namespace pdes;
 //   split form, diagonal-E: 4 waves per SIMD (2D p=1..3, 18,818 to 131,072
 //     triangles: 44.7, 68.6, 24.9 against 46.6, 70.6, 26.2), but 3 for p=4
 //     (232.7; small blocks 258.1);
-//   split form, dense faces: the small blocks (2D p=2, 45,000 triangles: 89.1
-//     against 106.3; 3D p=2, 16,464 tets: 176.1 against 238.3);
+//   split form, dense faces: large blocks, 4 waves (2D p=2, 45,000 triangles:
+//     61.7 against 63.0 to 64.5; p=3, 18,818: 66.0 against 67.6 to 70.1), 3D 3
+//     (p=2, 16,464 tets: 94.6 against 109.8);
 //   weak form, up to 512 blocks of 192 threads, and 2D Omega p=1: small blocks,
 //     vector ALUs (800 triangles: Omega p=1 5.9 against 6.5 to 7.5, p=3 7.9
 //     against 8.9, diagonal-E p=2 5.8 against 6.0 to 6.4; 3,072 tets p=2 11.6
@@ -73,7 +74,7 @@ using namespace pdes;
 //     60.1, diagonal-E p=2 45.6 against 48.7) and 4 waves, 3 for the 3D Omega
 //     ones (p=1, 48,000 tets: 20.1 against 23.0).
 static int default_variant(const pdes_ctx* c) {
-  if (c->phys.volume_integral_type == 2) return !c->diag_e ? 2 : c->Np > 18 ? 0 : 1;
+  if (c->phys.volume_integral_type == 2) return (c->diag_e ? c->Np > 18 : c->dim == 3) ? 0 : 1;
   if ((int64_t)c->numEl * c->Np < 512 * 192 || (c->dim == 2 && c->Np == 3)) return 2;
   return (c->Np >= 10 ? 4 : 0) + (c->dim == 2 ? 1 : 0);
 }

@@ -159,6 +159,18 @@ struct RKStage {
   int32_t stage;                 // 0..3
 };
 
+// threads per element: one per node; entropy-stable face integrals one per
+// (face, stencil node), of which the first NP take the nodes.  That scheme is a
+// chain of two-point fluxes, bound by latency: with a thread per node an element
+// of 2D p=2 took 3 fluxes and as many barriers for the volume and 18 in a row
+// for the faces, with one wave a workgroup; now 1 and 6.  Derivative, 7,442
+// triangles 64.6 -> 35.2 us (p=2), 3,072 tets (p=2) 119.6 -> 53.6 us; residual,
+// 45,000 triangles 89.1 -> 61.7 us, 16,464 tets 169 -> 94.6 us.
+template <class Op, int FLUX>
+constexpr int threads_per_element() {
+  return FLUX == PDES_FLUX_ESLF ? Op::NFACES * Op::ST : Op::NP;
+}
+
 template <class Op, int VOL, int FLUX, int EPB, class T, bool MF = false>
 struct ResidualSmem {
   static constexpr int NP = Op::NP, ND = Op::ND, DIM = Op::DIM, NF = Op::NF, NFACES = Op::NFACES;
@@ -187,21 +199,23 @@ struct ResidualSmem {
   static constexpr int FLUXES = (VOL == VOL_WEAK) ? DIM * NP * ND : NP * ND, FACES = 2 * ND * NFACES * NF;
   T F[EPB][(INTERP && FACES > FLUXES) ? FACES : FLUXES];
   // split form: partner contributions, two buffers used in alternate rounds
-  T C[(VOL == VOL_SPLIT) ? 2 : 1][EPB][(VOL == VOL_SPLIT) ? NP * ND : 1];
+  // (entropy-stable face integrals keep all pairs' at once, in Zn, Wn and H)
+  static constexpr bool ES = (FLUX == PDES_FLUX_ESLF);
+  T C[(VOL == VOL_SPLIT && !ES) ? 2 : 1][EPB][(VOL == VOL_SPLIT && !ES) ? NP * ND : 1];
   // entropy-stable element face integral (dense faces): own IR entropy
   // variables, the neighbours' stencil z and entropy variables per face, and
   // the entropy-conservative sums per (face, own stencil node)
-  static constexpr bool ES = (FLUX == PDES_FLUX_ESLF);
   T W[EPB][ES ? NP : 1][ND];
   T Zn[EPB][ES ? NFACES : 1][ES ? Op::ST : 1][ND];
   T Wn[EPB][ES ? NFACES : 1][ES ? Op::ST : 1][ND];
   T H[EPB][ES ? NFACES : 1][ES ? Op::ST : 1][ND];
+  static_assert(!ES || 3 * NFACES * Op::ST >= NP / 2 * NP, "the pairs' contributions must fit");
   // face contributions; the weak form keeps them in the flux planes F, which
   // are dead once the volume term is summed (one more barrier, less LDS); the
   // split form keeps them, where they fit, in the partner buffer that the last
   // pair round does not use (its last reads precede that round's barrier)
   static constexpr bool G_IN_F = (VOL == VOL_WEAK);
-  static constexpr bool G_IN_C = (VOL == VOL_SPLIT) && (NP >= NFACES * NF);
+  static constexpr bool G_IN_C = (VOL == VOL_SPLIT) && !ES && (NP >= NFACES * NF);
   static constexpr int G_C_BUF = ((NP / 2) + 1) & 1;
   static_assert(!G_IN_F || DIM * NP >= NFACES * NF, "face contributions must fit the weak-form flux planes");
   T G[(G_IN_F || G_IN_C) ? 1 : EPB][NFACES][NF][ND];
@@ -300,8 +314,9 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
                 "the matrix-core volume term is the FP64 weak form");
 
   const int tid = threadIdx.x;
-  const int el = tid / NP;
-  const int i = tid - el * NP;
+  constexpr int TPE = threads_per_element<Op, FLUX>();
+  const int el = tid / TPE;
+  const int i = tid - el * TPE;
   // LDS planes: value c of node n of this block's element el at
   // [c * PL + el * NP + n] (weak form: component k of the flux in parametric
   // direction d as c = d * ND + k; split form: IR parameter vector z)
@@ -314,8 +329,9 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
   // neighbours (the adjacent batches, or a mesh row away) were most likely
   // just read into the same L2
   const int64_t eslot = xcd_contiguous_batch(blockIdx.x, gridDim.x) * EPB + el;
-  const bool active = (el < EPB) && (eslot < launch_count(mesh));
-  const int64_t e = active ? element_of(mesh, eslot) : 0;
+  const bool present = (el < EPB) && (eslot < launch_count(mesh));
+  const bool active = present && i < NP;   // this thread has a node
+  const int64_t e = present ? element_of(mesh, eslot) : 0;
 
   // diagonal-E: the slot record of this thread's first face slot (f, k) =
   // (i / NF, i % NF), then the neighbour's face-node state (or the boundary
@@ -412,6 +428,26 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
     }
   }
 
+  // entropy-stable face integral: task i = (face, stencil node) of this
+  // element; the neighbour's state there, issued ahead of the volume term
+  constexpr bool ES = Smem::ES;
+  ElFace rece{-1, 0, 0, 0};
+  T qe[ES ? ND : 1];
+  if constexpr (ES) {
+    if (present) {
+      rece = mesh.elface[e * NFACES + i / ST];
+      if (rece.x >= 0) {
+        const int fN = rece.z & 0xff;
+        uint64_t bits = sbp.permbits[0];
+#pragma unroll
+        for (int g = 1; g < NFACES; ++g) bits = fN == g ? sbp.permbits[g] : bits;
+        const int node = (int)(bits >> (4 * (i % ST)) & 15);
+#pragma unroll
+        for (int c = 0; c < ND; ++c) qe[c] = Io<T>::load(qin, vin, ((int64_t)rece.x * NP + node) * ND + c);
+      }
+    }
+  }
+
   T qi[ND];
   if (active) {
 #pragma unroll
@@ -425,11 +461,12 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
     }
   }
   double dxi[DIM][DIM];  // dxidx[e][i][x][xi]
-  if (active) {
+  if (ES ? present : active) {
+    const int node = ES && i >= NP ? NP - 1 : i;
 #pragma unroll
     for (int x = 0; x < DIM; ++x)
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) dxi[x][d] = metric<DIM, NP>(mesh, e, i)[x * DIM + d];
+      for (int d = 0; d < DIM; ++d) dxi[x][d] = metric<DIM, NP>(mesh, e, node)[x * DIM + d];
   }
   // stage operator tables
   if constexpr (VOL == VOL_SPLIT) {
@@ -527,6 +564,65 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
     // barrier, which every thread passes after its reads of that buffer.
     constexpr int NPAIR = NP / 2;
     const double* const s2pl = sm.Q;   // 2 S by circulant distance, [d][dd][i]
+    if constexpr (ES) {
+      // the face integral's threads share out all pairs (node a and distance
+      // dd as slot (dd - 1) NP + a), whose contributions the nodes then add in
+      // the rounds' order: one barrier, and half the time of the rounds
+      T* const ppl = &sm.Zn[0][0][0][0];   // planes [c][element][slot]
+      constexpr int PAIRS = NPAIR * NP;
+      if (present) {
+        for (int t = i; t < PAIRS; t += TPE) {
+          const int dd = t / NP + 1, a = t - (dd - 1) * NP;
+          T g[ND];
+#pragma unroll
+          for (int k = 0; k < ND; ++k) g[k] = 0.0;
+          if (!(2 * dd == NP && a >= NP / 2)) {
+            int kk = a + dd;
+            if (kk >= NP) kk -= NP;
+            double s2[DIM], n[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) s2[d] = s2pl[(d * (NPAIR + 1) + dd) * NP + a];
+#pragma unroll
+            for (int x = 0; x < DIM; ++x) {
+              n[x] = s2[0] * dxi[x][0];
+#pragma unroll
+              for (int d = 1; d < DIM; ++d) n[x] = n[x] + s2[d] * dxi[x][d];
+            }
+            if (mesh.metric_per_node) {
+              const double* mk = metric<DIM, NP>(mesh, e, a > kk ? a : kk);
+#pragma unroll
+              for (int x = 0; x < DIM; ++x) {
+                n[x] = s2[0] * mk[x * DIM];
+#pragma unroll
+                for (int d = 1; d < DIM; ++d) n[x] = n[x] + s2[d] * mk[x * DIM + d];
+              }
+            }
+            T za[ND], zR[ND];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) {
+              za[k] = zpl[k * PL + me + a];
+              zR[k] = zpl[k * PL + me + kk];
+            }
+            ir_flux_z<DIM, 1>(phys, za, zR, n, g);
+          }
+#pragma unroll
+          for (int k = 0; k < ND; ++k) ppl[(k * EPB + el) * PAIRS + t] = g[k];
+        }
+      }
+      __syncthreads();
+      if (active) {
+        for (int dd = 1; dd <= NPAIR; ++dd) {
+          const int src = i < dd ? i - dd + NP : i - dd;
+#pragma unroll
+          for (int k = 0; k < ND; ++k) {
+            const T* const p = ppl + (k * EPB + el) * PAIRS + (dd - 1) * NP;
+            ri[k] = ri[k] - p[i];
+            ri[k] = ri[k] + p[src];
+          }
+        }
+      }
+      __syncthreads();   // the face integral stages the neighbours over the pairs
+    } else
     for (int dd = 1; dd <= NPAIR; ++dd) {
       const bool half = (2 * dd == NP);            // even NP: distance NP/2 owned by i < NP/2
       T* const cbuf = &sm.C[dd & 1][0][0];
@@ -666,30 +762,24 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
       to_ir_vars<DIM>(phys, qi, w);
 #pragma unroll
       for (int c = 0; c < ND; ++c) sm.W[el][i][c] = w[c];
-      for (int t = i; t < NFACES * ST; t += NP) {
-        const int f = t / ST, sn = t - f * ST;
-        const ElFace rec = mesh.elface[e * NFACES + f];
-        if (rec.x < 0) continue;
-        const int nodeN = sm.perm[sn][rec.z & 0xff];
-        T qn[ND], zn[ND], wn[ND];
+    }
+    if (rece.x >= 0) {
+      T zn[ND], wn[ND];
+      ir_zvars<DIM>(phys, qe, zn);
+      to_ir_vars<DIM>(phys, qe, wn);
 #pragma unroll
-        for (int c = 0; c < ND; ++c) qn[c] = Io<T>::load(qin, vin, ((int64_t)rec.x * NP + nodeN) * ND + c);
-        ir_zvars<DIM>(phys, qn, zn);
-        to_ir_vars<DIM>(phys, qn, wn);
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          sm.Zn[el][f][sn][c] = zn[c];
-          sm.Wn[el][f][sn][c] = wn[c];
-        }
+      for (int c = 0; c < ND; ++c) {
+        sm.Zn[el][i / ST][i % ST][c] = zn[c];
+        sm.Wn[el][i / ST][i % ST][c] = wn[c];
       }
     }
     __syncthreads();
-    if (active) {
+    if (present) {
       // boundary faces: BC flux at the face nodes; interior faces: the
       // entropy penalty (calcEntropyPenaltyIntegral :199-290) at face node k
-      for (int slot = i; slot < NFACES * NF; slot += NP) {
-        const int f = slot / NF;
-        const int k = slot - f * NF;
+      if (i < NFACES * NF) {
+        const int f = i / NF;
+        const int k = i - f * NF;
         const ElFace rec = mesh.elface[e * NFACES + f];
         T Fk[ND];
         int m = k;
@@ -750,9 +840,9 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
       // t of this element on face f against every stencil node of the
       // neighbour, E_ij^d = sum_k R[i][k] R[j][kR] B[k] n_d[k], IR flux in
       // the x, y (, z) directions
-      for (int tt = i; tt < NFACES * ST; tt += NP) {
-        const int f = tt / ST, t = tt - f * ST;
-        const ElFace rec = mesh.elface[e * NFACES + f];
+      {
+        const int f = i / ST, t = i - f * ST;
+        const ElFace rec = rece;
         T h[ND];
 #pragma unroll
         for (int c = 0; c < ND; ++c) h[c] = 0.0;

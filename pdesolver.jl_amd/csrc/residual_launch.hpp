@@ -1,11 +1,10 @@
 // residual_launch.hpp -- launch-variant interface of the fused residual kernel.
 //
 // Tunable launch variants of the FP64 value kernel (the directional-derivative
-// kernel always takes 128 threads, 64 for entropy-stable face integrals, 2 waves):
+// kernel always takes 128 threads, or 256, and 2 waves):
 //   0: large blocks, 3 waves per SIMD      1: large blocks, 4 waves per SIMD
 //   2: small blocks, 3 waves per SIMD      3: small blocks, 4 waves per SIMD
-// (whole elements in 256 and 128 threads; dense-face weak form 192 and 64;
-// entropy-stable face integrals 128 and 64)
+// (whole elements in 256 and 128 threads; dense-face weak form 192 and 64)
 //   4-7: the weak form only: variants 0-3 with the volume term Q^T F on the
 //        FP64 matrix cores (blocks rounded up to whole waves); the split form
 //        runs variant (v & 3) for these

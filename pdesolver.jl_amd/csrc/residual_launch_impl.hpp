@@ -11,7 +11,7 @@ static int launch_cfg(pdes_ctx* c, const double* q, const double* v, double* res
                       const RKStage* rk) {
   // the matrix-core variants run whole waves (the extra lanes only stage
   // tables and join the matrix products)
-  const int threads = MF ? (int)ceil_div(EPB * Op::NP, 64) * 64 : EPB * Op::NP;
+  const int threads = MF ? (int)ceil_div(EPB * Op::NP, 64) * 64 : EPB * threads_per_element<Op, FLUX>();
   if (c->active_count() == 0) return PDES_OK;
   const int blocks = (int)ceil_div(c->active_count(), EPB);
   if constexpr (std::is_same<T, double>::value) {
@@ -31,16 +31,17 @@ static int launch_cfg(pdes_ctx* c, const double* q, const double* v, double* res
 template <class Op, int VOL, int FLUX, class T>
 static int launch_one(pdes_ctx* c, const double* q, const double* v, double* res, double* jv, int32_t* flag,
                       const RKStage* rk, int variant) {
-  // threads per block.  The entropy-stable face integral stages the neighbours'
-  // stencil data in LDS: half the elements per block.  Dense-face weak form:
-  // three waves where blocks are many (3D p=2, 48,000 tets: 256 threads 63.5 us,
+  // threads per block.  Dense-face weak form: three waves where blocks are many (3D p=2, 48,000 tets: 256 threads 63.5 us,
   // 192 57.7, 128 66.2, 64 67.3; what fits a CU's LDS counts), one where they
   // are few (2D p=1, 800 triangles: 256 7.0 us, 128 6.2, 64 5.7).
   constexpr bool DENSE_WEAK = VOL == VOL_WEAK && !Op::DIAGE;
-  constexpr int FULL = (FLUX == PDES_FLUX_ESLF ? 128 : DENSE_WEAK ? 192 : 256) / Op::NP;
-  constexpr int HALF = (FLUX == PDES_FLUX_ESLF || DENSE_WEAK ? 64 : 128) / Op::NP;
+  constexpr int TPE = threads_per_element<Op, FLUX>();
+  constexpr int FULL = (DENSE_WEAK ? 192 : 256) / TPE;
+  constexpr int HALF = (DENSE_WEAK ? 64 : 128) / TPE;
   if constexpr (!std::is_same<T, double>::value) {
-    constexpr int EPB = (FLUX == PDES_FLUX_ESLF ? 64 : 128) / Op::NP;
+    // (derivatives, entropy-stable: 2D p=2, 7,442 triangles 128 threads 43 us,
+    // 256 51; 3D p=2, 3,072 tets 123 and 57; 2D p=4, 3,200 triangles 69 and 64)
+    constexpr int EPB = (FLUX == PDES_FLUX_ESLF && Op::ST >= 10 ? 256 : 128) / TPE;
     return launch_cfg<Op, VOL, FLUX, T, EPB, 2>(c, q, v, res, jv, flag, nullptr);
   } else {
     if constexpr (VOL == VOL_WEAK) {
