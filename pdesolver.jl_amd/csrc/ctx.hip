@@ -30,7 +30,11 @@ int sync_check_flag(pdes_ctx* c) {
   int32_t f = 0;
   PDES_HIP(hipMemcpyAsync(&f, c->d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
   PDES_HIP(hipStreamSynchronize(c->stream));
-  if (f) {
+  return check_flag(c, f);
+}
+
+int check_flag(pdes_ctx* c, int32_t flag) {
+  if (flag) {
     PDES_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int32_t), c->stream));
     set_error("non-positive density or pressure in the state (checkDensity/checkPressure)");
     return PDES_ERR_PHYS;
@@ -268,7 +272,6 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
   if (!st) st = upload(&c->d_nrm_face, m->nrm_face, nI * Nf * dim, sm);
   if (!st) st = upload(&c->d_nrm_bndry, m->nrm_bndry, nB * Nf * dim, sm);
   if (!st) st = upload(&c->d_coords_bndry, m->coords_bndry, nB * Nf * dim, sm);
-  if (!st) st = upload(&c->d_Q, s->Q, (size_t)dim * Np * Np, sm);
   {
     // 2 S_d[a][a + dd mod Np] = Q_d[a][b] - Q_d[b][a] for dd = 0..Np/2, the
     // order in which the split-form pair rounds read it
@@ -280,14 +283,32 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
           const int b = (a + dd) % Np;
           s2c[((size_t)d * ns + dd) * Np + a] = s->Q[((size_t)d * Np + a) * Np + b] - s->Q[((size_t)d * Np + b) * Np + a];
         }
-    if (!st) st = upload(&c->d_S2c, s2c.data(), s2c.size(), sm);
+    // the operator's tables, the norm's ticket (0) and its partial sums share
+    // one allocation and one copy
+    std::vector<unsigned char> tab;
+    std::vector<std::pair<void**, size_t>> at;
+    auto add = [&](auto** dst, const auto* src, size_t n) {
+      at.push_back({(void**)dst, tab.size()});
+      const unsigned char* bytes = (const unsigned char*)src;
+      tab.insert(tab.end(), bytes, bytes + n * sizeof(*src));
+      tab.resize((tab.size() + 15) / 16 * 16, 0);
+    };
+    const unsigned ticket = 0;
+    add(&c->d_Q, s->Q, (size_t)dim * Np * Np);
+    add(&c->d_S2c, s2c.data(), s2c.size());
+    add(&c->d_interp, s->interp, (size_t)s->stencil * Nf);
+    add(&c->d_wface, s->wface, (size_t)Nf);
+    add(&c->d_perm, s->perm, (size_t)s->stencil * nfaces);
+    add(&c->d_nbrperm, s->nbrperm, (size_t)Nf * s->norient);
+    add(&c->d_nodepos, c->h_nodepos.data(), c->h_nodepos.size());
+    add(&c->d_ticket, &ticket, 1);
+    at.push_back({(void**)&c->d_partial, tab.size()});
+    tab.resize(tab.size() + 4096 * sizeof(double), 0);
+    if (!st) st = upload(&c->d_tables, tab.data(), tab.size(), sm);
     if (!st) st = (hipStreamSynchronize(sm) == hipSuccess) ? PDES_OK : PDES_ERR_HIP;
+    if (!st)
+      for (auto& [dst, off] : at) *dst = c->d_tables + off;
   }
-  if (!st) st = upload(&c->d_interp, s->interp, (size_t)s->stencil * Nf, sm);
-  if (!st) st = upload(&c->d_perm, s->perm, (size_t)s->stencil * nfaces, sm);
-  if (!st) st = upload(&c->d_nbrperm, s->nbrperm, (size_t)Nf * s->norient, sm);
-  if (!st) st = upload(&c->d_nodepos, c->h_nodepos.data(), c->h_nodepos.size(), sm);
-  if (!st) st = upload(&c->d_wface, s->wface, (size_t)Nf, sm);
   if (!st) st = upload(&c->d_Minv, Minv.data(), Minv.size(), sm);
   if (!st) st = upload(&c->d_Minv_node, Minv_node.data(), Minv_node.size(), sm);
   if (!st) st = upload(&c->d_ptc_diag, ptc.data(), ptc.size(), sm);
@@ -296,9 +317,8 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
   if (!st) st = upload<double>(&c->d_res, nullptr, (size_t)c->numDof, sm);
   if (!st) st = upload<double>(&c->d_work, nullptr, (size_t)c->numDof, sm);
   if (!st) st = upload<double>(&c->d_work2, nullptr, (size_t)c->numDof, sm);
-  if (!st) st = upload<double>(&c->d_partial, nullptr, 4096, sm);
-  if (!st) st = upload<double>(&c->d_scalar, nullptr, 64, sm);
   if (!st) st = upload<int32_t>(&c->d_flag, nullptr, 1, sm);
+  if (!st && hipHostMalloc((void**)&c->h_norm, sizeof(*c->h_norm)) != hipSuccess) st = PDES_ERR_NOMEM;
   if (!st && hipMemsetAsync(c->d_flag, 0, sizeof(int32_t), sm) != hipSuccess) st = PDES_ERR_HIP;
   if (!st) st = upload<double>(&c->d_qbc, nullptr, std::max<size_t>(1, nB * Nf * c->nd), sm);
   if (!st) st = bc_state_setup(c);
@@ -331,7 +351,7 @@ int pdes_estimate_bytes(const pdes_mesh_desc* m, const pdes_sbp_desc* s, int fp6
   b += (dim * Np * Np + s->stencil * Nf + Nf) * 8 + (s->stencil * nfaces + Nf * s->norient + Np * nfaces) * 4;
   b += ndof * 8 * 5 + nel * Np * 8;                    // Minv (per DOF and per node), q, res, two work vectors
   b += nel * Np * 8;                                   // implicit-Euler diagonal
-  b += (4096 + 64 + 8) * 8;                            // reduction scratch, scalars, flags
+  b += (4096 + 8) * 8;                                 // reduction scratch, flag and ticket
   // BSR Jacobian: element blocks plus the face couplings of every interface
   const int64_t cpl = s->diag_e ? Nf : (int64_t)s->stencil * s->stencil;
   const int64_t nnzb = nel * Np * Np + 2 * nI * cpl;
@@ -358,13 +378,13 @@ int pdes_ctx_destroy(pdes_ctx* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   jacobian_free(c);
   precond_free(c);
-  void* ptrs[] = {c->d_dxidx, c->d_elface, c->d_slot, c->d_nrm_face, c->d_nrm_bndry, c->d_coords_bndry, c->d_Q, c->d_S2c,
-                  c->d_interp, c->d_perm, c->d_nbrperm, c->d_nodepos, c->d_wface, c->d_Minv, c->d_Minv_node, c->d_q,
-                  c->d_res, c->d_work, c->d_work2, c->d_partial, c->d_scalar, c->d_flag,
+  void* ptrs[] = {c->d_dxidx, c->d_elface, c->d_slot, c->d_nrm_face, c->d_nrm_bndry, c->d_coords_bndry, c->d_tables,
+                  c->d_Minv, c->d_Minv_node, c->d_q, c->d_res, c->d_work, c->d_work2, c->d_flag,
                   c->d_el_list, c->d_el_inst, c->d_inst_phys, c->d_ptc_diag, c->d_ptc_scale,
                   c->d_inst_active, c->d_qbc, c->d_w};
   for (void* p : ptrs)
     if (p) hipFree(p);
+  if (c->h_norm) hipHostFree(c->h_norm);
   if (c->own_stream && c->stream) hipStreamDestroy(c->stream);
   delete c;
   return PDES_OK;

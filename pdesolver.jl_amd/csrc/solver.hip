@@ -2204,15 +2204,8 @@ int pdes_newton_solve(pdes_ctx* c, const pdes_newton_opts* o, pdes_newton_report
     if (!s2 && c->hom_lambda >= 0.0)
       s2 = launch_homotopy(c, c->d_q, nullptr, 1.0 - c->hom_lambda, c->hom_lambda, res, nullptr);
     if (s2) return s2;
-    s2 = launch_wnorm2(c, res, c->d_Minv, n, c->d_scalar);
-    if (s2) return s2;
-    double v = 0;
-    PDES_HIP(hipMemcpyAsync(&v, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    PDES_HIP(hipStreamSynchronize(c->stream));
-    s2 = sync_check_flag(c);
-    if (s2) return s2;
-    *out = std::sqrt(v);
-    return PDES_OK;
+    s2 = launch_wnorm2(c, res, c->d_Minv, n, 0);
+    return s2 ? s2 : wait_norm(c, out);
   };
   double nrm = 0, tau = 0, prev_nrm = 0;
   if ((st = norm_res(&nrm)) != 0) goto fin;
@@ -2244,11 +2237,9 @@ int pdes_newton_solve(pdes_ctx* c, const pdes_newton_opts* o, pdes_newton_report
     rep->total_krylov_iters += kits;
     hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n)), dim3(256), 0, c->stream, dq, c->d_q, 1.0, 1, n);
     // step norm: norm(delta_q_vec)
-    if ((st = launch_wnorm2(c, dq, nullptr, n, c->d_scalar + 1)) != 0) goto fin;
-    double sn2 = 0;
-    PDES_HIP(hipMemcpyAsync(&sn2, c->d_scalar + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    if ((st = launch_wnorm2(c, dq, nullptr, n, 1)) != 0) goto fin;
     if ((st = norm_res(&nrm)) != 0) goto fin;
-    rep->step_norm = std::sqrt(sn2);
+    rep->step_norm = std::sqrt(c->h_norm->sum[1]);
     rep->res_norm = nrm;
     rep->iterations = it;
     // checkConvergence (newton.jl:402-455)
@@ -2305,14 +2296,8 @@ int pdes_homotopy_solve(pdes_ctx* c, const pdes_newton_opts* o, double psi_max, 
   auto phys_norm = [&](double* out) -> int {
     c->hom_lambda = -1.0;
     int s2 = launch_residual(c, c->d_q, nullptr, c->d_res, nullptr, c->phys.check_positivity != 0);
-    if (!s2) s2 = launch_wnorm2(c, c->d_res, c->d_Minv, n, c->d_scalar);
-    if (s2) return s2;
-    double v = 0;
-    PDES_HIP(hipMemcpyAsync(&v, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    PDES_HIP(hipStreamSynchronize(c->stream));
-    if ((s2 = sync_check_flag(c))) return s2;
-    *out = std::sqrt(v);
-    return PDES_OK;
+    if (!s2) s2 = launch_wnorm2(c, c->d_res, c->d_Minv, n, 0);
+    return s2 ? s2 : wait_norm(c, out);
   };
   // calcNorm (Utils.jl:427-449) and calcL2InnerProduct (:476-493): M-weighted
   auto mdot = [&](const std::vector<double>& a, const std::vector<double>& b) {

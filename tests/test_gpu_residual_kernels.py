@@ -46,3 +46,30 @@ def test_dense_face_residual_at_block_edges(oracle, kind, p, flux):
         jv = oracle.jv_complex_step(b, q, v)
         assert np.abs(euler.evaldRdqProduct(eqn, v) - jv).max() <= 1e-12 * np.abs(jv).max()
         eqn.free()
+
+
+@pytest.mark.parametrize("n,p", [(1, 1), (4, 1), (5, 2), (90, 2)])
+def test_residual_norm_of_one_and_many_blocks(n, p):
+    """calcNorm over 1, 2, 10 and 1,024 reduction blocks (several entries per
+    thread in the last), repeated: the same bits each time, and numpy's sum of
+    N positive terms to N rounding errors; a state with a negative density
+    fails once and not after the state is mended."""
+    m, op, ph = problems.make_problem("vortex", n, p, "omega" if p == 1 else "diage", "roe")
+    q = problems.vortex_noise_state(m, ph, seed=2)
+    eqn = euler.EulerData(m, op, ph)
+    eqn.set_q(q)
+    euler.evalResidual(m, op, eqn)
+    ref = np.sqrt((eqn.res ** 2 * eqn.Minv).sum())
+    got = [euler.calcNorm(eqn) for _ in range(4)]
+    assert len(set(got)) == 1
+    assert abs(got[0] - ref) <= q.size * 2.0 ** -53 * ref
+    bad = q.copy()
+    bad[-1, 0, 0] = -1.0
+    eqn.set_q(bad)
+    euler.evalResidual_device(eqn)
+    with pytest.raises(Exception):
+        euler.calcNorm(eqn)
+    eqn.set_q(q)
+    euler.evalResidual_device(eqn)
+    assert euler.calcNorm(eqn) == got[0]
+    eqn.free()
