@@ -708,7 +708,12 @@ euler_jacobian_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys, const double* __
 
 // y = J x (BSR, block rows of ndof, FP32 or FP64 blocks, FP64 vectors):
 // one thread per output dof; the threads of a block row read the block
-// rows [a][0..ND) in turn.
+// rows [a][0..ND) in turn, four of them (FP64: two) in flight, with the column
+// numbers a round ahead.  Bound by memory where rows are many, by the latency of
+// a round where they are few.  One block at a time, its column, then x: 101.8 us
+// for 3D p=2, 6,000 tets, 276 MB of blocks, now 80.1 us (3.5 TB/s; six blocks
+// 81.2, eight 85.6); 800 triangles p=1 8.4 -> 5.8 us; FP64, 882 triangles p=2
+// 13.0 -> 8.7 us (four blocks 12.4).
 template <int ND, class BT>
 __global__ void __launch_bounds__(256)
 bsr_spmv_kernel(int64_t nrows, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
@@ -727,11 +732,32 @@ bsr_spmv_kernel(int64_t nrows, const int64_t* __restrict__ rowptr, const int32_t
   const int64_t t = row * ND + a;
   double acc = 0.0;
   const int64_t b0 = rowptr[row], b1 = rowptr[row + 1];
-  for (int64_t b = b0; b < b1; ++b) {
-    const BT* blk = vals + b * (ND * ND) + a * ND;
-    const double* xc = x + (int64_t)colind[b] * ND;
+  constexpr int U = sizeof(BT) == 8 ? 2 : 4;
+  if (b0 < b1) {
+    int32_t col[U];
 #pragma unroll
-    for (int c = 0; c < ND; ++c) acc += (double)blk[c] * xc[c];
+    for (int u = 0; u < U; ++u) col[u] = colind[b0 + u < b1 ? b0 + u : b1 - 1];
+    for (int64_t b = b0; b < b1; b += U) {
+      BT m[U][ND];
+      double xc[U][ND];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t p = b + u < b1 ? b + u : b1 - 1;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+          m[u][c] = vals[p * (ND * ND) + a * ND + c];
+          xc[u][c] = x[(int64_t)col[u] * ND + c];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) col[u] = colind[b + U + u < b1 ? b + U + u : b1 - 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (b + u < b1) {
+#pragma unroll
+          for (int c = 0; c < ND; ++c) acc += (double)m[u][c] * xc[u][c];
+        }
+    }
   }
   double v = alpha * acc;
   if (yadd) v += beta * yadd[t];

@@ -90,6 +90,31 @@ def test_block_inverses(kind, p, opk, flux):
     e.free()
 
 
+@pytest.mark.parametrize("fp64", [False, True])
+@pytest.mark.parametrize("kind,p,opk,flux", SHAPES)
+def test_block_row_products(kind, p, opk, flux, fp64):
+    """J x over rows of 3 to 60 blocks, some a multiple of the blocks in flight
+    and some not, is numpy's sum of the same products to n rounding errors."""
+    print(f"case {kind} p={p} {opk} {flux} fp64={fp64}", flush=True)
+    m, op, ph, q = _problem(kind, 1 if kind == "cube" else 2, p, opk, flux, shuffle=True)
+    e = euler.EulerData(m, op, ph)
+    e.set_q(q)
+    lo = linsolve.HIPBSRLO(e, fp64_blocks=fp64)
+    lo.calcLinearOperator()
+    rowptr, colind = linsolve.getSparsityPattern(e, fp64_blocks=fp64)
+    vals = linsolve.getJacobianValues(e, fp64_blocks=fp64).astype(np.float64)
+    x = np.random.default_rng(6).standard_normal(q.shape)
+    y = np.zeros_like(x)
+    lo.applyLinearOperator(m, op, e, None, None, 0.0, x, y)
+    nd = q.shape[2]
+    xb, yb = x.reshape(-1, nd), y.reshape(-1, nd)
+    for r in range(len(rowptr) - 1):
+        blk, xc = vals[rowptr[r]:rowptr[r + 1]], xb[colind[rowptr[r]:rowptr[r + 1]]]
+        ref, mag = np.einsum("bij,bj->i", blk, xc), np.einsum("bij,bj->i", np.abs(blk), np.abs(xc))
+        assert np.all(np.abs(yb[r] - ref) <= 2 * nd * len(blk) * 2.0 ** -53 * mag)
+    e.free()
+
+
 @pytest.mark.parametrize("restart", [1, 2, 7, 8, 9, 16, 17, 33, 70])
 def test_gmres_cycle_is_the_least_squares_solution(restart):
     """One restart cycle of k steps reaches the least residual over
