@@ -1381,11 +1381,11 @@ static int ilu_factor(pdes_ctx* c) {
     const int32_t* lev = p->d_fel + p->fptr[l];
     if (j->fp64)
       hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, DIAGE, double>), dim3((unsigned)cnt), block, 0, c->stream,
-                         lev, j->d_rowptr, j->d_colind, p->d_own, (const double*)j->d_vals, c->d_elface, c->nfaces,
+                         lev, j->d_rowptr, j->d_colind, p->d_own, (const double*)j->d_vals, c->d_elface,
                          c->d_perm, c->d_nodepos, p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
     else
       hipLaunchKernelGGL((ilu_factor_level_kernel<NP, ND, NS, DIAGE, float>), dim3((unsigned)cnt), block, 0, c->stream,
-                         lev, j->d_rowptr, j->d_colind, p->d_own, (const float*)j->d_vals, c->d_elface, c->nfaces,
+                         lev, j->d_rowptr, j->d_colind, p->d_own, (const float*)j->d_vals, c->d_elface,
                          c->d_perm, c->d_nodepos, p->d_inv, j->d_err, c->d_el_inst, c->d_inst_active);
   }
   PDES_HIP(hipGetLastError());
