@@ -40,8 +40,10 @@ static int launch_one(pdes_ctx* c, const double* q, const double* v, double* res
   constexpr int HALF = (DENSE_WEAK ? 64 : 128) / TPE;
   if constexpr (!std::is_same<T, double>::value) {
     // (derivatives, entropy-stable: 2D p=2, 7,442 triangles 128 threads 43 us,
-    // 256 51; 3D p=2, 3,072 tets 123 and 57; 2D p=4, 3,200 triangles 69 and 64)
-    constexpr int EPB = (FLUX == PDES_FLUX_ESLF && Op::ST >= 10 ? 256 : 128) / TPE;
+    // 256 51; 3D p=2, 3,072 tets 123 and 57; 2D p=4, 3,200 triangles 69 and 64;
+    // weak form, 3D p=1, 10,368 tets 128 threads 22.8 us, 64 17.8; p=2 55.5 and 57.9)
+    constexpr int EPB =
+        (FLUX == PDES_FLUX_ESLF && Op::ST >= 10 ? 256 : DENSE_WEAK && Op::NP == Op::NFACES ? 64 : 128) / TPE;
     return launch_cfg<Op, VOL, FLUX, T, EPB, 2>(c, q, v, res, jv, flag, nullptr);
   } else {
     if constexpr (VOL == VOL_WEAK) {
