@@ -160,23 +160,44 @@ __device__ __forceinline__ void ir_zvars(const PhysConst& p, const T* q, T* z) {
   z[DIM + 1] = dsqrt(q[0] * pr);
 }
 
-// The series/log factor of logavg for aL, aR with r = 1/(aL + aR):
-// logavg = (aL + aR) / (2 F) and 1/logavg = 2 F r (bc_solvers.jl:942-956,
-// same branch test on u = f^2).
-// When logs of both arguments are at hand (lgL, lgR, e.g. staged per node),
-// log(aL/aR) is taken as lgL - lgR (the branch is only taken for
-// |f| >= 0.0316, where the difference loses no accuracy that matters).
-template <class T, class TR, class LP>
-__device__ __forceinline__ T logavg_factor(const T& aL, const TR& aR, const T& r, LP lgL, LP lgR) {
-  const T f = (aL - aR) * r;
-  const T u = f * f;
-  if (re(u) < 1e-3) {
-    // 1 + u/3 + u^2/5 + u^3/7 + u^4/9, evaluated as (1 + u/3) + u^2 ((1/5 + u/7) + u^2/9)
+// The series/log factors of logavg for the first and last IR variables of two
+// states, with r = 1/(aL + aR): logavg = (aL + aR) / (2 F) and 1/logavg = 2 F r
+// (bc_solvers.jl:942-956, same branch test on u = f^2).  UNIFORM: the series is
+// evaluated for all lanes and the logs only when a lane of the wave needs one,
+// one wave-uniform branch for both factors; for the pair rounds and faces of the
+// diagonal-E values (RK4 steps of 131,072 triangles, p=4: 5448 -> 5250 us; a
+// residual of states 10% and more apart, which need the logs, 515 -> 492 us).
+// Elsewhere a branch per factor: the logs, live together with both series, spill
+// (entropy-stable p=2, 45,000 triangles 121 us instead of 62; derivative of 7,442
+// triangles 38.5 us instead of 20.4).
+template <bool UNIFORM, class T, class TR>
+__device__ __forceinline__ void logavg_factors(const T& aL0, const TR& aR0, const T& r0, const T& aL3, const TR& aR3,
+                                               const T& r3, T& F0, T& F3) {
+  // 1 + u/3 + u^2/5 + u^3/7 + u^4/9, evaluated as (1 + u/3) + u^2 ((1/5 + u/7) + u^2/9)
+  auto series = [](const T& u) {
     const T u2 = u * u;
     return (1.0 + u * (1.0 / 3.0)) + u2 * ((1.0 / 5.0 + u * (1.0 / 7.0)) + u2 * (1.0 / 9.0));
+  };
+  if constexpr (UNIFORM) {
+    const T f0 = (aL0 - aR0) * r0, f3 = (aL3 - aR3) * r3;
+    const T u0 = f0 * f0, u3 = f3 * f3;
+    F0 = series(u0);
+    F3 = series(u3);
+    const bool log0 = !(re(u0) < 1e-3), log3 = !(re(u3) < 1e-3);
+    if (__any(log0 || log3)) {
+      if (log0) F0 = dlog(aL0 / aR0) * (0.5 * drcp(f0));
+      if (log3) F3 = dlog(aL3 / aR3) * (0.5 * drcp(f3));
+    }
+  } else {
+    auto factor = [&](const T& aL, const TR& aR, const T& r) {
+      const T f = (aL - aR) * r;
+      const T u = f * f;
+      if (re(u) < 1e-3) return series(u);
+      return T(dlog(aL / aR) * (0.5 * drcp(f)));
+    };
+    F0 = factor(aL0, aR0, r0);
+    F3 = factor(aL3, aR3, r3);
   }
-  if constexpr (std::is_same<LP, std::nullptr_t>::value) return dlog(aL / aR) * (0.5 * drcp(f));
-  else return (*lgL - *lgR) * (0.5 * drcp(f));
 }
 
 // calcEulerFlux_IR, multi-direction  bc_solvers.jl:776-805 (2D), 842-874 (3D),
@@ -189,16 +210,13 @@ __device__ __forceinline__ T logavg_factor(const T& aL, const TR& aR, const T& r
 //   h_hat = gamma/(gamma-1) p2_hat/rho_hat + |v|^2/2 = 4 gamma/(gamma-1) r0^2 (c1 F0 + c2 F3) + |v|^2/2.
 // r0 and r3 come from one drcp of s0 s3 and 1/F3 from another (Newton-refined
 // hardware estimates).
-// lzL / lzR: optional logs {log z1, log z4} of the two states (pointers to
-// log z1, with log z4 LS elements further; read only on the log branch of
-// logavg), or nullptr.  dl: optional output {log(zL1/zR1), log(zL4/zR4)},
+// dl: optional output {log(zL1/zR1), log(zL4/zR4)},
 // which the logavg factors give without a log: log(aL/aR) = 2 F f.
 // TR: the right state's type, T or, for derivatives with respect to the left
 // state only, double.
-template <int DIM, int NDIR, class T, class LP = std::nullptr_t, int LS = 1, class TN = double, class TR = T>
+template <int DIM, int NDIR, bool UNIFORM = false, class T, class TN = double, class TR = T>
 __device__ __forceinline__ void ir_flux_z(const PhysConst& p, const T* zL, const TR* zR,
-                                          const TN* dir, T* F, LP lzL = nullptr, LP lzR = nullptr,
-                                          T* dl = nullptr) {
+                                          const TN* dir, T* F, T* dl = nullptr) {
   constexpr int ND = DIM + 2;
   const double gamma = p.gamma, gamma_1 = p.gamma_1;
   const T s0 = zL[0] + zR[0];
@@ -208,13 +226,7 @@ __device__ __forceinline__ void ir_flux_z(const PhysConst& p, const T* zL, const
   const T r0 = s3 * t03;
   const T r3 = s0 * t03;
   T F0, F3;
-  if constexpr (std::is_same<LP, std::nullptr_t>::value) {
-    F0 = logavg_factor(zL[0], zR[0], r0, nullptr, nullptr);
-    F3 = logavg_factor(zL[ND - 1], zR[ND - 1], r3, nullptr, nullptr);
-  } else {
-    F0 = logavg_factor(zL[0], zR[0], r0, lzL, lzR);
-    F3 = logavg_factor(zL[ND - 1], zR[ND - 1], r3, lzL + LS, lzR + LS);
-  }
+  logavg_factors<UNIFORM>(zL[0], zR[0], r0, zL[ND - 1], zR[ND - 1], r3, F0, F3);
   if (dl) {
     dl[0] = (2.0 * F0) * ((zL[0] - zR[0]) * r0);
     dl[1] = (2.0 * F3) * ((zL[ND - 1] - zR[ND - 1]) * r3);
@@ -340,7 +352,7 @@ __device__ __forceinline__ void irslf_flux_z(const PhysConst& p, const T* qL, co
   constexpr int ND = DIM + 2;
   const double gamma = p.gamma;
   T dl[2];
-  ir_flux_z<DIM, 1>(p, zL, zR, nrm, F, nullptr, nullptr, dl);
+  ir_flux_z<DIM, 1, std::is_same<T, double>::value>(p, zL, zR, nrm, F, dl);
   T dv[ND], vR[ND];
   to_ir_vars<DIM, T, 2>(p, qL, dv);
   to_ir_vars<DIM, T, 2>(p, qR, vR);

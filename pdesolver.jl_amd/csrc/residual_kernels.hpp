@@ -682,7 +682,7 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
           T zR[ND];
 #pragma unroll
           for (int k = 0; k < ND; ++k) zR[k] = zpl[k * PL + me + kk];
-          ir_flux_z<DIM, 1>(phys, zi, zR, n, g);
+          ir_flux_z<DIM, 1, std::is_same<T, double>::value>(phys, zi, zR, n, g);
           // res_i -= 2 S[i][kk] F, and the partner gets -2 S[kk][i] F = +g
 #pragma unroll
           for (int k = 0; k < ND; ++k) ri[k] = ri[k] - g[k];
