@@ -73,3 +73,24 @@ def test_residual_norm_of_one_and_many_blocks(n, p):
     euler.evalResidual_device(eqn)
     assert euler.calcNorm(eqn) == got[0]
     eqn.free()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3, 4])
+@pytest.mark.parametrize("where", ["one node", "everywhere"])
+def test_split_form_where_logarithms_are_needed(oracle, p, where):
+    """Diagonal-E split form with states so far apart (density times 1 to 2) that
+    the logarithmic means leave their series: at one node, so that one lane of a
+    wave needs the logarithm, and everywhere; the oracle's values to 1e-12."""
+    m, op, ph = problems.make_problem("vortex", 5, p, "diage", "ir")
+    b = abi.make_descriptors(m, op, ph)
+    q = state_for("vortex", m, ph)
+    f = 1.0 + np.random.default_rng(p).uniform(0.0, 1.0, q.shape[:2] + (1,))
+    if where == "one node":
+        q[3, 1] *= 2.0
+    else:
+        q = q * f
+    eqn = euler.EulerData(m, op, ph)
+    eqn.set_q(q)
+    euler.evalResidual(m, op, eqn)
+    assert_parity(eqn.res, oracle.residual(b, q), oracle.residual_scale(b, q), 1e-12, f"p {p} {where}")
+    eqn.free()
