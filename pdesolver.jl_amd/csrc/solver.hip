@@ -353,6 +353,19 @@ bjacobi_factor_kernel(const int32_t* __restrict__ el_list, const int64_t* __rest
   __syncthreads();
   float a[GjShape<N>::R][GjShape<N>::R];
   load_own_block<NP, ND>(vals, run, a);
+  // The entries are values from here on, not loads whose addresses the unrolled
+  // pivots may still hold: without this the kernel took 231 registers for 50 and
+  // 60 unknowns (4 x 4 entries a thread) and spilled up to 516 bytes a lane for 72
+  // (5 x 5), now 37 to 59.  Set-up, FP32 blocks, 32,768 triangles: Omega p=4 3256
+  // -> 1106 us, diagonal-E p=3 10,400 -> 1890 us (FP64 blocks 16,190 -> 1938);
+  // 16,464 tets p=2 1389 -> 512 us.  The other sizes take 22 to 85 registers
+  // without it, and 108 unknowns 7% longer with it.
+  if constexpr (GjShape<N>::R == 4 || GjShape<N>::R == 5) {
+#pragma unroll
+    for (auto& row : a)
+#pragma unroll
+      for (float& x : row) asm volatile("" : "+v"(x));
+  }
   gauss_jordan_inverse<N>(a, sh, inv + e * InvLayout<N>::SIZE, err);
 }
 

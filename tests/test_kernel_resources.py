@@ -13,7 +13,7 @@ msgpack = pytest.importorskip("msgpack")
 PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pdesolver.jl_amd")
 LIB = os.path.join(PKG, "pdes_amd", "libpdes_amd.so")
 # registers of a lane at which n waves fit a SIMD (512 registers, in steps of 8)
-REGS_AT_WAVES = {3: 168}
+REGS_AT_WAVES = {3: 168, 4: 128}
 
 
 def _code_objects(data):
@@ -77,4 +77,12 @@ def test_diage_weak_form_derivatives_run_three_waves(kernels):
     found = _matching(kernels, r"euler_residual_kernelINS_7OpShapeILi2ELi\d+ELi\d+ELi\d+ELb1EEELi1E.*dualILi1E", 4)
     _no_spills(found)
     assert all(k[".vgpr_count"] <= REGS_AT_WAVES[3] for k in found.values()), \
+        {n: k[".vgpr_count"] for n, k in found.items()}
+
+
+def test_block_jacobi_factorizations_run_four_waves(kernels):
+    """Ten operators, FP32 and FP64 blocks."""
+    found = _matching(kernels, r"bjacobi_factor_kernel", 20)
+    _no_spills(found)
+    assert all(k[".vgpr_count"] <= REGS_AT_WAVES[4] for k in found.values()), \
         {n: k[".vgpr_count"] for n, k in found.items()}
