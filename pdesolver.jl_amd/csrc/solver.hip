@@ -975,11 +975,19 @@ ilu_sweep_dep_kernel(const int32_t* __restrict__ order, const int32_t* __restric
 
   // the computing waves: lane l of row r, elements g, g + G, ... of the set
   const int g = wave / W, gw = wave - g * W;
-  const int l = lane % LPR, first = lane - l;
+  const int lane_l = lane % LPR, first = lane - lane_l;
   const bool has_row = lane / LPR < RW && gw * RW + lane / LPR < N;
-  const int r = has_row ? gw * RW + lane / LPR : N - 1;
-  const int i = r / ND, a = r - i * ND;
+  const int lane_r = has_row ? gw * RW + lane / LPR : N - 1;
   for (int k = g; k < K; k += C::G) {
+    int l = lane_l, r = lane_r;
+    // FP64 blocks of dense faces from 40 rows on: the places that follow from the
+    // lane and the row are formed anew for each element.  Taken out of the loop
+    // they filled the registers that the blocks need: 15 to 36 of a share's values
+    // went to scratch memory, which ended the loading ahead.  Both
+    // triangles, same bits: 8,192 triangles Omega p=3 1037 -> 523 us, p=4 1563 ->
+    // 832 us, 6,000 tets p=2 350 -> 262 us.
+    if constexpr (!DIAGE && sizeof(BT) == 8 && N >= 40) asm volatile("" : "+v"(l), "+v"(r));
+    const int i = r / ND, a = r - i * ND;
     // this lane's share: entries l, l + LPR, ... of its row of D'_e^-1, row a
     // of the neighbour blocks l, l + LPR, ... (a valid block where there is
     // none), the places of their values, the right-hand side

@@ -60,6 +60,33 @@ def test_ilu0_sweeps_agree(monkeypatch, kind, p, opk, flux, shuffle):
 
 
 @pytest.mark.parametrize("kind,p,opk,flux", SHAPES)
+def test_ilu0_sweeps_agree_fp64_blocks(monkeypatch, kind, p, opk, flux):
+    """The same with FP64 blocks: the same bits from both kinds of sweep over
+    sets of one element, of a few and longer than the largest."""
+    for n in (1, 5, 45) if kind == "vortex" else (1, 6):
+        print(f"case {kind} n={n} p={p} {opk} {flux}", flush=True)
+        m, op, ph, q = _problem(kind, n, p, opk, flux)
+        b = np.random.default_rng(13).standard_normal(q.shape)
+        out = []
+        for env in ("PDES_ILU_DEP", "PDES_ILU_LEVELS"):
+            monkeypatch.delenv("PDES_ILU_DEP", raising=False)
+            monkeypatch.setenv(env, "1")
+            e = euler.EulerData(m, op, ph)
+            e.set_q(q)
+            linsolve.evalJacobian(m, op, e, fp64_blocks=True)
+            pc = linsolve.HIPILU0PC(e)
+            pc.calcPC()
+            x = np.zeros_like(b)
+            for _ in range(2):
+                pc.applyPC(m, op, e, None, 0.0, b, x)
+            out.append(x)
+            e.free()
+        monkeypatch.delenv("PDES_ILU_LEVELS")
+        assert np.all(np.isfinite(out[0]))
+        assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("kind,p,opk,flux", SHAPES)
 def test_block_inverses(kind, p, opk, flux):
     """The block-Jacobi apply solves with each element's block to what an FP32
     inverse of N unknowns allows: 8 N eps cond."""

@@ -86,3 +86,9 @@ def test_block_jacobi_factorizations_run_four_waves(kernels):
     _no_spills(found)
     assert all(k[".vgpr_count"] <= REGS_AT_WAVES[4] for k in found.values()), \
         {n: k[".vgpr_count"] for n, k in found.items()}
+
+
+def test_dependency_sweeps_do_not_spill(kernels):
+    """The ILU(0) sweeps of ten operators, FP32 and FP64 blocks: a share of an
+    element that does not stay in registers ends the loading ahead."""
+    _no_spills(_matching(kernels, r"ilu_sweep_dep_kernel", 20))
