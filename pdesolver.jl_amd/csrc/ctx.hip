@@ -62,24 +62,33 @@ int bc_state_setup(pdes_ctx* c) {
 using namespace pdes;
 
 // Default launch variant of the residual (residual_launch.hpp), from times of
-// all variants on MI355X (us):
-//   split form, diagonal-E: 4 waves per SIMD (2D p=1..3, 18,818 to 131,072
-//     triangles: 44.7, 68.6, 24.9 against 46.6, 70.6, 26.2), but 3 for p=4
-//     (232.7; small blocks 258.1);
-//   split form, dense faces: large blocks, 4 waves (2D p=2, 45,000 triangles:
-//     61.7 against 63.0 to 64.5; p=3, 18,818: 66.0 against 67.6 to 70.1), 3D 3
-//     (p=2, 16,464 tets: 94.6 against 109.8);
-//   weak form, up to 512 blocks of 192 threads, and 2D Omega p=1: small blocks,
-//     vector ALUs (800 triangles: Omega p=1 5.9 against 6.5 to 7.5, p=3 7.9
-//     against 8.9, diagonal-E p=2 5.8 against 6.0 to 6.4; 3,072 tets p=2 11.6
-//     against 12.1 to 12.5; 131,072 triangles Omega p=1 20.9 against 22.9);
+// all variants of every shape on meshes of 128 to 32,768 triangles and 162 to
+// 16,464 tets on MI355X (us):
+//   split form: large blocks at 4 waves per SIMD.  Diagonal-E (both bounds give
+//     the same code for p=4): 2D p=1..3 15.5, 22.7, 38.6 and small blocks 15.4 to
+//     15.5, 21.8 to 22.2, 36.0 to 37.1 at 32,768 triangles, but 8.1, 7.8, 9.3
+//     against 9.5, 9.1, 10.8 at 2,048 to 8,192.  Dense faces p=1..3 at 32,768
+//     triangles 23.2, 49.5, 102.9 against 25.4, 49.5, 107.9; but 3 waves for p=4,
+//     which spills with 4 (8,192 triangles 67.6 against 77.7, 32,768 229 against
+//     256), and in 3D (p=2, 16,464 tets: 95.2 against 110.3).
+//   weak form on dense faces, up to 512 blocks of 192 threads, and 2D Omega p=1:
+//     small blocks, vector ALUs (800 triangles: Omega p=1 5.6 against 6.4, p=3 7.9
+//     against 8.9; 6,000 tets p=2 14.9 against 16.6); not for p=4, where the matrix
+//     cores save more (800 triangles 7.8 against 7.7, 4,608 9.8 against 9.0).
+//   weak form on diagonal-E operators, as long as there is a CU for each small
+//     block (128 threads): those (4,608 triangles p=1 6.5 against 6.9, 800 p=3 6.7
+//     against 6.9); with more of them than CUs the large ones win until they
+//     outnumber the CUs too, and from there on it is the same (8,192 triangles p=1
+//     7.8 against 7.0, 2,048 p=3 7.7 against 6.9, p=4 9.5 against 8.6).
 //   weak form beyond: large blocks, with Q^T F on the matrix cores from 10 nodes
-//     an element (Omega p=4 18.1 against 20.7, 3D p=2, 48,000 tets, 57.3 against
-//     60.1, diagonal-E p=2 45.6 against 48.7) and 4 waves, 3 for the 3D Omega
-//     ones (p=1, 48,000 tets: 20.1 against 23.0).
+//     an element (32,768 triangles, Omega p=4 25.7 against 30.7, diagonal-E p=2
+//     15.8 against 17.2; 16,464 tets p=2 28.7 against 29.3) and 4 waves, 3 for the
+//     3D ones (p=2 28.7 against 30.0, p=1 12.3 against 14.6).
 static int default_variant(const pdes_ctx* c) {
-  if (c->phys.volume_integral_type == 2) return (c->diag_e ? c->Np > 18 : c->dim == 3) ? 0 : 1;
-  if ((int64_t)c->numEl * c->Np < 512 * 192 || (c->dim == 2 && c->Np == 3)) return 2;
+  if (c->phys.volume_integral_type == 2) return !c->diag_e && (c->dim == 3 || c->Np == 15) ? 0 : 1;
+  const int64_t nodes = (int64_t)c->numEl * c->Np;
+  const bool small = c->diag_e ? nodes <= 256 * 128 : c->Np != 15 && (nodes < 512 * 192 || (c->dim == 2 && c->Np == 3));
+  if (small) return 2;
   return (c->Np >= 10 ? 4 : 0) + (c->dim == 2 ? 1 : 0);
 }
 
