@@ -1750,6 +1750,11 @@ int pc_setup(pdes_ctx* c, int kind) {
 // wait of the host a step) took 73 us a step at n = 9,600 with the operator
 // and the preconditioner, these take 38.
 constexpr int CGS_MAX_BLOCKS = 512;
+// The coefficients of up to this many basis vectors are summed into LDS by every
+// workgroup; those of longer cycles once, by multidot_reduce, and read from
+// memory (LONG), so that the length of a cycle has no bound but the basis's
+// memory.  Beyond it the pass over the basis takes longer than the extra launch.
+constexpr int CGS_LDS_ROWS = 1024;
 
 static int cgs_blocks(int64_t n) {
   const int64_t full = std::max<int64_t>(1, ceil_div(n, CGS_THREADS));
@@ -1761,7 +1766,7 @@ static int cgs_blocks(int64_t n) {
 // by workgroup 0).  Then pout[i][block] = sum over the block's slice of V_i . w.
 // The first 8 MG basis values of an entry stay in registers for both uses; the
 // basis vectors beyond (m > 32) are read again, 32 at a time.
-template <int MG, bool AXPY>
+template <int MG, bool AXPY, bool LONG>
 __global__ void __launch_bounds__(CGS_THREADS)
 cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ w, int64_t n,
          const double* __restrict__ pin, int nb_in, double* __restrict__ hsave, double* __restrict__ pout) {
@@ -1769,10 +1774,11 @@ cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ 
   extern __shared__ double sh_h[];
   __shared__ double sh_w[CGS_THREADS / 64][NV];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  auto h = [&](int i) { return LONG ? pin[i] : sh_h[i]; };
   if constexpr (AXPY) {
-    sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
+    if constexpr (!LONG) sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
     if (blockIdx.x == 0)
-      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
+      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = h(i);
   }
   const int64_t stride = (int64_t)gridDim.x * CGS_THREADS, t0 = (int64_t)blockIdx.x * CGS_THREADS + tid;
   for (int i0 = 0; i0 < m; i0 += NV) {
@@ -1787,8 +1793,8 @@ cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ 
       if (AXPY && i0 == 0) {
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-          if (i < m) wt -= sh_h[i] * v[i];
-        for (int i = NV; i < m; ++i) wt -= sh_h[i] * V[(int64_t)i * ldv + t];
+          if (i < m) wt -= h(i) * v[i];
+        for (int i = NV; i < m; ++i) wt -= h(i) * V[(int64_t)i * ldv + t];
         w[t] = wt;
       }
 #pragma unroll
@@ -1809,7 +1815,7 @@ cgs_pass(const double* __restrict__ V, int m, int64_t ldv, double* __restrict__ 
 
 // w -= sum_i h_i V_i with h the sums of pin's rows, and the partial sum of w^2
 // (m = 0: w = b - w, the residual of a cycle's start)
-template <int MG>
+template <int MG, bool LONG>
 __global__ void __launch_bounds__(CGS_THREADS)
 cgs_norm(const double* __restrict__ V, int m, int64_t ldv, const double* __restrict__ b, const double* w, double* out,
          int64_t n, const double* __restrict__ pin, int nb_in, double* __restrict__ hsave,
@@ -1817,10 +1823,11 @@ cgs_norm(const double* __restrict__ V, int m, int64_t ldv, const double* __restr
   extern __shared__ double sh_h[];
   __shared__ double sh_w[CGS_THREADS / 64];
   const int tid = threadIdx.x;
+  auto h = [&](int i) { return LONG ? pin[i] : sh_h[i]; };
   if (m > 0) {
-    sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
+    if constexpr (!LONG) sum_partial_rows(pin, m, nb_in, nb_in, sh_h);
     if (blockIdx.x == 0)
-      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = sh_h[i];
+      for (int i = tid; i < m; i += CGS_THREADS) hsave[i] = h(i);
   }
   const int64_t stride = (int64_t)gridDim.x * CGS_THREADS;
   double acc = 0.0;
@@ -1832,7 +1839,7 @@ cgs_norm(const double* __restrict__ V, int m, int64_t ldv, const double* __restr
       for (int i = 0; i < 8 * MG; ++i) v[i] = i0 + i < m ? V[(int64_t)(i0 + i) * ldv + t] : 0.0;
 #pragma unroll
       for (int i = 0; i < 8 * MG; ++i)
-        if (i0 + i < m) wt -= sh_h[i0 + i] * v[i];
+        if (i0 + i < m) wt -= h(i0 + i) * v[i];
     }
     out[t] = wt;
     acc += wt * wt;
@@ -1911,7 +1918,9 @@ struct GmresWork {
   double* z = nullptr;
   double* partial = nullptr;    // two sets of block partials, [restart+1][CGS_MAX_BLOCKS] each
   double* coef = nullptr;       // h of the two passes, reduced rows, solution coefficients
-  double* hcol = nullptr;       // pinned host buffer: a Hessenberg column per step, [restart+1][restart+2]
+  // pinned host buffer, [3][restart+2]: the Hessenberg columns of the step that
+  // the host reads and of the one enqueued ahead of it, the solution coefficients
+  double* hcol = nullptr;
   hipEvent_t ev[2] = {nullptr, nullptr};
   int restart = 0;
   int64_t n = 0;
@@ -1933,7 +1942,7 @@ static int gmres_alloc(pdes_ctx* c, GmresWork& W, int restart) {
       hipMalloc((void**)&W.z, n * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&W.partial, (size_t)2 * (restart + 1) * CGS_MAX_BLOCKS * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&W.coef, (size_t)4 * (restart + 2) * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void**)&W.hcol, (size_t)(restart + 1) * (restart + 2) * sizeof(double)) != hipSuccess ||
+      hipHostMalloc((void**)&W.hcol, (size_t)3 * (restart + 2) * sizeof(double)) != hipSuccess ||
       hipEventCreateWithFlags(&W.ev[0], hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&W.ev[1], hipEventDisableTiming) != hipSuccess) {
     set_error("GMRES workspace allocation failed");
@@ -1970,7 +1979,7 @@ void gmres_release(pdes_ctx* c) {
 // rows of block partials as the next launch reads them: as they are, or
 // summed once where there are many
 static void cgs_rows(pdes_ctx* c, GmresWork& W, int m, double*& rows, int& nb) {
-  if (nb <= CGS_SELF_REDUCE) return;
+  if (nb <= CGS_SELF_REDUCE && m <= CGS_LDS_ROWS) return;
   double* out = W.coef + 2 * (W.restart + 2);
   hipLaunchKernelGGL(multidot_reduce, dim3(m), dim3(CGS_THREADS), 0, c->stream, rows, nb, out);
   rows = out;
@@ -1980,18 +1989,21 @@ static void cgs_rows(pdes_ctx* c, GmresWork& W, int m, double*& rows, int& nb) {
 template <bool AXPY>
 static void launch_cgs_pass(pdes_ctx* c, GmresWork& W, int m, double* w, const double* pin, int nb_in, double* pout,
                             int nb) {
-  const size_t lds = AXPY ? (size_t)m * sizeof(double) : 0;
+  const bool lng = AXPY && m > CGS_LDS_ROWS;
+  const size_t lds = AXPY && !lng ? (size_t)m * sizeof(double) : 0;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(CGS_THREADS), lds, c->stream, W.V, m, W.n, w, W.n, pin, nb_in, W.coef,
                        pout);
   };
-  if (m <= 8) go(cgs_pass<1, AXPY>);
-  else if (m <= 16) go(cgs_pass<2, AXPY>);
-  else go(cgs_pass<4, AXPY>);
+  if (m <= 8) go(cgs_pass<1, AXPY, false>);
+  else if (m <= 16) go(cgs_pass<2, AXPY, false>);
+  else if (!lng) go(cgs_pass<4, AXPY, false>);
+  else go(cgs_pass<4, AXPY, AXPY>);
 }
 
 // w is made orthogonal to V_0 .. V_{m-1} and normalised; the column (m
-// coefficients and the norm) goes to the host slot of step m - 1
+// coefficients and the norm) goes to the host slot of step m - 1, which the next
+// step but one writes again
 static int cgs2_step(pdes_ctx* c, GmresWork& W, int m, double* w) {
   const int nb0 = cgs_blocks(W.n);
   double* pa = W.partial;
@@ -2007,17 +2019,19 @@ static int cgs2_step(pdes_ctx* c, GmresWork& W, int m, double* w) {
   nb = nb0;
   cgs_rows(c, W, m, rows, nb);
   auto norm = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(nb0), dim3(CGS_THREADS), (size_t)m * sizeof(double), c->stream, W.V, m, W.n,
+    const size_t lds = m > CGS_LDS_ROWS ? 0 : (size_t)m * sizeof(double);
+    hipLaunchKernelGGL(kernel, dim3(nb0), dim3(CGS_THREADS), lds, c->stream, W.V, m, W.n,
                        (const double*)nullptr, w, w, W.n, rows, nb, h2, pa);
   };
-  if (m <= 8) norm(cgs_norm<1>);
-  else if (m <= 16) norm(cgs_norm<2>);
-  else norm(cgs_norm<4>);
+  if (m <= 8) norm(cgs_norm<1, false>);
+  else if (m <= 16) norm(cgs_norm<2, false>);
+  else if (m <= CGS_LDS_ROWS) norm(cgs_norm<4, false>);
+  else norm(cgs_norm<4, true>);
   rows = pa;
   nb = nb0;
   cgs_rows(c, W, 1, rows, nb);
   hipLaunchKernelGGL(cgs_finish, dim3(nb0), dim3(CGS_THREADS), 0, c->stream, w, W.n, rows, nb, m, h1, h2,
-                     W.hcol + (size_t)(m - 1) * (W.restart + 2));
+                     W.hcol + (size_t)((m - 1) & 1) * (W.restart + 2));
   PDES_HIP(hipGetLastError());
   return PDES_OK;
 }
@@ -2025,7 +2039,7 @@ static int cgs2_step(pdes_ctx* c, GmresWork& W, int m, double* w) {
 // V_0 = (b - w) / ||b - w|| (w null: b / ||b||); the norm goes to the host
 static int cgs_start(pdes_ctx* c, GmresWork& W, const double* b, double* w) {
   const int nb0 = cgs_blocks(W.n);
-  hipLaunchKernelGGL(cgs_norm<1>, dim3(nb0), dim3(CGS_THREADS), 0, c->stream, (const double*)nullptr, 0, W.n, b, w, W.V,
+  hipLaunchKernelGGL((cgs_norm<1, false>), dim3(nb0), dim3(CGS_THREADS), 0, c->stream, (const double*)nullptr, 0, W.n, b, w, W.V,
                      W.n, (const double*)nullptr, 0, (double*)nullptr, W.partial);
   double* rows = W.partial;
   int nb = nb0;
@@ -2097,7 +2111,7 @@ int gmres_device(pdes_ctx* c, const double* b, double* x, double rtol, double at
           (st = enqueue(enqueued++)) != 0)
         goto done;
       PDES_HIP(hipEventSynchronize(W.ev[j & 1]));
-      const double* col = W.hcol + (size_t)j * (restart + 2);
+      const double* col = W.hcol + (size_t)(j & 1) * (restart + 2);
       const double hn = col[j + 1];
       for (int i = 0; i <= j; ++i) H[(size_t)i * restart + j] = col[i];
       H[(size_t)(j + 1) * restart + j] = hn;
@@ -2130,7 +2144,7 @@ int gmres_device(pdes_ctx* c, const double* b, double* x, double rtol, double at
         for (int k = i + 1; k < jdone; ++k) s -= H[(size_t)i * restart + k] * y[k];
         y[i] = s / H[(size_t)i * restart + i];
       }
-      double* ypin = W.hcol + (size_t)restart * (restart + 2);
+      double* ypin = W.hcol + (size_t)2 * (restart + 2);
       double* yd = W.coef + 3 * (restart + 2);
       for (int i = 0; i < jdone; ++i) ypin[i] = y[i];
       PDES_HIP(hipMemcpyAsync(yd, ypin, jdone * sizeof(double), hipMemcpyHostToDevice, c->stream));

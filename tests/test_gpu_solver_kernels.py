@@ -188,6 +188,50 @@ def test_gmres_cycle_is_the_least_squares_solution(restart):
     e.free()
 
 
+def test_gmres_cycle_longer_than_the_coefficients_in_lds():
+    """A cycle of 1,100 unpreconditioned steps, whose coefficients no longer go
+    to LDS, reaches the least residual over its Krylov space (numpy, CGS2), to
+    the k N eps |A| |x| that a backward stable method allows; the problem is so
+    stiff that the residual is still falling there (from 1 to 0.1)."""
+    m, op, ph, q = _problem("vortex", 3, 4, "diage", "roe")
+    e = euler.EulerData(m, op, ph)
+    e.set_q(q)
+    lo, pc = linsolve.HIPBSRLO(e, fp64_blocks=True), linsolve.PCNone(e)
+    linsolve.StandardLinearSolver(pc, lo).calcPCandLO()
+    ndof, k = q.size, 1100
+    rowptr, colind = linsolve.getSparsityPattern(e, fp64_blocks=True)
+    vals = linsolve.getJacobianValues(e, fp64_blocks=True)
+    nd = q.shape[2]
+    A4 = np.zeros((ndof // nd, nd, ndof // nd, nd))
+    for r in range(len(rowptr) - 1):
+        for t in range(rowptr[r], rowptr[r + 1]):
+            A4[r, :, colind[t], :] += vals[t]
+    A = A4.reshape(ndof, ndof)
+    b = np.random.default_rng(4).standard_normal(q.shape)
+    V, H = np.zeros((k + 1, ndof)), np.zeros((k + 1, k))
+    V[0] = b.ravel() / np.linalg.norm(b)
+    for j in range(k):
+        w = A @ V[j]
+        for _ in range(2):
+            h = V[:j + 1] @ w
+            w -= V[:j + 1].T @ h
+            H[:j + 1, j] += h
+        H[j + 1, j] = np.linalg.norm(w)
+        V[j + 1] = w / H[j + 1, j]
+    g = np.zeros(k + 1)
+    g[0] = np.linalg.norm(b)
+    x_ref = V[:k].T @ np.linalg.lstsq(H, g, rcond=None)[0]
+    ref = np.linalg.norm(b.ravel() - A @ x_ref)
+    ls = linsolve.StandardLinearSolver(pc, lo, reltol=1e-14, restart=k, itermax=k)
+    x = np.zeros_like(b)
+    assert ls.linearSolve(b, x) == k
+    got = np.linalg.norm(b.ravel() - A @ x.ravel())
+    print(got, ref, flush=True)
+    assert ref > 1e-2 * np.linalg.norm(b)
+    assert abs(got - ref) <= 2 * k * ndof * 2.0 ** -53 * np.linalg.norm(A, 2) * np.linalg.norm(x_ref)
+    e.free()
+
+
 @pytest.mark.parametrize("kind,p,opk,flux", SHAPES)
 def test_jacobian_matches_coloring_at_the_smallest_meshes(kind, p, opk, flux):
     """The element-wise assembly equals the colouring one where the last
