@@ -171,7 +171,7 @@ int pdes_ctx_create(const pdes_mesh_desc* m, const pdes_sbp_desc* s, const pdes_
       int node = s->perm[st * nfaces + f];
       if (node < 0 || node >= Np) { set_error("perm entry out of range"); pdes_ctx_destroy(c); return PDES_ERR_ARG; }
       c->h_nodepos[(size_t)node * nfaces + f] = st;
-      c->permbits[f] |= (uint64_t)node << (4 * st);
+      if (!s->diag_e && Np <= 16) c->permbits[f] |= (uint64_t)node << (4 * st);
     }
 
   // element -> face connectivity

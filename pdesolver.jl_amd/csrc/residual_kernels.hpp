@@ -332,6 +332,7 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
   __shared__ Smem sm;
   static_assert(!MF || (VOL == VOL_WEAK && std::is_same<T, double>::value),
                 "the matrix-core volume term is the FP64 weak form");
+  static_assert(Op::DIAGE || NP <= 16, "DevSBP::permbits holds a node in four bits");
 
   const int tid = threadIdx.x;
   constexpr int TPE = threads_per_element<Op, FLUX>();
