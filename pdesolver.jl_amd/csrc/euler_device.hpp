@@ -165,8 +165,11 @@ __device__ __forceinline__ void ir_zvars(const PhysConst& p, const T* q, T* z) {
 // (bc_solvers.jl:942-956, same branch test on u = f^2).  UNIFORM: the series is
 // evaluated for all lanes and the logs only when a lane of the wave needs one,
 // one wave-uniform branch for both factors; for the pair rounds and faces of the
-// diagonal-E values (RK4 steps of 131,072 triangles, p=4: 5448 -> 5250 us; a
-// residual of states 10% and more apart, which need the logs, 515 -> 492 us).
+// diagonal-E values.  With it the pair rounds unroll well, which gives the larger
+// part (131,072 triangles p=4, residual: a branch per factor, rolled rounds 229.0
+// us, unrolled 222 to 225; one branch, rolled 225.1, unrolled 217.5; five RK4
+// steps 5430, 5375, 5320 and 5165 us; states 10% and more apart, which need the
+// logs, 521, 501, 519 and 496; the first pass of a context 6870 and 6600 us).
 // Elsewhere a branch per factor: the logs, live together with both series, spill
 // (entropy-stable p=2, 45,000 triangles 121 us instead of 62; derivative of 7,442
 // triangles 38.5 us instead of 20.4).
