@@ -50,7 +50,7 @@ __device__ __forceinline__ int64_t active_dof(const int32_t* el_list, int64_t t,
 // sums of chunk c are partial[i * nct + c]; a workgroup adds up its own
 // instance's (in chunk order, so the bits depend on the instance only).  An
 // instance of more than CGS_SELF_REDUCE chunks (262,144 dofs) has them added
-// up once, by seg_reduce_big, into sum[inst][i].  With one kernel for every dot,
+// up once, by seg_reduce, into sum[inst][i].  With one kernel for every dot,
 // sum, update and norm, 9 launches a step, and 4096-dof chunks, a launch of the
 // dots took 19 us and of the rest 19 us more on average in a batch of ten (8 to
 // 28 cells a side, five operators side by side); these take 13 us and there are

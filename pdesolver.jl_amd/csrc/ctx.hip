@@ -63,27 +63,27 @@ using namespace pdes;
 
 // Default launch variant of the residual (residual_launch.hpp), from times of
 // all variants of every shape on meshes of 128 to 32,768 triangles and 162 to
-// 16,464 tets on MI355X (us):
-//   split form: large blocks at 4 waves per SIMD.  Diagonal-E (both bounds give
-//     the same code for p=4): 2D p=1..3 15.5, 22.7, 38.6 and small blocks 15.4 to
-//     15.5, 21.8 to 22.2, 36.0 to 37.1 at 32,768 triangles, but 8.1, 7.8, 9.3
-//     against 9.5, 9.1, 10.8 at 2,048 to 8,192.  Dense faces p=1..3 at 32,768
-//     triangles 23.2, 49.5, 102.9 against 25.4, 49.5, 107.9; but 3 waves for p=4,
-//     which spills with 4 (8,192 triangles 67.6 against 77.7, 32,768 229 against
-//     256), and in 3D (p=2, 16,464 tets: 95.2 against 110.3).
+// 16,464 tets on MI355X (us, launches one after another):
+//   split form: large blocks at 4 waves per SIMD.  Diagonal-E p=1..3 at 32,768
+//     triangles 15.0, 21.3, 36.2, small blocks 15.2, 21.6, 35.8, but at 8,192,
+//     4,608 and 2,048 triangles 8.0, 7.9, 9.2 against 9.4, 9.0, 10.8 (p=4 compiles
+//     to the same code for 3 and 4 waves).  Dense faces p=1..3 at 32,768 triangles
+//     23.4, 49.5, 102.6 against 25.3, 49.6, 107.5; but 3 waves for p=4, which
+//     spills with 4 (8,192 triangles 67.6 against 77.7, 32,768 229 against 256),
+//     and in 3D (p=2, 16,464 tets 94.8 against 110.4).
 //   weak form on dense faces, up to 512 blocks of 192 threads, and 2D Omega p=1:
-//     small blocks, vector ALUs (800 triangles: Omega p=1 5.6 against 6.4, p=3 7.9
-//     against 8.9; 6,000 tets p=2 14.9 against 16.6); not for p=4, where the matrix
-//     cores save more (800 triangles 7.8 against 7.7, 4,608 9.8 against 9.0).
+//     small blocks, vector ALUs (800 triangles: Omega p=1 5.6 against 6.5, p=3 7.9
+//     against 8.9; 6,000 tets p=2 14.8 against 16.7); not for p=4, where the matrix
+//     cores save more (4,608 triangles 9.1 against 9.7, 800 the same).
 //   weak form on diagonal-E operators, as long as there is a CU for each small
 //     block (128 threads): those (4,608 triangles p=1 6.5 against 6.9, 800 p=3 6.7
 //     against 6.9); with more of them than CUs the large ones win until they
 //     outnumber the CUs too, and from there on it is the same (8,192 triangles p=1
-//     7.8 against 7.0, 2,048 p=3 7.7 against 6.9, p=4 9.5 against 8.6).
+//     7.8 against 6.9, 2,048 p=3 7.7 against 7.0, p=4 9.5 against 8.6).
 //   weak form beyond: large blocks, with Q^T F on the matrix cores from 10 nodes
-//     an element (32,768 triangles, Omega p=4 25.7 against 30.7, diagonal-E p=2
-//     15.8 against 17.2; 16,464 tets p=2 28.7 against 29.3) and 4 waves, 3 for the
-//     3D ones (p=2 28.7 against 30.0, p=1 12.3 against 14.6).
+//     an element (32,768 triangles, Omega p=4 25.7 against 29.3, diagonal-E p=2
+//     15.8 against 16.5; 16,464 tets p=2 28.6 against 28.8) and 4 waves, 3 for the
+//     3D ones (p=2 28.6 against 30.0, p=1 12.3 against 14.6).
 static int default_variant(const pdes_ctx* c) {
   if (c->phys.volume_integral_type == 2) return !c->diag_e && (c->dim == 3 || c->Np == 15) ? 0 : 1;
   const int64_t nodes = (int64_t)c->numEl * c->Np;

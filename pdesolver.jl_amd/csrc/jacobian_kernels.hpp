@@ -16,8 +16,9 @@
 // come from forward-mode dual numbers (dF/dqL, dF/dqR), the analytic
 // counterpart of the reference's hand-differentiated *_diff functions.
 //
-// The kernel is written so that no thread runs long and none spills: a face
-// node's derivative is one thread per seeded component (dual<1>), a volume
+// The kernel is written so that no thread runs long and few values spill (none
+// outside the entropy-stable form; there 3D p=2 puts 364 to 372 bytes a lane into
+// scratch memory): a face node's derivative is one thread per seeded component (dual<1>), a volume
 // pair one thread per ordered pair, differentiated in the combined direction
 // with respect to one state only (the flux is symmetric: the other state's
 // derivative is the other ordered pair's), and the weak form's blocks are
@@ -313,7 +314,8 @@ __device__ __forceinline__ void face_derivative(const PhysConst& phys, const dou
 
 // elements per workgroup: as many as give every thread about one row of
 // values (weak form: NP ndof^2 of them) or one volume pair column, in at most
-// 40 KB of LDS, so that four workgroups fit a CU
+// 40 KB of LDS for the elements (with the operator's tables 42 KB: three
+// workgroups of the split form a CU, and its 212 registers allow two waves a SIMD)
 template <class Op, int VOL, int FLUX>
 constexpr int jac_epb() {
   constexpr int per = VOL == VOL_WEAK ? Op::NP * Op::ND * Op::ND : Op::NP * JacElem<Op, VOL, FLUX>::KP;

@@ -183,9 +183,10 @@ struct RKStage {
 // (face, stencil node), of which the first NP take the nodes.  That scheme is a
 // chain of two-point fluxes, bound by latency: with a thread per node an element
 // of 2D p=2 took 3 fluxes and as many barriers for the volume and 18 in a row
-// for the faces, with one wave a workgroup; now 1 and 6.  Derivative, 7,442
-// triangles 64.6 -> 35.2 us (p=2), 3,072 tets (p=2) 119.6 -> 53.6 us; residual,
-// 45,000 triangles 89.1 -> 61.7 us, 16,464 tets 169 -> 94.6 us.
+// for the faces, with one wave a workgroup; now 1 and 6.  Launches one after
+// another: derivative, 7,442 triangles p=2 64.7 -> 33.7 us, 3,072 tets p=2 119.9
+// -> 52.7 us; residual, 45,000 triangles p=2 107 -> 62.5 us, 16,464 tets p=2 239
+// -> 95 us.
 template <class Op, int FLUX>
 constexpr int threads_per_element() {
   return FLUX == PDES_FLUX_ESLF ? Op::NFACES * Op::ST : Op::NP;
@@ -954,11 +955,11 @@ euler_residual_kernel(DevMesh mesh, DevSBP sbp, PhysConst phys,
     // one thread per (face, component) reads each node's value once for all
     // face nodes of both sides (the interpolation matrix is the same for every
     // lane and comes through the scalar cache), instead of every face node's
-    // thread reading every node of both sides.  Residual, before and after:
-    // 3D p=2, 48,000 tets 78 -> 57 us (0.67 TB/s; waves for the numerical flux
-    // and the lift wait, two a SIMD); 2D p=3, 18,818 triangles 19.6 -> 14.0 us,
-    // 800 triangles 12 -> 7.9 us; p=4 23.2 -> 18.1 us; p=2, 131,072 triangles
-    // 48 -> 39.6 us.
+    // thread reading every node of both sides.  Residual, before and after,
+    // launches one after another: 3D p=2, 48,000 tets 79.7 -> 62.1 us (0.6 TB/s;
+    // waves for the numerical flux and the lift wait, two a SIMD); 2D p=3, 18,818
+    // triangles 20.4 -> 14.6 us, 800 triangles 15.2 -> 8.4 us; p=4, 18,818
+    // triangles 25.9 -> 18.7 us; p=2, 131,072 triangles 51.2 -> 39.9 us.
     static_assert(VOL == VOL_WEAK && FLUX == PDES_FLUX_ROE && ST == NP, "dense weak form");
     typedef const double __attribute__((address_space(4))) uniform_double;
     uniform_double* const R = (uniform_double*)sbp.interp;

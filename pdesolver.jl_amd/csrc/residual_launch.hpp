@@ -1,7 +1,7 @@
 // residual_launch.hpp -- launch-variant interface of the fused residual kernel.
 //
 // Tunable launch variants of the FP64 value kernel (the directional-derivative
-// kernel always takes 128 threads, or 256, and 2 waves):
+// kernel takes 64, 128 or 256 threads, by operator, and 2 waves):
 //   0: large blocks, 3 waves per SIMD      1: large blocks, 4 waves per SIMD
 //   2: small blocks, 3 waves per SIMD      3: small blocks, 4 waves per SIMD
 // (whole elements in 256 and 128 threads; dense-face weak form 192 and 64)

@@ -39,9 +39,11 @@ static int launch_one(pdes_ctx* c, const double* q, const double* v, double* res
   constexpr int FULL = (DENSE_WEAK ? 192 : 256) / TPE;
   constexpr int HALF = (DENSE_WEAK ? 64 : 128) / TPE;
   if constexpr (!std::is_same<T, double>::value) {
-    // (derivatives, entropy-stable: 2D p=2, 7,442 triangles 128 threads 43 us,
-    // 256 51; 3D p=2, 3,072 tets 123 and 57; 2D p=4, 3,200 triangles 69 and 64;
-    // weak form, 3D p=1, 10,368 tets 128 threads 22.8 us, 64 17.8; p=2 55.5 and 57.9)
+    // (derivatives, 64, 128 and 256 threads, us.  Entropy-stable: 2D p=2, 7,442
+    // triangles 35.0, 35.8, 38.8; p=3, 18,818 triangles 222, 227, 228; p=4, 3,200
+    // triangles 72.7, 65.8, 61.5; 3D p=2, 3,072 tets 115.6, 116.8, 53.4.  Weak form
+    // on dense faces: 3D p=1, 10,368 tets 17.9, 23.0, 18.3; p=2 58.1, 55.8, 52.4;
+    // 2D p=1, 800 triangles 9.1, 10.1, 12.0)
     constexpr int EPB =
         (FLUX == PDES_FLUX_ESLF && Op::ST >= 10 ? 256 : DENSE_WEAK && Op::NP == Op::NFACES ? 64 : 128) / TPE;
     return launch_cfg<Op, VOL, FLUX, T, EPB, 2>(c, q, v, res, jv, flag, nullptr);

@@ -8,8 +8,8 @@
 // GMRES(restart) with right preconditioning replaces the PETSc KSP of
 // src/linearsolvers/ls_standard.jl:321-370 (KSP options read_input.jl:560-581);
 // the Arnoldi basis, Hessenberg and update stay FP64.  Orthogonalisation is
-// classical Gram-Schmidt applied twice (CGS2): two multi-dot and two
-// multi-axpy passes per step, each reading the basis once.
+// classical Gram-Schmidt applied twice (CGS2) in four launches per step, of
+// which three read the basis.
 // Newton follows newtonInner (src/NonlinearSolvers/newton.jl:137-304).
 #include <algorithm>
 #include <chrono>
@@ -1246,7 +1246,11 @@ static int ilu_structure(pdes_ctx* c, pdes_precond* p) {
   }
   PDES_HIP(hipMemcpyAsync(p->d_fel, fel.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
   PDES_HIP(hipMemcpyAsync(p->d_bel, bel.data(), nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  bool twice = false;   // an element that meets a neighbour at two faces (its rows then hold a column twice)
+  // an element that meets a neighbour at two faces: level sweeps, which walk the
+  // rows (the sets' kernel goes by faces).  Diagonal-E operators only: with dense
+  // faces such an element's rows hold every column of the neighbour twice, which
+  // the assembly refuses.
+  bool twice = false;
   for (int e = 0; e < nel && !twice; ++e)
     for (int f = 0; f < nf; ++f)
       for (int g = f + 1; g < nf; ++g) {
@@ -1610,8 +1614,8 @@ static int ilu_apply_graphed(pdes_ctx* c, const double* b, double* x) {
 }
 
 int pc_apply(pdes_ctx* c, const double* b, double* x) {
-  // the dependency-driven sweeps are 4 launches; the level-by-level ones are
-  // replayed from a captured graph
+  // the dependency-driven sweeps are two launches, one a triangle; the
+  // level-by-level ones are replayed from a captured graph
   if (c->pc_obj && c->pc_obj->kind == PDES_PC_ILU0)
     return c->use_graphs && !c->capturing && !ilu_use_dep(c, c->pc_obj) ? ilu_apply_graphed(c, b, x)
                                                                         : ilu_apply_dispatch(c, b, x);
